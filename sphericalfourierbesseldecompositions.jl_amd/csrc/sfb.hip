@@ -2138,7 +2138,7 @@ __global__ void k_pack(const TA* __restrict__ a, const int64_t* __restrict__ aof
     const int l = maps[q].l;
     if (m > l) return;
     const int par = (l - m) & 1, j = (l - m) >> 1;
-    const TA* src = a + aoff[m * 2 + par] + (int64_t)j * M2 + 2 * q;
+    const TA* src = a + (aoff[m * 2 + par] + j) * M2 + 2 * q;
     const double re = src[0], im = src[1];
     out[2 * (out_base[q] + m)] = re;
     out[2 * (out_base[q] + m) + 1] = im;
@@ -2182,7 +2182,7 @@ __global__ void k_pack_alm(const double* __restrict__ a, const int64_t* __restri
     const int64_t nalm = (int64_t)(L + 1) * (L + 2) / 2;
     for (int l = m; l <= L; ++l) {
         const int par = (l - m) & 1, j = (l - m) >> 1;
-        const double* src = a + aoff[m * 2 + par] + (int64_t)j * M2 + 2 * q;
+        const double* src = a + (aoff[m * 2 + par] + j) * M2 + 2 * q;
         int64_t idx = (int64_t)m * (2 * L + 1 - m) / 2 + l;
         out[2 * ((int64_t)q * nalm + idx)] = src[0];
         out[2 * ((int64_t)q * nalm + idx) + 1] = src[1];
@@ -2228,7 +2228,7 @@ __global__ void k_unpack_cot(const double* __restrict__ cot, const int64_t* __re
     const int l = maps[q].l;
     if (m > l) return;
     const int par = (l - m) & 1, j = (l - m) >> 1;
-    TA* dst = a + aoff[m * 2 + par] + (int64_t)j * M2 + 2 * q;
+    TA* dst = a + (aoff[m * 2 + par] + j) * M2 + 2 * q;
     const double re = cot[2 * (out_base[q] + m)], im = cot[2 * (out_base[q] + m) + 1];
     dst[0] = (TA)(m ? 0.5 * re : re);
     dst[1] = (TA)(m ? 0.5 * im : 0.0);
@@ -2626,7 +2626,7 @@ __global__ void k_field_contract(int32_t nmaps, int32_t Q, int64_t s0, int64_t n
     const int l = maps[q].l;
     if (m > l) return;
     const int par = (l - m) & 1, j = (l - m) >> 1;
-    const double* src = a + aoff[m * 2 + par] + (int64_t)j * M2;
+    const double* src = a + (aoff[m * 2 + par] + j) * M2;
     const double* g = gtab + (int64_t)q * nr;
     double sr = 0.0, si = 0.0;
     for (int s = 0; s < Q; ++s) {
@@ -2659,7 +2659,7 @@ __global__ void k_field_alm(int32_t nmax, int32_t L, int32_t Q, int64_t s0, int6
         si += g * fnlm[o + 1];
     }
     const int par = (l - m) & 1, j = (l - m) >> 1;
-    double* dst = a + aoff[m * 2 + par] + (int64_t)j * M2 + 2 * s;
+    double* dst = a + (aoff[m * 2 + par] + j) * M2 + 2 * s;
     dst[0] = sr;
     dst[1] = si;
 }
@@ -2883,6 +2883,26 @@ struct PinBuf {
     template <class T> T* as() const { return (T*)p; }
 };
 
+#include "sht_direct_kernels.h"
+
+// Tables and launch lists of the refined map2alm as one operator (sht_direct.h).
+struct DirectSht {
+    bool ok = false;               // the folded form applies (else jacobi_stage iterates)
+    int32_t S = 0, ct = 2;         // aliasing states; columns per k_alias_solve block
+    int32_t n_ana = 0, n_fix = 0, n_syn = 0, n_sfix = 0;  // batches of each launch
+    int32_t maxN = 1, maxNs = 1, maxNf = 1;
+    int64_t hrows = 0;
+    std::vector<int32_t> s0, na, ka;  // per m: first state, states, first ring pair
+    DevBuf d_lamP, d_lamPT, d_HB, d_GZ, d_UB, d_ZB, d_Q, d_qoff, d_st, d_term, d_h, d_r;
+    DevBuf d_ana, d_fix, d_syn, d_sfix;
+    void release()
+    {
+        DevBuf* b[] = {&d_lamP, &d_lamPT, &d_HB, &d_GZ, &d_UB, &d_ZB, &d_Q, &d_qoff, &d_st, &d_term, &d_h, &d_r,
+                       &d_ana, &d_fix, &d_syn, &d_sfix};
+        for (DevBuf* x : b) x->release();
+    }
+};
+
 struct sfb_plan {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -2894,7 +2914,8 @@ struct sfb_plan {
     int32_t fft_nt = 512, fft_nt32 = 256;           // FFT threads per block (FP64 / FP32)
     double tune_ms = 0.0;                           // time the plan-time tile search took
     std::vector<MapInfo> maps;
-    std::vector<int64_t> out_base, aoff, lam_off;
+    std::vector<int64_t> out_base, lam_off;
+    std::vector<int64_t> aoff;  // per (m, parity): first row of its block in the a buffers (rows of M2 values)
     std::vector<int32_t> nb;  // per (m, par): number of l
     std::vector<int32_t> kcut;  // per m: first ring pair whose Lam_lm matters (non-decreasing in m)
     DevBuf d_mall;              // per ring pair k: the largest m with kcut[m] <= k (-1: none)
@@ -2906,6 +2927,7 @@ struct sfb_plan {
     DevBuf d_maps, d_kx, d_seg, d_rings, d_tw, d_lam, d_lamT, d_outbase, d_aoff, d_desc_ana, d_desc_syn, d_flag;
     // work
     DevBuf d_delta, d_X0, d_G, d_R, d_a, d_a1, d_a2, d_ic0;
+    DirectSht dir;                 // map2alm with its refinements as one operator
     DevBuf d_mono;                 // mixed path: monopole partial sums and window sums
     DevBuf d_desc_synf;            // full synthesis a -> X0 (all ring pairs), per a buffer
     DevBuf d_desc_synf32;          // the same with a, LamT and X0 as floats (mixed adjoint)
@@ -2923,6 +2945,7 @@ struct sfb_plan {
     DevBuf d_lamT32, d_ic032, d_lamw32;  // FP32 copies of the Jacobi GEMM tables (mixed path)
     double* a_final = nullptr;     // the a buffer holding the last result
     bool a_f32 = false;            // ... stored as floats (mixed path)
+    int64_t a_ld = 0;              // ... its row stride
     // catalogue
     DevBuf d_keyr, d_keyr2, d_idx, d_idx2, d_pix, d_pixkey, d_pixkey2, d_rs, d_ws, d_pstart, d_sorttmp;
     // host-API staging
@@ -3014,6 +3037,10 @@ static void prof_collect(sfb_plan* P)
         P->pend[ph].clear();
     }
 }
+
+static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
+
+#include "sht_direct.h"
 
 static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_off, const double* kx,
                        const double* ky, const double* kypp)
@@ -3302,10 +3329,10 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
             size_t b = (size_t)(m * 2 + par);
             P->nb[b] = n;
             P->lam_off[b + 1] = P->lam_off[b] + (int64_t)n * P->K;
-            P->aoff[b + 1] = P->aoff[b] + (int64_t)n * P->M2;
+            P->aoff[b + 1] = P->aoff[b] + n;
         }
     P->lam_size = P->lam_off.back();
-    P->a_size = P->aoff.back();
+    P->a_size = P->aoff.back() * P->M2;
     std::vector<double> lam((size_t)P->lam_size), lamT((size_t)P->lam_size), col((size_t)(L + 1));
     for (int32_t k = 0; k < P->K; ++k) {
         const sfb::RingPair& R = rp[(size_t)k];
@@ -3341,9 +3368,10 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
     // m: pair k needs G and R only for m <= mall[k] (every such m has kcut[m] <= k), and
     // the phi-transform need not write (nor its inverse read) X of pair k beyond mall[k].
     P->kcut.assign((size_t)(L + 1), P->K);
+    std::vector<double> rowmax_all((size_t)((L + 1) * P->K), 0.0);  // [m][k]: max over l of |Lam_lm|
     for (int64_t m = 0; m <= L; ++m) {
         double mx = 0.0;
-        std::vector<double> rowmax((size_t)P->K, 0.0);
+        double* rowmax = rowmax_all.data() + m * P->K;
         for (int par = 0; par < 2; ++par) {
             const size_t b = (size_t)(m * 2 + par);
             const int64_t n = P->nb[b];
@@ -3449,7 +3477,7 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
     const int64_t nbat = 2 * (L + 1);
     std::vector<GemmDesc> ana, ana32, syn, syn32, cal, cal32;
     // mixed path: the iterate a (and b) held as floats: block offsets count floats
-    auto fa = [&](DevBuf& buf, size_t b) { return (double*)(buf.as<float>() + P->aoff[b]); };
+    auto fa = [&](DevBuf& buf, size_t b) { return (double*)(buf.as<float>() + P->aoff[b] * P->M2); };
     DevBuf* a_in_buf[3] = {&P->d_a, &P->d_a1, &P->d_a2};
     DevBuf* a_out_buf[3] = {&P->d_a1, &P->d_a2, &P->d_a1};
     double* a_in_slot[3] = {P->d_a.as<double>(), P->d_a1.as<double>(), P->d_a2.as<double>()};
@@ -3462,7 +3490,7 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
         GemmDesc d{};
         d.A = P->d_X0.as<double>() + (b * (int64_t)P->K + kc) * P->M2;
         d.B = P->d_lam.as<double>() + P->lam_off[(size_t)b] + kc * n;
-        d.C = P->d_a.as<double>() + P->aoff[(size_t)b];
+        d.C = P->d_a.as<double>() + P->aoff[(size_t)b] * P->M2;
         d.Cin = nullptr;
         d.K = (int32_t)(P->K - kc);
         d.N = n;
@@ -3481,7 +3509,7 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
             int32_t n = P->nb[(size_t)b];
             const int64_t kal = std::min<int64_t>(P->kcut[(size_t)(b / 2)], P->K_al);
             GemmDesc sd{};
-            sd.A = a_in_slot[slot] + P->aoff[(size_t)b];
+            sd.A = a_in_slot[slot] + P->aoff[(size_t)b] * P->M2;
             sd.B = P->d_lamT.as<double>() + P->lam_off[(size_t)b] + kal;
             sd.C = P->d_G.as<double>() + (b * (int64_t)P->K_al + kal) * P->M2;
             sd.Cin = nullptr;
@@ -3497,10 +3525,10 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
             sd.C = (double*)(P->d_G.as<float>() + (b * (int64_t)P->K_al + kal) * P->M2);
             syn32.push_back(sd);
             GemmDesc cd{};
-            cd.A = a_in_slot[slot] + P->aoff[(size_t)b];
+            cd.A = a_in_slot[slot] + P->aoff[(size_t)b] * P->M2;
             cd.B = P->d_ic0.as<double>() + P->ic0_off[(size_t)b];
-            cd.C = a_out_slot[slot] + P->aoff[(size_t)b];
-            cd.Cin = P->d_a.as<double>() + P->aoff[(size_t)b];
+            cd.C = a_out_slot[slot] + P->aoff[(size_t)b] * P->M2;
+            cd.Cin = P->d_a.as<double>() + P->aoff[(size_t)b] * P->M2;
             cd.K = n;
             cd.N = n;
             cd.lda = P->M2;
@@ -3536,7 +3564,7 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
             int32_t n = P->nb[(size_t)b];
             const int64_t kc = P->kcut[(size_t)(b / 2)];  // ring pairs from kc on
             GemmDesc fd{};
-            fd.A = a_in_slot[slot] + P->aoff[(size_t)b];
+            fd.A = a_in_slot[slot] + P->aoff[(size_t)b] * P->M2;
             fd.B = P->d_lamT.as<double>() + P->lam_off[(size_t)b] + kc;
             fd.C = P->d_X0.as<double>() + (b * (int64_t)P->K + kc) * P->M2;
             fd.Cin = nullptr;
@@ -3573,7 +3601,7 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
         return rc;
     HIP_TRY(hipMemcpy(P->d_desc_cal.p, cal.data(), sizeof(GemmDesc) * cal.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(P->d_desc_cal32.p, cal32.data(), sizeof(GemmDesc) * cal32.size(), hipMemcpyHostToDevice));
-    return SFB_OK;
+    return direct_tables(P, rd, rowmax_all);
 }
 
 extern "C" const char* sfb_version(void) { return "sfb_mi355x 0.1 (gfx950)"; }
@@ -3677,6 +3705,7 @@ extern "C" void sfb_plan_destroy(sfb_plan* P)
                       &P->d_reclo, &P->d_sblk32s, &P->d_mrange, &P->d_bflag};
     if (P->bg_exec) (void)hipGraphExecDestroy(P->bg_exec);
     for (DevBuf* b : bufs) b->release();
+    P->dir.release();
     P->pin_in.release();
     P->pin_out.release();
     if (P->stream) (void)hipStreamDestroy(P->stream);
@@ -3699,8 +3728,6 @@ extern "C" int sfb_plan_set_precision(sfb_plan* P, int32_t precision)
     P->precision = precision;
     return SFB_OK;
 }
-
-static inline unsigned nblk(int64_t n, int b) { return (unsigned)((n + b - 1) / b); }
 
 // Sort the catalogue and build the pixel segments.  Leaves r_s, w_s, pstart and,
 // when the records fit in LDS, the sliced layout sr, sw (soff, perm).  sort_r: galaxies
@@ -4139,8 +4166,9 @@ static InvShapes inv_shapes(int64_t nside, int64_t L, int64_t lds_max)
 // otherwise for every m <= lmax.  Tile shapes (maps and threads per FFT block, maps per
 // polar block) come from the plan's tile search (autotune_phi); they change no arithmetic.
 static int phi_transform(sfb_plan* P, int32_t nq, hipStream_t st, bool f32, bool cut = true,
-                         const void* src = nullptr)
+                         const void* src = nullptr, int64_t ld = 0)
 {
+    if (!ld) ld = P->M2;  // row stride of X
     const int32_t* mall = cut ? P->d_mall.as<int32_t>() : nullptr;
     const void* dsrc = src ? src : P->d_delta.p;  // the maps (P->d_delta unless given)
     const int32_t K = P->K, L = (int32_t)P->lmax;
@@ -4159,12 +4187,12 @@ static int phi_transform(sfb_plan* P, int32_t nq, hipStream_t st, bool f32, bool
     if (f32) {
         HIP_TRY(hipFuncSetAttribute((const void*)k_phi_fft<double, float>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shf));
         hipLaunchKernelGGL((k_phi_fft<double, float>), grid_f, dim3(P->fft_nt32), shf, st,
-                           (const float*)dsrc, P->npix, nq, P->M2, K, L, P->d_rings.as<RingDev>(),
+                           (const float*)dsrc, P->npix, nq, ld, K, L, P->d_rings.as<RingDev>(),
                            P->d_tw.as<double2>(), P->d_X0.as<float>(), tqf, k_eq0, P->logM, mall, P->delta_perm, nring_f, ntile_f);
     } else {
         HIP_TRY(hipFuncSetAttribute((const void*)k_phi_fft<double>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shf));
         hipLaunchKernelGGL(k_phi_fft<double>, grid_f, dim3(P->fft_nt), shf, st,
-                           (const double*)dsrc, P->npix, nq, P->M2, K, L, P->d_rings.as<RingDev>(),
+                           (const double*)dsrc, P->npix, nq, ld, K, L, P->d_rings.as<RingDev>(),
                            P->d_tw.as<double2>(), P->d_X0.as<double>(), tqf, k_eq0, P->logM, mall, P->delta_perm, nring_f, ntile_f);
     }
     LAUNCH_CHECK();
@@ -4178,7 +4206,7 @@ static int phi_transform(sfb_plan* P, int32_t nq, hipStream_t st, bool f32, bool
     const dim3 grid_p((unsigned)(32 * (((int64_t)k_eq0 * gy4 + 31) / 32)));
     auto go = [&](auto kern, const auto* src, auto* x) -> int {
         HIP_TRY(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shp));
-        hipLaunchKernelGGL(kern, grid_p, dim3(256), shp, st, src, P->npix, nq, P->M2, K, L, P->d_rings.as<RingDev>(),
+        hipLaunchKernelGGL(kern, grid_p, dim3(256), shp, st, src, P->npix, nq, ld, K, L, P->d_rings.as<RingDev>(),
                            P->d_tw.as<double2>(), x, mall, P->delta_perm, k_eq0, gy4);
         return SFB_OK;
     };
@@ -4358,6 +4386,14 @@ static int sht_stage(sfb_plan* P, int32_t nq, hipStream_t st, bool f32 = false, 
 {
     const int32_t L = (int32_t)P->lmax;
     const double domega = 4.0 * kPi / (double)P->npix;
+    if (!f32 && P->dir.ok) {
+        // X and a in compact rows of the nq maps: a few shells (field2anlm) then read and
+        // write whole lines instead of 2 nq values every 2 nmaps
+        P->a_ld = 2 * (int64_t)nq;
+        int rc = phi_transform(P, nq, st, false, true, src, P->a_ld);
+        return rc ? rc : direct_analysis(P, 2 * nq, P->a_ld, st);
+    }
+    P->a_ld = P->M2;
     {
         int rc = phi_transform(P, nq, st, f32, true, src);
         if (rc) return rc;
@@ -4377,7 +4413,7 @@ static int sht_stage(sfb_plan* P, int32_t nq, hipStream_t st, bool f32 = false, 
 // block does not fit in LDS); equatorial ones: the inverse FFT (the direct sum where its
 // block does not fit).
 template <typename R>
-static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st)
+static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st, int64_t ld)
 {
     const int32_t K = P->K, L = (int32_t)P->lmax;
     const InvShapes S = inv_shapes(P->nside, L, P->lds_max);  // sized for FP64: FP32 blocks use less
@@ -4389,7 +4425,7 @@ static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st
         const int32_t ntile = (int32_t)((nq + S.tqmin - 1) / S.tqmin);
         const int64_t units = (int64_t)S.nip4 * ntile;
         hipLaunchKernelGGL(k_phi_ipolar4<R>, dim3((unsigned)(32 * ((units + 31) / 32))), dim3(256), S.shq, st, X,
-                           P->npix, nq, P->M2, K, L, P->d_rings.as<RingDev>(), P->d_tw.as<double2>(), scale, out,
+                           P->npix, nq, ld, K, L, P->d_rings.as<RingDev>(), P->d_tw.as<double2>(), scale, out,
                            IP_TQMAX, P->d_mall.as<int32_t>(), S.nip4, ntile);
         LAUNCH_CHECK();
     }
@@ -4398,7 +4434,7 @@ static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st
         const size_t shs = sizeof(double2) * 2 * TQS * (size_t)(L + 1);
         HIP_TRY(hipFuncSetAttribute((const void*)k_phi_synth<R>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shs));
         hipLaunchKernelGGL(k_phi_synth<R>, dim3((unsigned)(S.k_eq0 - S.nip4), nblk(nq, TQS)), dim3(256), shs, st, X,
-                           P->npix, nq, P->M2, K, L, P->d_rings.as<RingDev>(), scale, out, TQS,
+                           P->npix, nq, ld, K, L, P->d_rings.as<RingDev>(), scale, out, TQS,
                            P->d_mall.as<int32_t>(), S.nip4);
         LAUNCH_CHECK();
     }
@@ -4406,16 +4442,18 @@ static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st
         HIP_TRY(hipFuncSetAttribute((const void*)k_phi_ifft<R>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S.shi));
         const int64_t units = (int64_t)(K - S.k_eq0) * nblk(nq, S.tqi);
         hipLaunchKernelGGL(k_phi_ifft<R>, dim3((unsigned)(32 * ((units + 31) / 32))), dim3(512), S.shi, st, X,
-                           P->npix, nq, P->M2, K, L, P->d_rings.as<RingDev>(), P->d_tw.as<double2>(), scale, out,
+                           P->npix, nq, ld, K, L, P->d_rings.as<RingDev>(), P->d_tw.as<double2>(), scale, out,
                            S.tqi, S.k_eq0, P->logM, P->d_mall.as<int32_t>());
         LAUNCH_CHECK();
     }
     return SFB_OK;
 }
 
-static int phi_synthesis(sfb_plan* P, int32_t nq, double scale, hipStream_t st, bool f32 = false)
+static int phi_synthesis(sfb_plan* P, int32_t nq, double scale, hipStream_t st, bool f32 = false,
+                         int64_t ld = 0)
 {
-    return f32 ? phi_synthesis_t<float>(P, nq, scale, st) : phi_synthesis_t<double>(P, nq, scale, st);
+    if (!ld) ld = P->M2;
+    return f32 ? phi_synthesis_t<float>(P, nq, scale, st, ld) : phi_synthesis_t<double>(P, nq, scale, st, ld);
 }
 
 // Launch shapes of the ring transforms for a geometry (host arithmetic, no device).
@@ -4526,11 +4564,11 @@ static int cat2amln_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const d
         if (P->a_f32)
             hipLaunchKernelGGL(k_pack<float>, dim3(nblk(P->nmaps, 256), (unsigned)(P->lmax + 1)), dim3(256), 0, st,
                                (const float*)P->a_final, P->d_aoff.as<int64_t>(), P->d_maps.as<MapInfo>(),
-                               P->d_outbase.as<int64_t>(), (int32_t)P->nmaps, P->M2, d_out, P->d_flag.as<int32_t>());
+                               P->d_outbase.as<int64_t>(), (int32_t)P->nmaps, P->a_ld, d_out, P->d_flag.as<int32_t>());
         else
             hipLaunchKernelGGL(k_pack<double>, dim3(nblk(P->nmaps, 256), (unsigned)(P->lmax + 1)), dim3(256), 0, st,
                                P->a_final, P->d_aoff.as<int64_t>(), P->d_maps.as<MapInfo>(),
-                               P->d_outbase.as<int64_t>(), (int32_t)P->nmaps, P->M2, d_out, P->d_flag.as<int32_t>());
+                               P->d_outbase.as<int64_t>(), (int32_t)P->nmaps, P->a_ld, d_out, P->d_flag.as<int32_t>());
         LAUNCH_CHECK();
     }
     if (f32 && (rc = monopole_fix(P, N, nbar, win_kind, d_win_a, d_win_b, d_out, st))) return rc;
@@ -4722,7 +4760,8 @@ extern "C" int sfb_cat2amln_vjp_device(sfb_plan* P, int64_t N, const double* d_r
     LAUNCH_CHECK();
     const bool prof = P->prof;
     P->prof = false;  // the adjoint's stages are timed as one phase
-    rc = jacobi_stage(P, nq, st, f32);
+    const bool direct = !f32 && P->dir.ok;
+    rc = direct ? direct_synthesis(P, 2 * nq, P->M2, st) : jacobi_stage(P, nq, st, f32);
     P->prof = prof;
     if (rc) return rc;
     // dbar = dOmega S a_final on every pixel of every map
@@ -4730,7 +4769,7 @@ extern "C" int sfb_cat2amln_vjp_device(sfb_plan* P, int64_t N, const double* d_r
     const unsigned nbat = (unsigned)(2 * (L + 1));
     if (f32)
         launch_gemm(P->d_desc_synf32.as<GemmDesc>() + slot * nbat, nbat, 2 * nq, P->K, 1.0, 0.0, st, true, true, true);
-    else
+    else if (!direct)
         launch_gemm(P->d_desc_synf.as<GemmDesc>() + slot * nbat, nbat, 2 * nq, P->K, 1.0, 0.0, st);
     LAUNCH_CHECK();
     const double domega = 4.0 * kPi / (double)P->npix;
@@ -5128,7 +5167,7 @@ extern "C" int sfb_field2anlm_device(sfb_plan* P, int64_t nr, const double* d_r,
         if ((rc = sht_stage(P, Q, st, false))) return rc;
         hipLaunchKernelGGL(k_field_contract, dim3(nblk(P->nmaps, 256), (unsigned)(P->lmax + 1)), dim3(256), 0, st,
                            (int32_t)P->nmaps, Q, s0, nr, d_r, dr, P->d_gtab.as<double>(), P->d_maps.as<MapInfo>(),
-                           P->d_aoff.as<int64_t>(), P->d_outbase.as<int64_t>(), P->M2, P->a_final, d_out);
+                           P->d_aoff.as<int64_t>(), P->d_outbase.as<int64_t>(), P->a_ld, P->a_final, d_out);
         LAUNCH_CHECK();
     }
     HIP_TRY(hipStreamSynchronize(st));
@@ -5779,7 +5818,7 @@ extern "C" int sfb_map2alm(sfb_plan* P, int64_t nmap, const double* maps, double
     int64_t nalm = (P->lmax + 1) * (P->lmax + 2) / 2;
     if ((rc = P->h_out.ensure(sizeof(double) * 2 * (size_t)(nalm * nmap)))) return rc;
     hipLaunchKernelGGL(k_pack_alm, dim3(nblk(nmap, 256), (unsigned)(P->lmax + 1)), dim3(256), 0, P->stream,
-                       P->a_final, P->d_aoff.as<int64_t>(), (int32_t)nmap, (int32_t)P->lmax, P->M2,
+                       P->a_final, P->d_aoff.as<int64_t>(), (int32_t)nmap, (int32_t)P->lmax, P->a_ld,
                        P->h_out.as<double>());
     LAUNCH_CHECK();
     HIP_TRY(hipMemcpyAsync(alm_out, P->h_out.p, sizeof(double) * 2 * (size_t)(nalm * nmap), hipMemcpyDeviceToHost,
