@@ -147,12 +147,14 @@ __device__ __forceinline__ uint64_t sortable_bits(double v)
 
 // flag[1] |= 1 when an angle is not finite (the reference's floor(Int, NaN) throws).
 __global__ void k_prep(int64_t N, const double* __restrict__ rtp, int64_t nside, uint64_t* __restrict__ key_r,
-                       uint32_t* __restrict__ idx, uint32_t* __restrict__ pix, int32_t* __restrict__ flag)
+                       uint32_t* __restrict__ idx, uint32_t* __restrict__ pix, double* __restrict__ rcol,
+                       int32_t* __restrict__ flag)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     double r = rtp[3 * i], th = rtp[3 * i + 1], ph = rtp[3 * i + 2];
     key_r[i] = sortable_bits(r);
+    if (rcol) rcol[i] = r;
     idx[i] = (uint32_t)i;
     int64_t p = 0;
     if (isfinite(th) && isfinite(ph)) {
@@ -351,49 +353,7 @@ __global__ __launch_bounds__(256) void k_win_sum(int64_t npix, const MapInfo* __
 // ---------------------------------------------------------------------------
 constexpr int SELL_SIGMA = 1024;
 
-__global__ void k_sell_keys(int64_t npix, const int32_t* __restrict__ pstart, uint32_t* __restrict__ key,
-                            uint32_t* __restrict__ val)
-{
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npix) return;
-    const int32_t cnt = pstart[p + 1] - pstart[p];
-    key[p] = ((uint32_t)(p / SELL_SIGMA) << 16) | (uint32_t)(0xffff - min(cnt, 0xffff));
-    val[p] = (uint32_t)p;
-}
-
-// slice widths 64 * (largest count among the slice's pixels) and the inverse
-// pixel permutation; one thread per slice
-// One wavefront per slice, one lane per slice row: the pixel, its inverse position,
-// its (pixel, galaxy count) and the slice width 64 * (largest count in the slice).
-__global__ __launch_bounds__(256) void k_sell_slices(int64_t npix, int32_t nslice, const uint32_t* __restrict__ perm,
-                                                     const int32_t* __restrict__ pstart, int64_t* __restrict__ width,
-                                                     uint32_t* __restrict__ invperm, int2* __restrict__ pinfo,
-                                                     int32_t* __restrict__ smin)
-{
-    const int32_t s = (int32_t)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const int lane = threadIdx.x & 63;
-    if (s >= nslice) return;  // whole wavefronts leave together
-    const int64_t e = 64 * (int64_t)s + lane;
-    int32_t c = 0;
-    if (e < npix) {
-        const uint32_t p = perm[e];
-        invperm[p] = (uint32_t)e;
-        c = pstart[p + 1] - pstart[p];
-        pinfo[e] = make_int2((int)p, c);
-    } else {  // lanes past the last pixel: no pixel, no galaxies
-        pinfo[e] = make_int2(0, 0);
-    }
-    int32_t cmin = c;  // the fullest and the emptiest lane of the slice
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        c = max(c, __shfl_xor(c, o, 64));
-        cmin = min(cmin, __shfl_xor(cmin, o, 64));
-    }
-    if (lane == 0) {
-        width[s] = 64 * (int64_t)c;
-        smin[s] = cmin;
-    }
-}
+#include "pixel_sort.h"
 
 // separable window: the pixel factor of every slice lane, win_a[pixel] (0 past npix)
 __global__ void k_slice_win(int64_t nlane, int64_t npix, const int2* __restrict__ pinfo,
@@ -448,13 +408,13 @@ __global__ void k_sell_fill(int64_t N, const uint32_t* __restrict__ pix_s, const
 }
 
 // padding of the T = *Tdev slots (r = -inf, w = 0: they add an exact +-0 to every pixel
-// sum); flag[2] = 1 when T exceeds the capacity tcap
+// sum); flag[2] bit 0 when T exceeds the capacity tcap
 __global__ void k_sell_pad(int64_t tcap, const int64_t* __restrict__ Tdev, double* __restrict__ sr,
                            double* __restrict__ sw, int32_t* __restrict__ flag)
 {
     const int64_t T = *Tdev;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0 && T > tcap) flag[2] = 1;
+    if (i == 0 && T > tcap) atomicOr(flag + 2, 1);
     if (i >= min(T, tcap)) return;
     sr[i] = -INFINITY;
     sw[i] = 0.0;
@@ -2962,7 +2922,10 @@ struct sfb_plan {
     int32_t sell_nslice = 0;
     int64_t sell_cap = 0;   // capacity of the sliced layout's slot arrays (the slot total's bound)
     int64_t sell_hint = 0;  // the exact slot total of a call that overflowed the bound
-    DevBuf d_skey, d_skey2, d_sval, d_perm, d_invperm, d_swidth, d_soff, d_sr, d_sw;
+    DevBuf d_invperm, d_swidth, d_soff, d_sr, d_sw;
+    DevBuf d_cnt;            // galaxies per pixel and per scan chunk
+    bool crowded = false;    // a catalogue crowded a pixel: group by radix sorts
+    const uint32_t* cat_idx = nullptr;  // the last catalogue's input indices, by pixel
     DevBuf d_smin;  // per slice: the smallest galaxy count of its lanes
     DevBuf d_pinfo, d_pwin;  // per slice lane: (pixel, count), separable window factor
     DevBuf d_vgm, d_vgs, d_vrange;  // adjoint gather: group-ordered maps, group starts, map ranges
@@ -3695,7 +3658,7 @@ extern "C" void sfb_plan_destroy(sfb_plan* P)
                       &P->d_pix, &P->d_pixkey, &P->d_pixkey2, &P->d_rs, &P->d_ws, &P->d_pstart, &P->d_sorttmp,
                       &P->h_rtp, &P->h_w, &P->h_wa, &P->h_wb, &P->h_out,
                       &P->d_desc_synf, &P->d_part, &P->h_cot, &P->h_dr, &P->h_dw,
-                      &P->d_skey, &P->d_skey2, &P->d_sval, &P->d_perm, &P->d_invperm, &P->d_swidth, &P->d_smin, &P->d_soff,
+                      &P->d_cnt, &P->d_invperm, &P->d_swidth, &P->d_smin, &P->d_soff,
                       &P->d_sr, &P->d_sw, &P->d_groups, &P->d_gx, &P->d_grh, &P->d_rec4, &P->d_qorder,
                       &P->d_it_i, &P->d_it_t, &P->d_sblk, &P->d_sblk32, &P->d_rec4f, &P->d_swf, &P->d_pinfo,
                       &P->d_pwin, &P->d_vgm, &P->d_vgs, &P->d_vrange, &P->d_lamw, &P->d_desc_cal,
@@ -3729,109 +3692,138 @@ extern "C" int sfb_plan_set_precision(sfb_plan* P, int32_t precision)
     return SFB_OK;
 }
 
-// Sort the catalogue and build the pixel segments.  Leaves r_s, w_s, pstart and,
-// when the records fit in LDS, the sliced layout sr, sw (soff, perm).  sort_r: galaxies
-// of a pixel in the reference's order (by r, then input order: the FP64 path's bit-exact
-// sums); without it in input order (one sort fewer).
+// Order of the galaxies inside a pixel: any (per-galaxy results), by input index, or by
+// (r, input index), the reference's summation order (the FP64 path's bit-exact sums).
+enum CatOrder { CAT_ANY = 0, CAT_INPUT = 1, CAT_RADIUS = 2 };
+
+// Groups the catalogue by pixel (cat_idx, pstart).  slots: also pixel, r and w in that order
+// and, when the records fit in LDS, the sliced layout sr, sw (soff, pinfo); without them
+// (the shells' spread) the radii go to d_rs as one column in input order.  The adjoint's
+// gather takes r and w in order without the sliced layout (gather only).
 static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const double* d_w, hipStream_t st,
-                         bool sort_r = true)
+                         CatOrder order, bool slots, bool gather)
 {
     int rc;
     if (N > 0x7fffffff) return fail(SFB_ERR_ARG, "N > 2^31-1 galaxies");
     P->ncat = N;
     P->unit_w = d_w == nullptr;
     if ((rc = P->d_pstart.ensure(sizeof(int32_t) * (size_t)(P->npix + 1)))) return rc;
-    hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P->d_flag.as<int32_t>(), 4, 0);
-    LAUNCH_CHECK();
     if (N == 0) {
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P->d_flag.as<int32_t>(), 4, 0);
+        LAUNCH_CHECK();
         hipLaunchKernelGGL(k_fill_i32, dim3(nblk(P->npix + 1, 256)), dim3(256), 0, st, P->d_pstart.as<int32_t>(),
                            P->npix + 1, 0);
         LAUNCH_CHECK();
-        if ((rc = P->d_rs.ensure(8)) || (rc = P->d_ws.ensure(8))) return rc;
+        if ((rc = P->d_rs.ensure(8)) || (rc = P->d_ws.ensure(8)) || (rc = P->d_idx.ensure(4))) return rc;
+        P->cat_idx = P->d_idx.as<uint32_t>();
         P->sell_empty = true;  // the scatter takes the per-pixel kernel: delta = -W
         return SFB_OK;
     }
     P->sell_empty = false;
     size_t n = (size_t)N;
     if ((rc = P->d_keyr.ensure(8 * n)) || (rc = P->d_keyr2.ensure(8 * n)) || (rc = P->d_idx.ensure(4 * n)) ||
-        (rc = P->d_idx2.ensure(4 * n)) || (rc = P->d_pix.ensure(4 * n)) || (rc = P->d_pixkey.ensure(4 * n)) ||
-        (rc = P->d_pixkey2.ensure(4 * n)) || (rc = P->d_rs.ensure(8 * n)) || (rc = P->d_ws.ensure(8 * n)))
+        (rc = P->d_rs.ensure(8 * n)))
         return rc;
+    if ((slots || gather) && ((rc = P->d_ws.ensure(8 * n)) || (rc = P->d_pixkey2.ensure(4 * n)))) return rc;
+    double* rcol = (slots || gather) ? nullptr : P->d_rs.as<double>();
     PhaseTimer timer(P, SFB_PHASE_CATALOG, st);
-    hipLaunchKernelGGL(k_prep, dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, P->d_keyr.as<uint64_t>(),
-                       P->d_idx.as<uint32_t>(), P->d_pix.as<uint32_t>(), P->d_flag.as<int32_t>());
-    LAUNCH_CHECK();
-    // 1) stable sort by r (sort_r), 2) stable sort by pixel: temporary sizes
-    size_t tmp1 = 0, tmp2 = 0;
-    HIP_TRY(rocprim::radix_sort_pairs(nullptr, tmp1, P->d_keyr.as<uint64_t>(), P->d_keyr2.as<uint64_t>(),
-                                      P->d_idx.as<uint32_t>(), P->d_idx2.as<uint32_t>(), (unsigned)N, 0, 64, st));
-    unsigned pbits = 1;
-    while (((int64_t)1 << pbits) < P->npix) ++pbits;
-    HIP_TRY(rocprim::radix_sort_pairs(nullptr, tmp2, P->d_pixkey.as<uint32_t>(), P->d_pixkey2.as<uint32_t>(),
-                                      P->d_idx2.as<uint32_t>(), P->d_idx.as<uint32_t>(), (unsigned)N, 0, pbits, st));
+    if (!P->crowded && N <= PS_MEAN * P->npix) {
+        const unsigned nb = nblk(P->npix, PS_CHUNK);
+        if ((rc = P->d_cnt.ensure(sizeof(int32_t) * ((size_t)P->npix + nb))) ||
+            (order == CAT_RADIUS && (rc = P->d_sorttmp.ensure(8 * n))))
+            return rc;
+        int32_t* cnt = P->d_cnt.as<int32_t>();
+        int32_t* sums = cnt + P->npix;
+        uint64_t* key = order == CAT_RADIUS ? P->d_sorttmp.as<uint64_t>() : nullptr;
+        hipLaunchKernelGGL(k_zero_counts, dim3(nblk(P->npix, 256)), dim3(256), 0, st, P->npix, cnt,
+                           P->d_flag.as<int32_t>());
+        LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_count, dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, cnt,
+                           P->d_keyr.as<uint2>(), rcol, P->d_flag.as<int32_t>());
+        LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_count_sums, dim3(nb), dim3(256), 0, st, P->npix, cnt, sums,
+                           order == CAT_ANY ? nullptr : P->d_flag.as<int32_t>());
+        LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_count_scan, dim3(nb), dim3(256), 0, st, P->npix, (int32_t)N, cnt, sums,
+                           P->d_pstart.as<int32_t>());
+        LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_place, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_keyr.as<uint2>(),
+                           P->d_pstart.as<int32_t>(), d_rtp, P->d_keyr2.as<uint2>(), key);
+        LAUNCH_CHECK();
+        auto rank = [&](auto kern) -> int {
+            hipLaunchKernelGGL(kern, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_keyr2.as<uint2>(), key,
+                               P->d_pstart.as<int32_t>(), d_rtp, d_w, P->d_idx.as<uint32_t>(),
+                               rcol ? nullptr : P->d_pixkey2.as<uint32_t>(), rcol ? nullptr : P->d_rs.as<double>(),
+                               rcol ? nullptr : P->d_ws.as<double>());
+            LAUNCH_CHECK();
+            return SFB_OK;
+        };
+        rc = order == CAT_RADIUS ? rank(k_rank<CAT_RADIUS>) : order == CAT_INPUT ? rank(k_rank<CAT_INPUT>) : rank(k_rank<CAT_ANY>);
+        if (rc) return rc;
+        P->cat_idx = P->d_idx.as<uint32_t>();
+    } else {
+        // crowded pixels: stable radix sorts, by r (CAT_RADIUS) and by pixel
+        if ((rc = P->d_idx2.ensure(4 * n)) || (rc = P->d_pix.ensure(4 * n)) || (rc = P->d_pixkey.ensure(4 * n)) ||
+            (rc = P->d_pixkey2.ensure(4 * n)))
+            return rc;
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P->d_flag.as<int32_t>(), 4, 0);
+        LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_prep, dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, P->d_keyr.as<uint64_t>(),
+                           P->d_idx.as<uint32_t>(), P->d_pix.as<uint32_t>(), rcol, P->d_flag.as<int32_t>());
+        LAUNCH_CHECK();
+        size_t tmp1 = 0, tmp2 = 0;
+        HIP_TRY(rocprim::radix_sort_pairs(nullptr, tmp1, P->d_keyr.as<uint64_t>(), P->d_keyr2.as<uint64_t>(),
+                                          P->d_idx.as<uint32_t>(), P->d_idx2.as<uint32_t>(), (unsigned)N, 0, 64, st));
+        unsigned pbits = 1;
+        while (((int64_t)1 << pbits) < P->npix) ++pbits;
+        HIP_TRY(rocprim::radix_sort_pairs(nullptr, tmp2, P->d_pixkey.as<uint32_t>(), P->d_pixkey2.as<uint32_t>(),
+                                          P->d_idx2.as<uint32_t>(), P->d_idx.as<uint32_t>(), (unsigned)N, 0, pbits,
+                                          st));
+        // every temporary size is known before the first sort is enqueued: the buffer
+        // is never reallocated under work in flight
+        if ((rc = P->d_sorttmp.ensure(std::max(tmp1, tmp2)))) return rc;
+        if (order == CAT_RADIUS) {
+            tmp1 = P->d_sorttmp.bytes;
+            HIP_TRY(rocprim::radix_sort_pairs(P->d_sorttmp.p, tmp1, P->d_keyr.as<uint64_t>(),
+                                              P->d_keyr2.as<uint64_t>(), P->d_idx.as<uint32_t>(),
+                                              P->d_idx2.as<uint32_t>(), (unsigned)N, 0, 64, st));
+            hipLaunchKernelGGL(k_gather_pix, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_idx2.as<uint32_t>(),
+                               P->d_pix.as<uint32_t>(), P->d_pixkey.as<uint32_t>());
+            LAUNCH_CHECK();
+            tmp2 = P->d_sorttmp.bytes;
+            HIP_TRY(rocprim::radix_sort_pairs(P->d_sorttmp.p, tmp2, P->d_pixkey.as<uint32_t>(),
+                                              P->d_pixkey2.as<uint32_t>(), P->d_idx2.as<uint32_t>(),
+                                              P->d_idx.as<uint32_t>(), (unsigned)N, 0, pbits, st));
+        } else {
+            tmp2 = P->d_sorttmp.bytes;
+            HIP_TRY(rocprim::radix_sort_pairs(P->d_sorttmp.p, tmp2, P->d_pix.as<uint32_t>(),
+                                              P->d_pixkey2.as<uint32_t>(), P->d_idx.as<uint32_t>(),
+                                              P->d_idx2.as<uint32_t>(), (unsigned)N, 0, pbits, st));
+        }
+        P->cat_idx = (order == CAT_RADIUS ? P->d_idx : P->d_idx2).as<uint32_t>();
+        if (!rcol) {
+            hipLaunchKernelGGL(k_gather, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->cat_idx, d_rtp, d_w,
+                               P->d_rs.as<double>(), P->d_ws.as<double>());
+            LAUNCH_CHECK();
+        }
+        hipLaunchKernelGGL(k_pixel_start, dim3(nblk(P->npix + 1, 256)), dim3(256), 0, st, P->npix, N,
+                           P->d_pixkey2.as<uint32_t>(), P->d_pstart.as<int32_t>());
+        LAUNCH_CHECK();
+    }
     // the sliced layout and the shared segment search need a map's records in LDS;
     // otherwise the scatter evaluates per pixel from global memory
-    const bool sell = P->sell_ok;
     P->sell_nslice = (int32_t)((P->npix + 63) / 64);
-    unsigned wbits = 1;
-    while (((int64_t)1 << wbits) <= P->npix / SELL_SIGMA) ++wbits;
-    size_t tmp4 = 0;
-    if (sell) {
-        if ((rc = P->d_skey.ensure(4 * (size_t)P->npix)) || (rc = P->d_skey2.ensure(4 * (size_t)P->npix)) ||
-            (rc = P->d_sval.ensure(4 * (size_t)P->npix)) || (rc = P->d_perm.ensure(4 * (size_t)P->npix)) ||
-            (rc = P->d_invperm.ensure(4 * (size_t)P->npix)) ||
+    if (P->sell_ok && slots) {
+        if ((rc = P->d_invperm.ensure(4 * (size_t)P->npix)) ||
             (rc = P->d_pinfo.ensure(sizeof(int2) * 64 * (size_t)P->sell_nslice)) ||
             (rc = P->d_swidth.ensure(8 * (size_t)P->sell_nslice)) ||
             (rc = P->d_smin.ensure(4 * (size_t)P->sell_nslice)) ||
             (rc = P->d_soff.ensure(8 * (size_t)(P->sell_nslice + 1))))
             return rc;
-        HIP_TRY(rocprim::radix_sort_pairs(nullptr, tmp4, P->d_skey.as<uint32_t>(), P->d_skey2.as<uint32_t>(),
-                                          P->d_sval.as<uint32_t>(), P->d_perm.as<uint32_t>(), (unsigned)P->npix, 0,
-                                          16 + wbits, st));
-    }
-    // every temporary size is known before the first sort is enqueued: the buffer
-    // is never reallocated under work in flight
-    if ((rc = P->d_sorttmp.ensure(std::max(std::max(tmp1, tmp2), tmp4)))) return rc;
-    if (sort_r) {
-        tmp1 = P->d_sorttmp.bytes;
-        HIP_TRY(rocprim::radix_sort_pairs(P->d_sorttmp.p, tmp1, P->d_keyr.as<uint64_t>(), P->d_keyr2.as<uint64_t>(),
-                                          P->d_idx.as<uint32_t>(), P->d_idx2.as<uint32_t>(), (unsigned)N, 0, 64, st));
-        hipLaunchKernelGGL(k_gather_pix, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_idx2.as<uint32_t>(),
-                           P->d_pix.as<uint32_t>(), P->d_pixkey.as<uint32_t>());
-        LAUNCH_CHECK();
-        // 2) stable sort by pixel: (pixel, r, original index) order
-        tmp2 = P->d_sorttmp.bytes;
-        HIP_TRY(rocprim::radix_sort_pairs(P->d_sorttmp.p, tmp2, P->d_pixkey.as<uint32_t>(),
-                                          P->d_pixkey2.as<uint32_t>(), P->d_idx2.as<uint32_t>(),
-                                          P->d_idx.as<uint32_t>(), (unsigned)N, 0, pbits, st));
-    } else {
-        // mixed path: one stable sort by pixel, (pixel, original index) order; its FP64 pixel
-        // sums of FP32 values do not need the reference's order inside a pixel
-        tmp2 = P->d_sorttmp.bytes;
-        HIP_TRY(rocprim::radix_sort_pairs(P->d_sorttmp.p, tmp2, P->d_pix.as<uint32_t>(), P->d_pixkey2.as<uint32_t>(),
-                                          P->d_idx.as<uint32_t>(), P->d_idx2.as<uint32_t>(), (unsigned)N, 0, pbits,
-                                          st));
-    }
-    const uint32_t* sidx = (sort_r ? P->d_idx : P->d_idx2).as<uint32_t>();
-    hipLaunchKernelGGL(k_gather, dim3(nblk(N, 256)), dim3(256), 0, st, N, sidx, d_rtp, d_w, P->d_rs.as<double>(),
-                       P->d_ws.as<double>());
-    LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_pixel_start, dim3(nblk(P->npix + 1, 256)), dim3(256), 0, st, P->npix, N,
-                       P->d_pixkey2.as<uint32_t>(), P->d_pstart.as<int32_t>());
-    LAUNCH_CHECK();
-    if (sell) {
-        // 3) pixel slices: pixels by count inside windows, slice widths, offsets
-        hipLaunchKernelGGL(k_sell_keys, dim3(nblk(P->npix, 256)), dim3(256), 0, st, P->npix,
-                           P->d_pstart.as<int32_t>(), P->d_skey.as<uint32_t>(), P->d_sval.as<uint32_t>());
-        LAUNCH_CHECK();
-        tmp4 = P->d_sorttmp.bytes;
-        HIP_TRY(rocprim::radix_sort_pairs(P->d_sorttmp.p, tmp4, P->d_skey.as<uint32_t>(), P->d_skey2.as<uint32_t>(),
-                                          P->d_sval.as<uint32_t>(), P->d_perm.as<uint32_t>(), (unsigned)P->npix, 0,
-                                          16 + wbits, st));
-        hipLaunchKernelGGL(k_sell_slices, dim3(nblk(64 * (int64_t)P->sell_nslice, 256)), dim3(256), 0, st, P->npix,
-                           P->sell_nslice,
-                           P->d_perm.as<uint32_t>(), P->d_pstart.as<int32_t>(), P->d_swidth.as<int64_t>(),
-                           P->d_invperm.as<uint32_t>(), P->d_pinfo.as<int2>(), P->d_smin.as<int32_t>());
+        // pixel slices: pixels by count inside windows, slice widths, offsets
+        hipLaunchKernelGGL(k_sell_window, dim3(nblk(P->npix, SELL_SIGMA)), dim3(1024), 0, st, P->npix, P->sell_nslice,
+                           P->d_pstart.as<int32_t>(), P->d_swidth.as<int64_t>(), P->d_invperm.as<uint32_t>(),
+                           P->d_pinfo.as<int2>(), P->d_smin.as<int32_t>());
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_scan_i64, dim3(1), dim3(1024), 0, st, P->sell_nslice, P->d_swidth.as<int64_t>(),
                            P->d_soff.as<int64_t>());
@@ -4486,10 +4478,13 @@ static int check_window(const sfb_plan* P, int32_t win_kind, const double* wa, c
     return SFB_OK;
 }
 
-// After a call whose sliced layout overflowed its capacity (flag[2]): the exact slot
-// total becomes the plan's capacity hint (it only grows), for the call to be redone.
-static int take_slot_total(sfb_plan* P)
+// After a call whose sliced layout overflowed its capacity (flag[2] bit 0): the exact slot
+// total becomes the plan's capacity hint (it only grows), for the call to be redone.  Bit 1: a
+// pixel too full for the pairwise rank; the plan groups by radix sorts from then on.
+static int take_slot_total(sfb_plan* P, int32_t over)
 {
+    if (over & 2) P->crowded = true;
+    if (!(over & 1)) return SFB_OK;
     int64_t T = 0;
     HIP_TRY(hipMemcpy(&T, P->d_soff.as<int64_t>() + P->sell_nslice, sizeof(int64_t), hipMemcpyDeviceToHost));
     if (T <= P->sell_cap) return fail(SFB_ERR_ARG, "internal: slot overflow flagged below the capacity");
@@ -4556,7 +4551,7 @@ static int cat2amln_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const d
     // mixed path: FP32 spline values and delta maps, FP32 MFMA for the Jacobi passes
     size_t shp4;
     const bool f32 = P->precision != SFB_PREC_FP64 && polar4_fits(P, sizeof(float), &shp4);
-    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, !f32))) return rc;
+    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, f32 ? CAT_INPUT : CAT_RADIUS, true, true))) return rc;
     if ((rc = scatter_stage(P, nbar, win_kind, d_win_a, d_win_b, st, f32))) return rc;
     if ((rc = sht_stage(P, (int32_t)P->nmaps, st, f32))) return rc;
     {
@@ -4598,7 +4593,7 @@ extern "C" int sfb_cat2amln_device(sfb_plan* P, int64_t N, const double* d_rtp, 
     if (flag[2]) {
         // the sliced layout outgrew its bound (a crowded catalogue): redo the call with the
         // exact slot total, which the plan keeps as the capacity for later calls
-        if ((rc = take_slot_total(P))) return rc;
+        if ((rc = take_slot_total(P, flag[2]))) return rc;
         return sfb_cat2amln_device(P, N, d_rtp, d_w, nbar, win_kind, d_win_a, d_win_b, d_out, stream);
     }
     if (flag[0]) return fail(SFB_ERR_NONFINITE, "AssertionError: all(isfinite.(anlm)) failed");
@@ -4712,7 +4707,7 @@ extern "C" int sfb_cat2amln(sfb_plan* P, int64_t N, const double* rtp, const dou
         }
         // the sliced layout outgrew its bound: the device entry point redoes the call with the
         // exact slot total (inputs already on the device)
-        if ((rc = take_slot_total(P))) return rc;
+        if ((rc = take_slot_total(P, flag[2]))) return rc;
     }
     sfb::clear_error();
     rc = sfb_cat2amln_device(P, N, d_rtp, d_w, nbar, win_kind, d_wa, d_wb, P->h_out.as<double>(), P->stream);
@@ -4737,7 +4732,7 @@ extern "C" int sfb_cat2amln_vjp_device(sfb_plan* P, int64_t N, const double* d_r
     hipStream_t st = stream ? (hipStream_t)stream : P->stream;
     if (N == 0) return SFB_OK;
     int rc;
-    if ((rc = catalog_stage(P, N, d_rtp, d_w, st))) return rc;
+    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, CAT_ANY, false, true))) return rc;
     const int32_t nq = (int32_t)P->nmaps, L = (int32_t)P->lmax;
     // mixed precision (the plan's SFB_PREC_MIXED): FP32 Jacobi recursion, synthesis GEMM,
     // ring synthesis, delta-bar maps and per-galaxy products, FP64 sums; it needs the
@@ -4816,7 +4811,7 @@ extern "C" int sfb_cat2amln_vjp_device(sfb_plan* P, int64_t N, const double* d_r
     }
     const double inv = 1.0 / (nbar * domega);
     hipLaunchKernelGGL(k_vjp_reduce, dim3(nblk(N, 256)), dim3(256), 0, st, N, ngroups, P->d_part.as<double2>(),
-                       P->d_idx.as<uint32_t>(), P->d_ws.as<double>(), inv, d_dr, d_dw);
+                       P->cat_idx, P->d_ws.as<double>(), inv, d_dr, d_dw);
     LAUNCH_CHECK();
     tj.end();
     int32_t flag[2] = {0, 0};  // (the adjoint does not read the sliced layout: its overflow flag is moot)
@@ -5772,14 +5767,14 @@ extern "C" int sfb_delta_map(sfb_plan* P, int64_t N, const double* rtp, const do
     if ((rc = stage_inputs(P, N, rtp, w, win_kind, win_a, win_b, &d_rtp, &d_w, &d_wa, &d_wb))) return rc;
     const bool f32 = P->precision != SFB_PREC_FP64;
     for (int pass = 0; pass < 2; ++pass) {
-        if ((rc = catalog_stage(P, N, d_rtp, d_w, P->stream, !f32))) return rc;
+        if ((rc = catalog_stage(P, N, d_rtp, d_w, P->stream, f32 ? CAT_INPUT : CAT_RADIUS, true, true))) return rc;
         if ((rc = scatter_stage(P, nbar, win_kind, d_wa, d_wb, P->stream, f32))) return rc;
         int32_t over = 0;
         HIP_TRY(hipMemcpyAsync(&over, P->d_flag.as<int32_t>() + 2, sizeof(int32_t), hipMemcpyDeviceToHost, P->stream));
         HIP_TRY(hipStreamSynchronize(P->stream));
         if (!over) break;
         if (pass == 1) return fail(SFB_ERR_ARG, "internal: slot overflow after resizing");
-        if ((rc = take_slot_total(P))) return rc;
+        if ((rc = take_slot_total(P, over))) return rc;
     }
     if (f32) {
         std::vector<float> m32((size_t)P->npix);
