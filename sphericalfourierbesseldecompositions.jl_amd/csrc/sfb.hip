@@ -33,9 +33,11 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <future>
 #include <mutex>
 #include <new>
 #include <string>
+#include <system_error>
 #include <vector>
 
 #include "sfb_internal.h"
@@ -2863,6 +2865,21 @@ struct DirectSht {
     }
 };
 
+#include "shells_kernels.h"
+
+// Device tables of the mixed path's radial basis (shells.h).
+struct Shells {
+    bool ok = false;
+    int32_t nc = 0;  // basis functions
+    DevBuf d_knots, d_recip, d_gamma;
+    void release()
+    {
+        d_knots.release();
+        d_recip.release();
+        d_gamma.release();
+    }
+};
+
 struct sfb_plan {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -2887,6 +2904,7 @@ struct sfb_plan {
     DevBuf d_maps, d_kx, d_seg, d_rings, d_tw, d_lam, d_lamT, d_outbase, d_aoff, d_desc_ana, d_desc_syn, d_flag;
     // work
     DevBuf d_delta, d_X0, d_G, d_R, d_a, d_a1, d_a2, d_ic0;
+    Shells shells;                 // the mixed path's common radial basis
     DirectSht dir;                 // map2alm with its refinements as one operator
     DevBuf d_mono;                 // mixed path: monopole partial sums and window sums
     DevBuf d_desc_synf;            // full synthesis a -> X0 (all ring pairs), per a buffer
@@ -3569,6 +3587,7 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
 
 extern "C" const char* sfb_version(void) { return "sfb_mi355x 0.1 (gfx950)"; }
 
+static int shells_tables(sfb_plan* P, const sfb::RadialBasis& R, bool fitted);  // shells.h
 static int autotune_phi(sfb_plan* P);  // plan-time phi-transform tile search (defined below)
 
 extern "C" int sfb_plan_create(sfb_plan** out, int64_t nside, int64_t lmax, int64_t nmax, const int64_t* lmax_n,
@@ -3636,7 +3655,17 @@ extern "C" int sfb_plan_create(sfb_plan** out, int64_t nside, int64_t lmax, int6
         delete P;
         return fail(SFB_ERR_DEVICE, "hipStreamCreate failed: %s", hipGetErrorString(e));
     }
+    // the radial fit runs on host threads beside the plan's other tables
+    sfb::RadialBasis basis;
+    auto fit_basis = [&]() { return sfb::radial_basis(nmaps, knot_off, knot_x, knot_y, knot_ypp, &basis); };
+    std::future<bool> fit;
+    try {
+        fit = std::async(std::launch::async, fit_basis);
+    } catch (const std::system_error&) {  // no thread to spare
+    }
     int rc = plan_tables(P, lmax_n, knot_off, knot_x, knot_y, knot_ypp);
+    const bool fitted = fit.valid() ? fit.get() : fit_basis();
+    if (!rc) rc = shells_tables(P, basis, fitted && P->dir.ok);
     if (!rc) rc = autotune_phi(P);
     if (rc) {
         sfb_plan_destroy(P);
@@ -3669,6 +3698,7 @@ extern "C" void sfb_plan_destroy(sfb_plan* P)
     if (P->bg_exec) (void)hipGraphExecDestroy(P->bg_exec);
     for (DevBuf* b : bufs) b->release();
     P->dir.release();
+    P->shells.release();
     P->pin_in.release();
     P->pin_out.release();
     if (P->stream) (void)hipStreamDestroy(P->stream);
@@ -4541,6 +4571,8 @@ static int monopole_fix(sfb_plan* P, int64_t N, double nbar, int32_t win_kind, c
     return SFB_OK;
 }
 
+#include "shells.h"
+
 // One cat2amln enqueued on stream st with no host synchronisation: its flags (non-finite
 // a_nlm, non-finite angle, slot overflow) are left in d_flag[0..2].
 static int cat2amln_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const double* d_w, double nbar,
@@ -4548,7 +4580,12 @@ static int cat2amln_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const d
                             hipStream_t st)
 {
     int rc;
-    // mixed path: FP32 spline values and delta maps, FP32 MFMA for the Jacobi passes
+    // mixed path on the plan's radial basis.  It needs a window that is one map times w_ln (a
+    // dense one has a map per (n, l) anyway); the split-BF16 precisions keep the per-map
+    // pipeline, whose Jacobi products they select.
+    if (P->precision == SFB_PREC_MIXED && P->shells.ok && win_kind == SFB_WIN_SEPARABLE)
+        return shells_enqueue(P, N, d_rtp, d_w, nbar, d_win_a, d_win_b, d_out, st);
+    // else FP32 spline values and delta maps, FP32 MFMA for the Jacobi passes
     size_t shp4;
     const bool f32 = P->precision != SFB_PREC_FP64 && polar4_fits(P, sizeof(float), &shp4);
     if ((rc = catalog_stage(P, N, d_rtp, d_w, st, f32 ? CAT_INPUT : CAT_RADIUS, true, true))) return rc;

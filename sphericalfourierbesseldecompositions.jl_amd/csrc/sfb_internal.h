@@ -39,6 +39,23 @@ int spline_build(int64_t n, const double* x, const double* y, double* ypp);
 double spline_eval(int64_t n, const double* x, const double* y, const double* ypp, double r);
 double spline_deriv(int64_t n, const double* x, const double* y, const double* ypp, double r);
 
+// The common radial basis of the mixed path (radial.cpp): nc clamped B-splines of degree
+// RADIAL_DEGREE on niv intervals, t their nc + RADIAL_DEGREE + 1 knots, gamma[q nc + s] the
+// coefficients of map q's spline.  radial_basis returns false when the maps' knots do not share
+// their ends, the basis would exceed RADIAL_MAX functions, or a spline is further than
+// RADIAL_TOL of its largest value from its representation (half an FP32 unit: what the
+// per-map path's FP32 records lose); err is the largest such distance.
+constexpr int RADIAL_DEGREE = 9;
+constexpr int64_t RADIAL_MAX = 448;
+constexpr double RADIAL_TOL = 5.9604644775390625e-8;
+struct RadialBasis {
+    int nc = 0, niv = 0;
+    std::vector<double> t, gamma;
+    double err = 0.0;
+};
+bool radial_basis(int64_t nmaps, const int64_t* off, const double* kx, const double* ky, const double* kypp,
+                  RadialBasis* out);
+
 // Fault injection for the error-path tests, from the environment variable SFB_FAULT:
 // "alloc" makes every device allocation fail (SFB_ERR_DEVICE), "maxevals" gives the k_nl
 // root finder no evaluations (the reference's doublesecant_method returns NaN after
