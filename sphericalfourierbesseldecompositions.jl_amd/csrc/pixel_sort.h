@@ -20,15 +20,15 @@ __global__ __launch_bounds__(256) void k_zero_counts(int64_t npix, int32_t* __re
     if (i < 4) flag[i] = 0;
 }
 
-// pixel and arrival rank of every galaxy; rcol (or NULL) takes the radii as one column.
+// pixel and arrival rank of every galaxy.
 // flag[1] |= 1 when an angle is not finite (the reference's floor(Int, NaN) throws).
 __global__ __launch_bounds__(256) void k_count(int64_t N, const double* __restrict__ rtp, int64_t nside,
                                                int32_t* __restrict__ cnt, uint2* __restrict__ pr,
-                                               double* __restrict__ rcol, int32_t* __restrict__ flag)
+                                               int32_t* __restrict__ flag)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
-    const double r = rtp[3 * i], th = rtp[3 * i + 1], ph = rtp[3 * i + 2];
+    const double th = rtp[3 * i + 1], ph = rtp[3 * i + 2];
     int64_t p = 0;
     if (isfinite(th) && isfinite(ph)) {
         p = ang2pix_ring_dev(nside, th, ph);
@@ -37,7 +37,6 @@ __global__ __launch_bounds__(256) void k_count(int64_t N, const double* __restri
         atomicOr(flag + 1, 1);
     }
     pr[i] = make_uint2((uint32_t)p, (uint32_t)atomicAdd(cnt + p, 1));
-    if (rcol) rcol[i] = r;
 }
 
 // per PS_CHUNK pixels: their galaxies, and the crowding flag
@@ -99,56 +98,63 @@ __global__ __launch_bounds__(256) void k_count_scan(int64_t npix, int32_t N, con
     if (blockIdx.x == 0 && t == 0) pstart[npix] = N;
 }
 
-// galaxy i to its place by arrival: (i, pixel) and, for an order by r, its sort key
+// A galaxy at its place by arrival: everything the rank pass needs in one 32-byte sector, so
+// the scattered writes touch one sector per galaxy (index and pixel placed alone, with the rank
+// pass gathering r and w from the catalogue, ran 17 + 25 us at N = 1e6 and 64 + 166 us at 4e6).
+struct alignas(32) CatSlot {
+    double r, w;
+    uint32_t i, pix;
+};
+
 __global__ __launch_bounds__(256) void k_place(int64_t N, const uint2* __restrict__ pr,
                                                const int32_t* __restrict__ pstart, const double* __restrict__ rtp,
-                                               uint2* __restrict__ slot, uint64_t* __restrict__ key)
+                                               const double* __restrict__ w, CatSlot* __restrict__ slot)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     const uint2 q = pr[i];
-    const int64_t at = (int64_t)pstart[q.x] + q.y;
-    slot[at] = make_uint2((uint32_t)i, q.x);
-    if (key) key[at] = sortable_bits(rtp[3 * i]);
+    CatSlot c;
+    c.r = rtp[3 * i];
+    c.w = w ? w[i] : 1.0;
+    c.i = (uint32_t)i;
+    c.pix = q.x;
+    slot[(int64_t)pstart[q.x] + q.y] = c;
 }
 
 // order inside a pixel: 0 as placed (where any order does), 1 by input index, 2 by (r, input
-// index), the order of the reference's sums.  Writes the sorted list of input indices and,
-// when asked, pixel, r and w in that order.
+// index), the order of the reference's sums.  Writes the sorted list of input indices, and
+// pixel, r and w in that order.
 template <int ORDER>
-__global__ __launch_bounds__(256) void k_rank(int64_t N, const uint2* __restrict__ slot,
-                                              const uint64_t* __restrict__ key, const int32_t* __restrict__ pstart,
-                                              const double* __restrict__ rtp, const double* __restrict__ w,
-                                              uint32_t* __restrict__ idx, uint32_t* __restrict__ pix_s,
-                                              double* __restrict__ r_s, double* __restrict__ w_s)
+__global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restrict__ slot,
+                                              const int32_t* __restrict__ pstart, uint32_t* __restrict__ idx,
+                                              uint32_t* __restrict__ pix_s, double* __restrict__ r_s,
+                                              double* __restrict__ w_s)
 {
     const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (e >= N) return;
-    const uint2 me = slot[e];
+    const CatSlot me = slot[e];
     int64_t f = e;
     if (ORDER) {
-        const int32_t s0 = pstart[me.y], s1 = pstart[me.y + 1];
+        const int32_t s0 = pstart[me.pix], s1 = pstart[me.pix + 1];
         if (s1 - s0 <= PS_CROWD) {  // (fuller: the call is redone)
-            const uint64_t k = ORDER == 2 ? key[e] : 0;
+            const uint64_t k = sortable_bits(me.r);
             int32_t before = 0;
             for (int32_t s = s0; s < s1; ++s) {
-                const uint32_t i = slot[s].x;
+                const uint32_t i = slot[s].i;
                 if (ORDER == 2) {
-                    const uint64_t ks = key[s];
-                    before += ks < k || (ks == k && i < me.x);
+                    const uint64_t ks = sortable_bits(slot[s].r);
+                    before += ks < k || (ks == k && i < me.i);
                 } else {
-                    before += i < me.x;
+                    before += i < me.i;
                 }
             }
             f = (int64_t)s0 + before;
         }
     }
-    idx[f] = me.x;
-    if (pix_s) pix_s[f] = me.y;
-    if (r_s) {
-        r_s[f] = rtp[3 * (int64_t)me.x];
-        w_s[f] = w ? w[me.x] : 1.0;
-    }
+    idx[f] = me.i;
+    pix_s[f] = me.pix;
+    r_s[f] = me.r;
+    w_s[f] = me.w;
 }
 
 // Slices of the sliced layout from the counts: one block per window of SELL_SIGMA pixels sorts

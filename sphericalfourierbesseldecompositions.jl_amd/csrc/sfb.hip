@@ -149,14 +149,12 @@ __device__ __forceinline__ uint64_t sortable_bits(double v)
 
 // flag[1] |= 1 when an angle is not finite (the reference's floor(Int, NaN) throws).
 __global__ void k_prep(int64_t N, const double* __restrict__ rtp, int64_t nside, uint64_t* __restrict__ key_r,
-                       uint32_t* __restrict__ idx, uint32_t* __restrict__ pix, double* __restrict__ rcol,
-                       int32_t* __restrict__ flag)
+                       uint32_t* __restrict__ idx, uint32_t* __restrict__ pix, int32_t* __restrict__ flag)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
     double r = rtp[3 * i], th = rtp[3 * i + 1], ph = rtp[3 * i + 2];
     key_r[i] = sortable_bits(r);
-    if (rcol) rcol[i] = r;
     idx[i] = (uint32_t)i;
     int64_t p = 0;
     if (isfinite(th) && isfinite(ph)) {
@@ -2855,11 +2853,11 @@ struct DirectSht {
     int32_t maxN = 1, maxNs = 1, maxNf = 1;
     int64_t hrows = 0;
     std::vector<int32_t> s0, na, ka;  // per m: first state, states, first ring pair
-    DevBuf d_lamP, d_lamPT, d_HB, d_GZ, d_UB, d_ZB, d_Q, d_qoff, d_st, d_term, d_h, d_r;
+    DevBuf d_lamP, d_lamPT, d_HB, d_GZ, d_UB, d_ZB, d_Q, d_qoff, d_st, d_term, d_h, d_r, d_one;
     DevBuf d_ana, d_fix, d_syn, d_sfix;
     void release()
     {
-        DevBuf* b[] = {&d_lamP, &d_lamPT, &d_HB, &d_GZ, &d_UB, &d_ZB, &d_Q, &d_qoff, &d_st, &d_term, &d_h, &d_r,
+        DevBuf* b[] = {&d_lamP, &d_lamPT, &d_HB, &d_GZ, &d_UB, &d_ZB, &d_Q, &d_qoff, &d_st, &d_term, &d_h, &d_r, &d_one,
                        &d_ana, &d_fix, &d_syn, &d_sfix};
         for (DevBuf* x : b) x->release();
     }
@@ -2871,12 +2869,13 @@ struct DirectSht {
 struct Shells {
     bool ok = false;
     int32_t nc = 0;  // basis functions
-    DevBuf d_knots, d_recip, d_gamma;
+    DevBuf d_knots, d_gamma, d_lstart, d_lq;  // gamma by l and shell; the maps of each l
     void release()
     {
         d_knots.release();
-        d_recip.release();
         d_gamma.release();
+        d_lstart.release();
+        d_lq.release();
     }
 };
 
@@ -3726,12 +3725,11 @@ extern "C" int sfb_plan_set_precision(sfb_plan* P, int32_t precision)
 // (r, input index), the reference's summation order (the FP64 path's bit-exact sums).
 enum CatOrder { CAT_ANY = 0, CAT_INPUT = 1, CAT_RADIUS = 2 };
 
-// Groups the catalogue by pixel (cat_idx, pstart).  slots: also pixel, r and w in that order
-// and, when the records fit in LDS, the sliced layout sr, sw (soff, pinfo); without them
-// (the shells' spread) the radii go to d_rs as one column in input order.  The adjoint's
-// gather takes r and w in order without the sliced layout (gather only).
+// Groups the catalogue by pixel: cat_idx, pstart, and pixel, r and w in that order; slots: also
+// the sliced layout sr, sw (soff, pinfo) when the records fit in LDS (the per-map scatter reads
+// it; the shells' spread and the adjoint's gather do not).
 static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const double* d_w, hipStream_t st,
-                         CatOrder order, bool slots, bool gather)
+                         CatOrder order, bool slots)
 {
     int rc;
     if (N > 0x7fffffff) return fail(SFB_ERR_ARG, "N > 2^31-1 galaxies");
@@ -3751,25 +3749,22 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
     }
     P->sell_empty = false;
     size_t n = (size_t)N;
-    if ((rc = P->d_keyr.ensure(8 * n)) || (rc = P->d_keyr2.ensure(8 * n)) || (rc = P->d_idx.ensure(4 * n)) ||
-        (rc = P->d_rs.ensure(8 * n)))
+    if ((rc = P->d_keyr.ensure(8 * n)) || (rc = P->d_idx.ensure(4 * n)) ||
+        (rc = P->d_rs.ensure(8 * n)) || (rc = P->d_ws.ensure(8 * n)) || (rc = P->d_pixkey2.ensure(4 * n)))
         return rc;
-    if ((slots || gather) && ((rc = P->d_ws.ensure(8 * n)) || (rc = P->d_pixkey2.ensure(4 * n)))) return rc;
-    double* rcol = (slots || gather) ? nullptr : P->d_rs.as<double>();
     PhaseTimer timer(P, SFB_PHASE_CATALOG, st);
     if (!P->crowded && N <= PS_MEAN * P->npix) {
         const unsigned nb = nblk(P->npix, PS_CHUNK);
         if ((rc = P->d_cnt.ensure(sizeof(int32_t) * ((size_t)P->npix + nb))) ||
-            (order == CAT_RADIUS && (rc = P->d_sorttmp.ensure(8 * n))))
+            (rc = P->d_sorttmp.ensure(sizeof(CatSlot) * n)))
             return rc;
         int32_t* cnt = P->d_cnt.as<int32_t>();
         int32_t* sums = cnt + P->npix;
-        uint64_t* key = order == CAT_RADIUS ? P->d_sorttmp.as<uint64_t>() : nullptr;
         hipLaunchKernelGGL(k_zero_counts, dim3(nblk(P->npix, 256)), dim3(256), 0, st, P->npix, cnt,
                            P->d_flag.as<int32_t>());
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_count, dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, cnt,
-                           P->d_keyr.as<uint2>(), rcol, P->d_flag.as<int32_t>());
+                           P->d_keyr.as<uint2>(), P->d_flag.as<int32_t>());
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_count_sums, dim3(nb), dim3(256), 0, st, P->npix, cnt, sums,
                            order == CAT_ANY ? nullptr : P->d_flag.as<int32_t>());
@@ -3778,28 +3773,28 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
                            P->d_pstart.as<int32_t>());
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_place, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_keyr.as<uint2>(),
-                           P->d_pstart.as<int32_t>(), d_rtp, P->d_keyr2.as<uint2>(), key);
+                           P->d_pstart.as<int32_t>(), d_rtp, d_w, P->d_sorttmp.as<CatSlot>());
         LAUNCH_CHECK();
         auto rank = [&](auto kern) -> int {
-            hipLaunchKernelGGL(kern, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_keyr2.as<uint2>(), key,
-                               P->d_pstart.as<int32_t>(), d_rtp, d_w, P->d_idx.as<uint32_t>(),
-                               rcol ? nullptr : P->d_pixkey2.as<uint32_t>(), rcol ? nullptr : P->d_rs.as<double>(),
-                               rcol ? nullptr : P->d_ws.as<double>());
+            hipLaunchKernelGGL(kern, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_sorttmp.as<CatSlot>(),
+                               P->d_pstart.as<int32_t>(), P->d_idx.as<uint32_t>(), P->d_pixkey2.as<uint32_t>(),
+                               P->d_rs.as<double>(), P->d_ws.as<double>());
             LAUNCH_CHECK();
             return SFB_OK;
         };
-        rc = order == CAT_RADIUS ? rank(k_rank<CAT_RADIUS>) : order == CAT_INPUT ? rank(k_rank<CAT_INPUT>) : rank(k_rank<CAT_ANY>);
+        rc = order == CAT_RADIUS  ? rank(k_rank<CAT_RADIUS>)
+             : order == CAT_INPUT ? rank(k_rank<CAT_INPUT>)
+                                  : rank(k_rank<CAT_ANY>);
         if (rc) return rc;
         P->cat_idx = P->d_idx.as<uint32_t>();
     } else {
         // crowded pixels: stable radix sorts, by r (CAT_RADIUS) and by pixel
-        if ((rc = P->d_idx2.ensure(4 * n)) || (rc = P->d_pix.ensure(4 * n)) || (rc = P->d_pixkey.ensure(4 * n)) ||
-            (rc = P->d_pixkey2.ensure(4 * n)))
+        if ((rc = P->d_keyr2.ensure(8 * n)) || (rc = P->d_idx2.ensure(4 * n)) || (rc = P->d_pix.ensure(4 * n)) || (rc = P->d_pixkey.ensure(4 * n)))
             return rc;
         hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P->d_flag.as<int32_t>(), 4, 0);
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_prep, dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, P->d_keyr.as<uint64_t>(),
-                           P->d_idx.as<uint32_t>(), P->d_pix.as<uint32_t>(), rcol, P->d_flag.as<int32_t>());
+                           P->d_idx.as<uint32_t>(), P->d_pix.as<uint32_t>(), P->d_flag.as<int32_t>());
         LAUNCH_CHECK();
         size_t tmp1 = 0, tmp2 = 0;
         HIP_TRY(rocprim::radix_sort_pairs(nullptr, tmp1, P->d_keyr.as<uint64_t>(), P->d_keyr2.as<uint64_t>(),
@@ -3831,11 +3826,9 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
                                               P->d_idx2.as<uint32_t>(), (unsigned)N, 0, pbits, st));
         }
         P->cat_idx = (order == CAT_RADIUS ? P->d_idx : P->d_idx2).as<uint32_t>();
-        if (!rcol) {
-            hipLaunchKernelGGL(k_gather, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->cat_idx, d_rtp, d_w,
-                               P->d_rs.as<double>(), P->d_ws.as<double>());
-            LAUNCH_CHECK();
-        }
+        hipLaunchKernelGGL(k_gather, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->cat_idx, d_rtp, d_w,
+                           P->d_rs.as<double>(), P->d_ws.as<double>());
+        LAUNCH_CHECK();
         hipLaunchKernelGGL(k_pixel_start, dim3(nblk(P->npix + 1, 256)), dim3(256), 0, st, P->npix, N,
                            P->d_pixkey2.as<uint32_t>(), P->d_pstart.as<int32_t>());
         LAUNCH_CHECK();
@@ -4588,7 +4581,7 @@ static int cat2amln_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const d
     // else FP32 spline values and delta maps, FP32 MFMA for the Jacobi passes
     size_t shp4;
     const bool f32 = P->precision != SFB_PREC_FP64 && polar4_fits(P, sizeof(float), &shp4);
-    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, f32 ? CAT_INPUT : CAT_RADIUS, true, true))) return rc;
+    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, f32 ? CAT_INPUT : CAT_RADIUS, true))) return rc;
     if ((rc = scatter_stage(P, nbar, win_kind, d_win_a, d_win_b, st, f32))) return rc;
     if ((rc = sht_stage(P, (int32_t)P->nmaps, st, f32))) return rc;
     {
@@ -4769,7 +4762,7 @@ extern "C" int sfb_cat2amln_vjp_device(sfb_plan* P, int64_t N, const double* d_r
     hipStream_t st = stream ? (hipStream_t)stream : P->stream;
     if (N == 0) return SFB_OK;
     int rc;
-    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, CAT_ANY, false, true))) return rc;
+    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, CAT_ANY, false))) return rc;
     const int32_t nq = (int32_t)P->nmaps, L = (int32_t)P->lmax;
     // mixed precision (the plan's SFB_PREC_MIXED): FP32 Jacobi recursion, synthesis GEMM,
     // ring synthesis, delta-bar maps and per-galaxy products, FP64 sums; it needs the
@@ -5804,7 +5797,7 @@ extern "C" int sfb_delta_map(sfb_plan* P, int64_t N, const double* rtp, const do
     if ((rc = stage_inputs(P, N, rtp, w, win_kind, win_a, win_b, &d_rtp, &d_w, &d_wa, &d_wb))) return rc;
     const bool f32 = P->precision != SFB_PREC_FP64;
     for (int pass = 0; pass < 2; ++pass) {
-        if ((rc = catalog_stage(P, N, d_rtp, d_w, P->stream, f32 ? CAT_INPUT : CAT_RADIUS, true, true))) return rc;
+        if ((rc = catalog_stage(P, N, d_rtp, d_w, P->stream, f32 ? CAT_INPUT : CAT_RADIUS, true))) return rc;
         if ((rc = scatter_stage(P, nbar, win_kind, d_wa, d_wb, P->stream, f32))) return rc;
         int32_t over = 0;
         HIP_TRY(hipMemcpyAsync(&over, P->d_flag.as<int32_t>() + 2, sizeof(int32_t), hipMemcpyDeviceToHost, P->stream));

@@ -222,6 +222,7 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
     HIP_TRY(hipStreamSynchronize(P->stream));  // done before the scratch is freed
     // launch descriptors.  Sector sg of block (m, par): l parity sg = (m + par) & 1.
     std::vector<RowGemm> ana, fix, syn, sfix;
+    D.hrows = 2 * (int64_t)J * S;
     D.maxN = D.maxNs = D.maxNf = 1;
     for (int64_t b = 0; b < nbat; ++b) {
         const int64_t m = b / 2, n = P->nb[(size_t)b], kc = P->kcut[(size_t)m];
@@ -277,6 +278,20 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
         sfix.push_back(f);
         D.maxNf = std::max<int32_t>(D.maxNf, (int32_t)n);
     }
+    {
+        // one more row of h: sum over the ring pairs of the m = 0 coefficients, the maps' pixel
+        // sums (the mixed path's monopoles)
+        const std::vector<double> one((size_t)K, 1.0);
+        if ((rc = D.d_one.ensure(sizeof(double) * one.size()))) return rc;
+        HIP_TRY(hipMemcpy(D.d_one.p, one.data(), sizeof(double) * one.size(), hipMemcpyHostToDevice));
+        RowGemm d{};
+        d.ncol = -1;
+        d.crow = D.hrows;
+        d.dst = d.N = d.ldb = 1;
+        d.K = K;
+        d.B = D.d_one.as<double>();
+        ana.push_back(d);
+    }
     struct { DevBuf* d; std::vector<RowGemm>* v; int32_t* n; } up[] = {
         {&D.d_ana, &ana, &D.n_ana}, {&D.d_fix, &fix, &D.n_fix}, {&D.d_syn, &syn, &D.n_syn}, {&D.d_sfix, &sfix, &D.n_sfix}};
     for (auto& u : up) {
@@ -285,8 +300,7 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
         if (!u.v->empty())
             HIP_TRY(hipMemcpy(u.d->p, u.v->data(), sizeof(RowGemm) * u.v->size(), hipMemcpyHostToDevice));
     }
-    D.hrows = 2 * (int64_t)J * S;
-    if ((rc = D.d_h.ensure(dbl(D.hrows * P->M2))) || (rc = D.d_r.ensure(dbl(D.hrows * P->M2)))) return rc;
+    if ((rc = D.d_h.ensure(dbl((D.hrows + 1) * P->M2))) || (rc = D.d_r.ensure(dbl(D.hrows * P->M2)))) return rc;
     D.s0 = s0;
     D.na = na;
     D.ka = ka;
