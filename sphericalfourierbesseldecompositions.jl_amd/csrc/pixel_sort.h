@@ -20,8 +20,9 @@ __global__ __launch_bounds__(256) void k_zero_counts(int64_t npix, int32_t* __re
     if (i < 4) flag[i] = 0;
 }
 
-// pixel and arrival rank of every galaxy.
+// pixel (FOLD: folded, with the hemisphere in bit 0) and arrival rank of every galaxy.
 // flag[1] |= 1 when an angle is not finite (the reference's floor(Int, NaN) throws).
+template <bool FOLD>
 __global__ __launch_bounds__(256) void k_count(int64_t N, const double* __restrict__ rtp, int64_t nside,
                                                int32_t* __restrict__ cnt, uint2* __restrict__ pr,
                                                int32_t* __restrict__ flag)
@@ -36,7 +37,8 @@ __global__ __launch_bounds__(256) void k_count(int64_t N, const double* __restri
     } else {
         atomicOr(flag + 1, 1);
     }
-    pr[i] = make_uint2((uint32_t)p, (uint32_t)atomicAdd(cnt + p, 1));
+    const uint32_t f = FOLD ? fold_pixel(p, nside) : (uint32_t)p;
+    pr[i] = make_uint2(f, (uint32_t)atomicAdd(cnt + (FOLD ? f >> 1 : f), 1));
 }
 
 // per PS_CHUNK pixels: their galaxies, and the crowding flag
@@ -108,7 +110,7 @@ struct alignas(32) CatSlot {
 
 __global__ __launch_bounds__(256) void k_place(int64_t N, const uint2* __restrict__ pr,
                                                const int32_t* __restrict__ pstart, const double* __restrict__ rtp,
-                                               const double* __restrict__ w, CatSlot* __restrict__ slot)
+                                               const double* __restrict__ w, int32_t sh, CatSlot* __restrict__ slot)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
@@ -118,15 +120,17 @@ __global__ __launch_bounds__(256) void k_place(int64_t N, const uint2* __restric
     c.w = w ? w[i] : 1.0;
     c.i = (uint32_t)i;
     c.pix = q.x;
-    slot[(int64_t)pstart[q.x] + q.y] = c;
+    slot[(int64_t)pstart[q.x >> sh] + q.y] = c;
 }
 
 // order inside a pixel: 0 as placed (where any order does), 1 by input index, 2 by (r, input
-// index), the order of the reference's sums.  Writes the sorted list of input indices, and
+// index), the order of the reference's sums; in a folded pixel northern galaxies first, as the
+// radix sorts leave them.  Writes the sorted list of input indices, and
 // pixel, r and w in that order.
 template <int ORDER>
 __global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restrict__ slot,
-                                              const int32_t* __restrict__ pstart, uint32_t* __restrict__ idx,
+                                              const int32_t* __restrict__ pstart, int32_t sh,
+                                              uint32_t* __restrict__ idx,
                                               uint32_t* __restrict__ pix_s, double* __restrict__ r_s,
                                               double* __restrict__ w_s)
 {
@@ -135,17 +139,17 @@ __global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restri
     const CatSlot me = slot[e];
     int64_t f = e;
     if (ORDER) {
-        const int32_t s0 = pstart[me.pix], s1 = pstart[me.pix + 1];
+        const int32_t s0 = pstart[me.pix >> sh], s1 = pstart[(me.pix >> sh) + 1];
         if (s1 - s0 <= PS_CROWD) {  // (fuller: the call is redone)
             const uint64_t k = sortable_bits(me.r);
             int32_t before = 0;
             for (int32_t s = s0; s < s1; ++s) {
-                const uint32_t i = slot[s].i;
+                const uint32_t i = slot[s].i, ps = slot[s].pix;
                 if (ORDER == 2) {
                     const uint64_t ks = sortable_bits(slot[s].r);
-                    before += ks < k || (ks == k && i < me.i);
+                    before += ps < me.pix || (ps == me.pix && (ks < k || (ks == k && i < me.i)));
                 } else {
-                    before += i < me.i;
+                    before += ps < me.pix || (ps == me.pix && i < me.i);
                 }
             }
             f = (int64_t)s0 + before;

@@ -147,9 +147,33 @@ __device__ __forceinline__ uint64_t sortable_bits(double v)
     return (b >> 63) ? ~b : (b | 0x8000000000000000ull);
 }
 
+// southern pixel -> folded pixel f and the flag 1, northern and equatorial ones -> (p, 0): f << 1 | flag
+__device__ __forceinline__ uint32_t fold_pixel(int64_t p, int64_t nside)
+{
+    const int64_t npix = 12 * nside * nside, npf = 6 * nside * nside + 2 * nside;
+    if (p < npf) return (uint32_t)p << 1;
+    const int64_t pm = npix - 1 - p, ncap = 2 * nside * (nside - 1);  // the mirror pixel, counted backwards in its ring
+    int64_t start, npr;
+    if (pm < ncap) {
+        int64_t i = (int64_t)((1.0 + sqrt(1.0 + 2.0 * (double)pm)) * 0.5);
+        while (2 * i * (i - 1) > pm) --i;
+        while (2 * i * (i + 1) <= pm) ++i;
+        start = 2 * i * (i - 1);
+        npr = 4 * i;
+    } else {
+        npr = 4 * nside;
+        start = ncap + (pm - ncap) / npr * npr;
+    }
+    const int64_t js = npr - 1 - (pm - start);  // pixel in the southern ring
+    int64_t j = js + npr / 2;
+    if (j >= npr) j -= npr;
+    return ((uint32_t)(start + j) << 1) | 1u;
+}
+
 // flag[1] |= 1 when an angle is not finite (the reference's floor(Int, NaN) throws).
 __global__ void k_prep(int64_t N, const double* __restrict__ rtp, int64_t nside, uint64_t* __restrict__ key_r,
-                       uint32_t* __restrict__ idx, uint32_t* __restrict__ pix, int32_t* __restrict__ flag)
+                       uint32_t* __restrict__ idx, uint32_t* __restrict__ pix, int32_t* __restrict__ flag,
+                       bool fold)
 {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
@@ -163,7 +187,7 @@ __global__ void k_prep(int64_t N, const double* __restrict__ rtp, int64_t nside,
     } else {
         atomicOr(flag + 1, 1);
     }
-    pix[i] = (uint32_t)p;
+    pix[i] = fold ? fold_pixel(p, nside) : (uint32_t)p;
 }
 
 __global__ void k_ang2pix(int64_t N, const double* __restrict__ th, const double* __restrict__ ph, int64_t nside,
@@ -194,14 +218,14 @@ __global__ void k_gather(int64_t N, const uint32_t* __restrict__ idx, const doub
 
 // pstart[p] = first sorted galaxy with pixel >= p, p = 0..npix.
 __global__ void k_pixel_start(int64_t npix, int64_t N, const uint32_t* __restrict__ pix_sorted,
-                              int32_t* __restrict__ pstart)
+                              int32_t sh, int32_t* __restrict__ pstart)
 {
     int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (p > npix) return;
     int64_t lo = 0, hi = N;
     while (lo < hi) {
         int64_t mid = (lo + hi) >> 1;
-        if ((int64_t)pix_sorted[mid] < p) lo = mid + 1;
+        if ((int64_t)(pix_sorted[mid] >> sh) < p) lo = mid + 1;
         else hi = mid;
     }
     pstart[p] = (int32_t)lo;
@@ -394,17 +418,18 @@ __global__ __launch_bounds__(1024) void k_scan_i64(int32_t n, const int64_t* __r
 __global__ void k_sell_fill(int64_t N, const uint32_t* __restrict__ pix_s, const int32_t* __restrict__ pstart,
                             const uint32_t* __restrict__ invperm, const int64_t* __restrict__ soff,
                             const double* __restrict__ r_s, const double* __restrict__ w_s, double* __restrict__ sr,
-                            double* __restrict__ sw, int64_t tcap)
+                            double* __restrict__ sw, int64_t tcap, int32_t sh, uint8_t* __restrict__ ss)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= N) return;
-    const uint32_t p = pix_s[k];
+    const uint32_t p = pix_s[k] >> sh;
     const int64_t j = k - pstart[p];
     const uint32_t e = invperm[p];
     const int64_t dst = soff[e >> 6] + 64 * j + (e & 63);
     if (dst >= tcap) return;
     sr[dst] = r_s[k];
     sw[dst] = w_s[k];
+    if (sh) ss[dst] = (uint8_t)(pix_s[k] & 1u);  // folded maps: a southern galaxy
 }
 
 // padding of the T = *Tdev slots (r = -inf, w = 0: they add an exact +-0 to every pixel
@@ -453,7 +478,7 @@ __global__ __launch_bounds__(1024) void k_seg_t(int64_t Tcap, const int64_t* __r
                                                const double* __restrict__ sr,
                                                const GroupInfo* __restrict__ groups, const double* __restrict__ gx,
                                                const double* __restrict__ grh, uint16_t* __restrict__ it_i,
-                                               TT* __restrict__ it_t)
+                                               TT* __restrict__ it_t, const uint8_t* __restrict__ ss)
 {
     extern __shared__ double sm_seg[];
     const int64_t T = min(*Tdev, Tcap);
@@ -472,10 +497,12 @@ __global__ __launch_bounds__(1024) void k_seg_t(int64_t Tcap, const int64_t* __r
     TT* ot = it_t + (int64_t)g * Tcap;
     for (int64_t eb = e0 + threadIdx.x; eb < e1; eb += 4 * (int64_t)blockDim.x) {
         double rr[4];
+        bool south[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int64_t e = eb + u * (int64_t)blockDim.x;
             rr[u] = e < e1 ? sr[e] : 0.0;
+            south[u] = ss && e < e1 && (ss[e] & 1);
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -510,6 +537,9 @@ __global__ __launch_bounds__(1024) void k_seg_t(int64_t Tcap, const int64_t* __r
                 i = 0;
                 t = r;
             }
+            // folded maps: t's sign carries the hemisphere (t >= 0 otherwise, and the boundary
+            // records' slopes are 0)
+            if (ss) t = south[u] ? -fabs(t) : fabs(t);
             oi[e] = (uint16_t)i;
             ot[e] = (TT)t;
         }
@@ -628,7 +658,11 @@ __device__ __forceinline__ void load_rows(RowLoad<UNIT, R>& L, __amdgpu_buffer_r
 // radii (it_r) are resolved by seg_uniform against record tables staged one slot up.
 // TS > 0: the tables' stride in records as a constant (tstride <= TS), so a row's gathers
 // from its NM tables share one address register and carry the table offsets as immediates.
-template <bool DENSE, int NM, bool UNIT, typename R, bool SPLIT = false, bool ONFLY = false, int TS = 0>
+// FOLD (FP64): pixels are folded ones (fold_kernels.h); t's sign bit marks a southern galaxy,
+// which odd-l maps subtract, and the window factors are the folded sums of each l parity (pwin's
+// halves; a dense window's two pixels).
+template <bool DENSE, int NM, bool UNIT, typename R, bool SPLIT = false, bool ONFLY = false, int TS = 0,
+          bool FOLD = false>
 __global__ __launch_bounds__(1024) void k_scatter_it(int64_t npix, int32_t nslice, int32_t spc, int64_t Tcap,
                                                      const int64_t* __restrict__ Tdev, const double* __restrict__ msel,
                                                      const ScatterBlock* __restrict__ blk, int32_t per_xcd,
@@ -643,8 +677,10 @@ __global__ __launch_bounds__(1024) void k_scatter_it(int64_t npix, int32_t nslic
                                                      const double* __restrict__ win_b, int64_t lmax,
                                                      R* __restrict__ delta, int32_t slot_order,
                                                      const float* __restrict__ reclo,
-                                                     const double* __restrict__ it_r)
+                                                     const double* __restrict__ it_r,
+                                                     const int32_t* __restrict__ south, int64_t nwin)
 {
+    static_assert(!FOLD || (sizeof(R) == 8 && !SPLIT && !ONFLY), "folded maps: the FP64 kernel");
     static_assert(!ONFLY || sizeof(R) == 4, "radii resolved in the scatter: FP32 records only");
     static_assert(TS == 0 || (sizeof(R) == 4 && !SPLIT), "constant stride: FP32 records only");
     typedef typename Vec4T<R>::T R4;
@@ -660,6 +696,7 @@ __global__ __launch_bounds__(1024) void k_scatter_it(int64_t npix, int32_t nslic
     bool has[NM];
     int64_t col[NM];
     double wcol[NM];
+    uint32_t odd[NM];  // FOLD: the sign bit for odd l
     const R4* tab[NM];
     int pad = 0;
     int nkm1 = 0;  // ONFLY: the group's uniform knots (nk - 1 segments, x0, 1/H)
@@ -686,6 +723,7 @@ __global__ __launch_bounds__(1024) void k_scatter_it(int64_t npix, int32_t nslic
         // TS: a missing map reads its own (unstaged, in-bounds) table and writes nothing
         tab[k] = sm4 + (TS ? k : (has[k] ? k : 0)) * tstride;
         col[k] = m.l + (lmax + 1) * (int64_t)(m.n - 1);
+        odd[k] = FOLD ? (uint32_t)__builtin_amdgcn_readfirstlane(m.l & 1) << 31 : 0u;
         wcol[k] = DENSE ? 0.0 : win_b[col[k]];
     }
     const __amdgpu_buffer_rsrc_t gi = ONFLY ? slot_rsrc(it_r, (uint32_t)(8 * T))
@@ -715,12 +753,21 @@ __global__ __launch_bounds__(1024) void k_scatter_it(int64_t npix, int32_t nslic
         st.pc = pinfo[e];
         st.minc = __builtin_amdgcn_readfirstlane(smin[min(sl, nslice - 1)]);
 #pragma unroll
-        for (int k = 0; k < NM; ++k) st.w[k] = DENSE ? 0.0 : pwin[e];
+        for (int k = 0; k < NM; ++k) st.w[k] = DENSE ? 0.0 : pwin[FOLD && odd[k] ? e + 64 * (int64_t)nslice : e];
     };
     auto load_dense_w = [&](SliceSt& st) {  // needs st.pc: issued when the slice starts
         if (DENSE)
 #pragma unroll
-            for (int k = 0; k < NM; ++k) st.w[k] = win_a[st.pc.x + npix * col[k]];
+            for (int k = 0; k < NM; ++k) {
+                if (!FOLD) {
+                    st.w[k] = win_a[st.pc.x + npix * col[k]];
+                } else {  // (win_a's columns hold the whole sky's nwin pixels)
+                    const int64_t o = nwin * col[k];
+                    const int sp = south[st.pc.x];
+                    const double v = sp >= 0 ? win_a[o + sp] : 0.0;
+                    st.w[k] = win_a[o + st.pc.x] + (odd[k] ? -v : v);
+                }
+            }
     };
     // per-pixel sums in FP64 on both paths (FP32 spline values are widened exactly)
     double acc[NM];
@@ -822,7 +869,7 @@ __global__ __launch_bounds__(1024) void k_scatter_it(int64_t npix, int32_t nslic
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             if (r + u > rlast) break;
-            const R t = cur.t[u];
+            const R t = FOLD ? (R)fabs((double)cur.t[u]) : cur.t[u];
             if (SPLIT) {
                 // g = d_hi + (d_lo + t (c + t (b + t a))): the FP32 part rounds once, relative to
                 // t c; d_hi and that part are added in FP64
@@ -842,6 +889,12 @@ __global__ __launch_bounds__(1024) void k_scatter_it(int64_t npix, int32_t nslic
                 R v[NM];
 #pragma unroll
                 for (int k = 0; k < NM; ++k) v[k] = fma(t, fma(t, fma(t, c[u][k].w, c[u][k].z), c[u][k].y), c[u][k].x);
+                if constexpr (FOLD) {
+                    const uint32_t sg = (uint32_t)__double2hiint(cur.t[u]);
+#pragma unroll
+                    for (int k = 0; k < NM; ++k)
+                        v[k] = __hiloint2double(__double2hiint(v[k]) ^ (int)(sg & odd[k]), __double2loint(v[k]));
+                }
                 if (UNIT && r + u - first >= cs.minc) {  // wave-uniform: some lane is past its galaxies
                     const bool live = r + u - first < cs.pc.y;
 #pragma unroll
@@ -2853,6 +2906,7 @@ struct DirectSht {
     int32_t maxN = 1, maxNs = 1, maxNf = 1;
     int64_t hrows = 0;
     std::vector<int32_t> s0, na, ka;  // per m: first state, states, first ring pair
+    std::vector<int64_t> hboff, voff;  // per (m, parity): table offsets
     DevBuf d_lamP, d_lamPT, d_HB, d_GZ, d_UB, d_ZB, d_Q, d_qoff, d_st, d_term, d_h, d_r, d_one;
     DevBuf d_ana, d_fix, d_syn, d_sfix;
     void release()
@@ -2863,7 +2917,23 @@ struct DirectSht {
     }
 };
 
+#include "fold_kernels.h"
 #include "shells_kernels.h"
+
+// Tables and launch shapes of the folded FP64 path (fold.h).
+struct Fold {
+    bool ok = false;
+    int64_t npf = 0;               // northern and equatorial pixels
+    int32_t neven = 0, maxcnt = 1, n_h = 0, maxh = 1;
+    int32_t tq = 1, tqi[2] = {1, 1}, tqp = 1;  // maps per FFT block, inverse (FP64, FP32), inverse polar (fewest)
+    size_t shi = 0;
+    DevBuf d_cols, d_m, d_h, d_south, d_gzoff;
+    void release()
+    {
+        DevBuf* b[] = {&d_cols, &d_m, &d_h, &d_south, &d_gzoff};
+        for (DevBuf* x : b) x->release();
+    }
+};
 
 // Device tables of the mixed path's radial basis (shells.h).
 struct Shells {
@@ -2903,6 +2973,7 @@ struct sfb_plan {
     DevBuf d_maps, d_kx, d_seg, d_rings, d_tw, d_lam, d_lamT, d_outbase, d_aoff, d_desc_ana, d_desc_syn, d_flag;
     // work
     DevBuf d_delta, d_X0, d_G, d_R, d_a, d_a1, d_a2, d_ic0;
+    Fold fold;                     // the folded FP64 path
     Shells shells;                 // the mixed path's common radial basis
     DirectSht dir;                 // map2alm with its refinements as one operator
     DevBuf d_mono;                 // mixed path: monopole partial sums and window sums
@@ -2942,6 +3013,9 @@ struct sfb_plan {
     DevBuf d_invperm, d_swidth, d_soff, d_sr, d_sw;
     DevBuf d_cnt;            // galaxies per pixel and per scan chunk
     bool crowded = false;    // a catalogue crowded a pixel: group by radix sorts
+    int64_t cat_np = 0;      // pixels of the last catalogue's grouping (npix, or npf folded)
+    bool cat_fold = false;   // ... with southern pixels folded onto northern ones
+    DevBuf d_ss;             // folded sliced layout: 1 where a slot's galaxy is southern
     const uint32_t* cat_idx = nullptr;  // the last catalogue's input indices, by pixel
     DevBuf d_smin;  // per slice: the smallest galaxy count of its lanes
     DevBuf d_pinfo, d_pwin;  // per slice lane: (pixel, count), separable window factor
@@ -3587,6 +3661,7 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
 extern "C" const char* sfb_version(void) { return "sfb_mi355x 0.1 (gfx950)"; }
 
 static int shells_tables(sfb_plan* P, const sfb::RadialBasis& R, bool fitted);  // shells.h
+static int fold_tables(sfb_plan* P);    // fold.h
 static int autotune_phi(sfb_plan* P);  // plan-time phi-transform tile search (defined below)
 
 extern "C" int sfb_plan_create(sfb_plan** out, int64_t nside, int64_t lmax, int64_t nmax, const int64_t* lmax_n,
@@ -3665,6 +3740,7 @@ extern "C" int sfb_plan_create(sfb_plan** out, int64_t nside, int64_t lmax, int6
     int rc = plan_tables(P, lmax_n, knot_off, knot_x, knot_y, knot_ypp);
     const bool fitted = fit.valid() ? fit.get() : fit_basis();
     if (!rc) rc = shells_tables(P, basis, fitted && P->dir.ok);
+    if (!rc) rc = fold_tables(P);
     if (!rc) rc = autotune_phi(P);
     if (rc) {
         sfb_plan_destroy(P);
@@ -3686,7 +3762,7 @@ extern "C" void sfb_plan_destroy(sfb_plan* P)
                       &P->d_pix, &P->d_pixkey, &P->d_pixkey2, &P->d_rs, &P->d_ws, &P->d_pstart, &P->d_sorttmp,
                       &P->h_rtp, &P->h_w, &P->h_wa, &P->h_wb, &P->h_out,
                       &P->d_desc_synf, &P->d_part, &P->h_cot, &P->h_dr, &P->h_dw,
-                      &P->d_cnt, &P->d_invperm, &P->d_swidth, &P->d_smin, &P->d_soff,
+                      &P->d_cnt, &P->d_ss, &P->d_invperm, &P->d_swidth, &P->d_smin, &P->d_soff,
                       &P->d_sr, &P->d_sw, &P->d_groups, &P->d_gx, &P->d_grh, &P->d_rec4, &P->d_qorder,
                       &P->d_it_i, &P->d_it_t, &P->d_sblk, &P->d_sblk32, &P->d_rec4f, &P->d_swf, &P->d_pinfo,
                       &P->d_pwin, &P->d_vgm, &P->d_vgs, &P->d_vrange, &P->d_lamw, &P->d_desc_cal,
@@ -3698,6 +3774,7 @@ extern "C" void sfb_plan_destroy(sfb_plan* P)
     for (DevBuf* b : bufs) b->release();
     P->dir.release();
     P->shells.release();
+    P->fold.release();
     P->pin_in.release();
     P->pin_out.release();
     if (P->stream) (void)hipStreamDestroy(P->stream);
@@ -3725,13 +3802,31 @@ extern "C" int sfb_plan_set_precision(sfb_plan* P, int32_t precision)
 // (r, input index), the reference's summation order (the FP64 path's bit-exact sums).
 enum CatOrder { CAT_ANY = 0, CAT_INPUT = 1, CAT_RADIUS = 2 };
 
+// Capacity of the sliced layout's slot arrays.  The slot total T stays on the device (no host
+// round trip).  Pixels are sorted by count inside each window of 1024, so a slice is never
+// wider than the previous slice's mean count, and T <= N + 64 x (the largest count of every
+// window); the bound takes the Poisson tail of a uniform catalogue's largest count (or the
+// exact T of an earlier call that overflowed).
+constexpr int64_t SELL_MAX = (int64_t)1 << 29;  // 8 x slots < 2^32 (32-bit slot offsets)
+static int64_t sell_bound(const sfb_plan* P, int64_t N, int64_t np)
+{
+    const int64_t nwin = (np + SELL_SIGMA - 1) / SELL_SIGMA;
+    const double cbar = (double)N / (double)np;
+    const int64_t cmax = (int64_t)(cbar + 8.0 * std::sqrt(cbar) + 16.0);
+    return std::max<int64_t>(N + 64 * nwin * cmax, P->sell_hint);
+}
+
 // Groups the catalogue by pixel: cat_idx, pstart, and pixel, r and w in that order; slots: also
 // the sliced layout sr, sw (soff, pinfo) when the records fit in LDS (the per-map scatter reads
-// it; the shells' spread and the adjoint's gather do not).
+// it; the shells' spread and the adjoint's gather do not).  fold: by folded pixel (fold_pixel).
 static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const double* d_w, hipStream_t st,
-                         CatOrder order, bool slots)
+                         CatOrder order, bool slots, bool fold = false)
 {
     int rc;
+    const int64_t np = fold ? P->fold.npf : P->npix;
+    const int32_t sh = fold ? 1 : 0;  // folded pixels carry the hemisphere in bit 0
+    P->cat_np = np;
+    P->cat_fold = fold;
     if (N > 0x7fffffff) return fail(SFB_ERR_ARG, "N > 2^31-1 galaxies");
     P->ncat = N;
     P->unit_w = d_w == nullptr;
@@ -3753,31 +3848,31 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         (rc = P->d_rs.ensure(8 * n)) || (rc = P->d_ws.ensure(8 * n)) || (rc = P->d_pixkey2.ensure(4 * n)))
         return rc;
     PhaseTimer timer(P, SFB_PHASE_CATALOG, st);
-    if (!P->crowded && N <= PS_MEAN * P->npix) {
-        const unsigned nb = nblk(P->npix, PS_CHUNK);
-        if ((rc = P->d_cnt.ensure(sizeof(int32_t) * ((size_t)P->npix + nb))) ||
+    if (!P->crowded && N <= PS_MEAN * np) {
+        const unsigned nb = nblk(np, PS_CHUNK);
+        if ((rc = P->d_cnt.ensure(sizeof(int32_t) * ((size_t)np + nb))) ||
             (rc = P->d_sorttmp.ensure(sizeof(CatSlot) * n)))
             return rc;
         int32_t* cnt = P->d_cnt.as<int32_t>();
-        int32_t* sums = cnt + P->npix;
-        hipLaunchKernelGGL(k_zero_counts, dim3(nblk(P->npix, 256)), dim3(256), 0, st, P->npix, cnt,
+        int32_t* sums = cnt + np;
+        hipLaunchKernelGGL(k_zero_counts, dim3(nblk(np, 256)), dim3(256), 0, st, np, cnt,
                            P->d_flag.as<int32_t>());
         LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_count, dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, cnt,
+        hipLaunchKernelGGL((fold ? k_count<true> : k_count<false>), dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, cnt,
                            P->d_keyr.as<uint2>(), P->d_flag.as<int32_t>());
         LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_count_sums, dim3(nb), dim3(256), 0, st, P->npix, cnt, sums,
+        hipLaunchKernelGGL(k_count_sums, dim3(nb), dim3(256), 0, st, np, cnt, sums,
                            order == CAT_ANY ? nullptr : P->d_flag.as<int32_t>());
         LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_count_scan, dim3(nb), dim3(256), 0, st, P->npix, (int32_t)N, cnt, sums,
+        hipLaunchKernelGGL(k_count_scan, dim3(nb), dim3(256), 0, st, np, (int32_t)N, cnt, sums,
                            P->d_pstart.as<int32_t>());
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_place, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_keyr.as<uint2>(),
-                           P->d_pstart.as<int32_t>(), d_rtp, d_w, P->d_sorttmp.as<CatSlot>());
+                           P->d_pstart.as<int32_t>(), d_rtp, d_w, sh, P->d_sorttmp.as<CatSlot>());
         LAUNCH_CHECK();
         auto rank = [&](auto kern) -> int {
             hipLaunchKernelGGL(kern, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_sorttmp.as<CatSlot>(),
-                               P->d_pstart.as<int32_t>(), P->d_idx.as<uint32_t>(), P->d_pixkey2.as<uint32_t>(),
+                               P->d_pstart.as<int32_t>(), sh, P->d_idx.as<uint32_t>(), P->d_pixkey2.as<uint32_t>(),
                                P->d_rs.as<double>(), P->d_ws.as<double>());
             LAUNCH_CHECK();
             return SFB_OK;
@@ -3794,13 +3889,13 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P->d_flag.as<int32_t>(), 4, 0);
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_prep, dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, P->d_keyr.as<uint64_t>(),
-                           P->d_idx.as<uint32_t>(), P->d_pix.as<uint32_t>(), P->d_flag.as<int32_t>());
+                           P->d_idx.as<uint32_t>(), P->d_pix.as<uint32_t>(), P->d_flag.as<int32_t>(), fold);
         LAUNCH_CHECK();
         size_t tmp1 = 0, tmp2 = 0;
         HIP_TRY(rocprim::radix_sort_pairs(nullptr, tmp1, P->d_keyr.as<uint64_t>(), P->d_keyr2.as<uint64_t>(),
                                           P->d_idx.as<uint32_t>(), P->d_idx2.as<uint32_t>(), (unsigned)N, 0, 64, st));
         unsigned pbits = 1;
-        while (((int64_t)1 << pbits) < P->npix) ++pbits;
+        while (((int64_t)1 << pbits) < (np << sh)) ++pbits;
         HIP_TRY(rocprim::radix_sort_pairs(nullptr, tmp2, P->d_pixkey.as<uint32_t>(), P->d_pixkey2.as<uint32_t>(),
                                           P->d_idx2.as<uint32_t>(), P->d_idx.as<uint32_t>(), (unsigned)N, 0, pbits,
                                           st));
@@ -3829,39 +3924,32 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         hipLaunchKernelGGL(k_gather, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->cat_idx, d_rtp, d_w,
                            P->d_rs.as<double>(), P->d_ws.as<double>());
         LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_pixel_start, dim3(nblk(P->npix + 1, 256)), dim3(256), 0, st, P->npix, N,
-                           P->d_pixkey2.as<uint32_t>(), P->d_pstart.as<int32_t>());
+        hipLaunchKernelGGL(k_pixel_start, dim3(nblk(np + 1, 256)), dim3(256), 0, st, np, N,
+                           P->d_pixkey2.as<uint32_t>(), sh, P->d_pstart.as<int32_t>());
         LAUNCH_CHECK();
     }
     // the sliced layout and the shared segment search need a map's records in LDS;
     // otherwise the scatter evaluates per pixel from global memory
-    P->sell_nslice = (int32_t)((P->npix + 63) / 64);
+    P->sell_nslice = (int32_t)((np + 63) / 64);
     if (P->sell_ok && slots) {
-        if ((rc = P->d_invperm.ensure(4 * (size_t)P->npix)) ||
+        if ((rc = P->d_invperm.ensure(4 * (size_t)np)) ||
             (rc = P->d_pinfo.ensure(sizeof(int2) * 64 * (size_t)P->sell_nslice)) ||
             (rc = P->d_swidth.ensure(8 * (size_t)P->sell_nslice)) ||
             (rc = P->d_smin.ensure(4 * (size_t)P->sell_nslice)) ||
             (rc = P->d_soff.ensure(8 * (size_t)(P->sell_nslice + 1))))
             return rc;
         // pixel slices: pixels by count inside windows, slice widths, offsets
-        hipLaunchKernelGGL(k_sell_window, dim3(nblk(P->npix, SELL_SIGMA)), dim3(1024), 0, st, P->npix, P->sell_nslice,
+        hipLaunchKernelGGL(k_sell_window, dim3(nblk(np, SELL_SIGMA)), dim3(1024), 0, st, np, P->sell_nslice,
                            P->d_pstart.as<int32_t>(), P->d_swidth.as<int64_t>(), P->d_invperm.as<uint32_t>(),
                            P->d_pinfo.as<int2>(), P->d_smin.as<int32_t>());
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_scan_i64, dim3(1), dim3(1024), 0, st, P->sell_nslice, P->d_swidth.as<int64_t>(),
                            P->d_soff.as<int64_t>());
         LAUNCH_CHECK();
-        // The slot total T stays on the device (no host round trip): the slot arrays get a
-        // capacity from a bound.  Pixels are sorted by count inside each window of 1024, so a
-        // slice is never wider than the previous slice's mean count, and T <= N + 64 x (the
-        // largest count of every window); the bound takes the Poisson tail of a uniform
-        // catalogue's largest count (or the exact T of an earlier call that overflowed).
-        const int64_t nwin = (P->npix + SELL_SIGMA - 1) / SELL_SIGMA;
-        const double cbar = (double)N / (double)P->npix;
-        const int64_t cmax = (int64_t)(cbar + 8.0 * std::sqrt(cbar) + 16.0);
-        const int64_t tcap = std::max<int64_t>(N + 64 * nwin * cmax, P->sell_hint);
+        const int64_t tcap = sell_bound(P, N, np);
         P->sell_cap = tcap;
-        P->sell_fits = tcap < ((int64_t)1 << 29);
+        P->sell_fits = tcap < SELL_MAX;
+        if (fold && (rc = P->d_ss.ensure((size_t)tcap))) return rc;
         if ((rc = P->d_sr.ensure(8 * (size_t)tcap)) || (rc = P->d_sw.ensure(8 * (size_t)tcap))) return rc;
         const int64_t* Tdev = P->d_soff.as<int64_t>() + P->sell_nslice;
         hipLaunchKernelGGL(k_sell_pad, dim3(nblk(tcap, 256)), dim3(256), 0, st, tcap, Tdev, P->d_sr.as<double>(),
@@ -3870,7 +3958,7 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         hipLaunchKernelGGL(k_sell_fill, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_pixkey2.as<uint32_t>(),
                            P->d_pstart.as<int32_t>(), P->d_invperm.as<uint32_t>(), P->d_soff.as<int64_t>(),
                            P->d_rs.as<double>(), P->d_ws.as<double>(), P->d_sr.as<double>(), P->d_sw.as<double>(),
-                           tcap);
+                           tcap, sh, P->d_ss.as<uint8_t>());
         LAUNCH_CHECK();
     }
     return SFB_OK;
@@ -3889,17 +3977,27 @@ static int launch_scatter_nm(sfb_plan* P, bool dense, bool unit, dim3 grid, size
 {
     auto go = [&](auto kern) -> int {
         HIP_TRY(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-        hipLaunchKernelGGL(kern, grid, dim3(1024), shm, st, P->npix, P->sell_nslice, spc, T,
+        hipLaunchKernelGGL(kern, grid, dim3(1024), shm, st, P->cat_np, P->sell_nslice, spc, T,
                            P->d_soff.as<int64_t>() + P->sell_nslice, msel, blk, per_xcd, tstride,
                            P->d_pinfo.as<int2>(), P->d_smin.as<int32_t>(), P->d_pwin.as<double>(),
                            P->d_soff.as<int64_t>(), sw,
                            P->d_it_i.as<uint16_t>(), P->d_it_t.as<R>(), P->d_maps.as<MapInfo>(), rec, inv, d_wa,
                            d_wb, P->lmax, P->d_delta.as<R>(), (int32_t)(P->delta_perm != nullptr),
-                           P->d_reclo.as<float>(), P->d_sr.as<double>());
+                           P->d_reclo.as<float>(), P->d_sr.as<double>(), P->fold.d_south.as<int32_t>(),
+                           P->npix);
         LAUNCH_CHECK();
         return SFB_OK;
     };
     constexpr bool F = sizeof(R) == 4;
+    if constexpr (!F) {
+        if (P->cat_fold) {
+            if (dense)
+                return unit ? go(k_scatter_it<true, NM, true, R, false, false, 0, true>)
+                            : go(k_scatter_it<true, NM, false, R, false, false, 0, true>);
+            return unit ? go(k_scatter_it<false, NM, true, R, false, false, 0, true>)
+                        : go(k_scatter_it<false, NM, false, R, false, false, 0, true>);
+        }
+    }
     constexpr int TSC = 2560;  // constant table stride: four FP32 tables fill 160 KiB of LDS
     if constexpr (F && NM == 4 && !SPLIT) {
         const size_t shm_c = (size_t)TSC * sizeof(typename Vec4T<R>::T) * NM;
@@ -4009,7 +4107,7 @@ static int scatter_stage(sfb_plan* P, double nbar, int32_t win_kind, const doubl
         // delta in slot order when the slices tile the pixels exactly (npix a multiple of 64):
         // each slice end stores one contiguous row per map (FP64 4.2 -> 3.5 ms, FP32 2.35 ->
         // 2.10 ms at C2) and the phi-transform gathers through the permutation (+0.14 ms).
-        if (64 * (int64_t)P->sell_nslice == P->npix) P->delta_perm = P->d_invperm.as<uint32_t>();
+        if (64 * (int64_t)P->sell_nslice == P->cat_np) P->delta_perm = P->d_invperm.as<uint32_t>();
         // shared segment search per knot group, then three fma per map and galaxy.  The slot
         // total stays on the device; arrays are sized by the catalogue stage's bound Tcap.
         const int64_t T = std::max<int64_t>(P->sell_cap, 1);
@@ -4038,11 +4136,12 @@ static int scatter_stage(sfb_plan* P, double nbar, int32_t win_kind, const doubl
             if (!onfly)
                 hipLaunchKernelGGL(k_seg_t<float>, gseg, dim3(1024), shm_seg, st, T, Tdev, P->d_sr.as<double>(),
                                    P->d_groups.as<GroupInfo>(), P->d_gx.as<double>(), P->d_grh.as<double>(),
-                                   P->d_it_i.as<uint16_t>(), P->d_it_t.as<float>());
+                                   P->d_it_i.as<uint16_t>(), P->d_it_t.as<float>(), (const uint8_t*)nullptr);
         } else {
             hipLaunchKernelGGL(k_seg_t<double>, gseg, dim3(1024), shm_seg, st, T, Tdev, P->d_sr.as<double>(),
                                P->d_groups.as<GroupInfo>(), P->d_gx.as<double>(), P->d_grh.as<double>(),
-                               P->d_it_i.as<uint16_t>(), P->d_it_t.as<double>());
+                               P->d_it_i.as<uint16_t>(), P->d_it_t.as<double>(),
+                               P->cat_fold ? P->d_ss.as<uint8_t>() : (const uint8_t*)nullptr);
         }
         LAUNCH_CHECK();
         tseg.end();
@@ -4050,9 +4149,13 @@ static int scatter_stage(sfb_plan* P, double nbar, int32_t win_kind, const doubl
         const bool dense = win_kind == SFB_WIN_DENSE;
         if (!dense) {
             const int64_t nlane = 64 * (int64_t)P->sell_nslice;
-            if ((rc = P->d_pwin.ensure(sizeof(double) * (size_t)nlane))) return rc;
-            hipLaunchKernelGGL(k_slice_win, dim3(nblk(nlane, 256)), dim3(256), 0, st, nlane, P->npix,
-                               P->d_pinfo.as<int2>(), d_wa, P->d_pwin.as<double>());
+            if ((rc = P->d_pwin.ensure(sizeof(double) * (size_t)nlane * (P->cat_fold ? 2 : 1)))) return rc;
+            if (P->cat_fold)
+                hipLaunchKernelGGL(k_slice_win_fold, dim3(nblk(nlane, 256)), dim3(256), 0, st, nlane, P->cat_np,
+                                   P->d_pinfo.as<int2>(), P->fold.d_south.as<int32_t>(), d_wa, P->d_pwin.as<double>());
+            else
+                hipLaunchKernelGGL(k_slice_win, dim3(nblk(nlane, 256)), dim3(256), 0, st, nlane, P->npix,
+                                   P->d_pinfo.as<int2>(), d_wa, P->d_pwin.as<double>());
             LAUNCH_CHECK();
         }
         // Mixed path: the FP32 records' rounding is the same for every galaxy in a segment,
@@ -4564,6 +4667,7 @@ static int monopole_fix(sfb_plan* P, int64_t N, double nbar, int32_t win_kind, c
     return SFB_OK;
 }
 
+#include "fold.h"
 #include "shells.h"
 
 // One cat2amln enqueued on stream st with no host synchronisation: its flags (non-finite
@@ -4581,8 +4685,12 @@ static int cat2amln_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const d
     // else FP32 spline values and delta maps, FP32 MFMA for the Jacobi passes
     size_t shp4;
     const bool f32 = P->precision != SFB_PREC_FP64 && polar4_fits(P, sizeof(float), &shp4);
-    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, f32 ? CAT_INPUT : CAT_RADIUS, true))) return rc;
+    // FP64: folded hemispheres when the sliced scatter takes the catalogue (an empty one, or one
+    // beyond its 32-bit slots, goes the unfolded way)
+    const bool fold = !f32 && P->fold.ok && N > 0 && sell_bound(P, N, P->fold.npf) < SELL_MAX;
+    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, f32 ? CAT_INPUT : CAT_RADIUS, true, fold))) return rc;
     if ((rc = scatter_stage(P, nbar, win_kind, d_win_a, d_win_b, st, f32))) return rc;
+    if (fold) return fold_analysis(P, d_out, st);
     if ((rc = sht_stage(P, (int32_t)P->nmaps, st, f32))) return rc;
     {
         PhaseTimer timer(P, SFB_PHASE_PACK, st);

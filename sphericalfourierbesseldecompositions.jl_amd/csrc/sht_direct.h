@@ -302,6 +302,8 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
     }
     if ((rc = D.d_h.ensure(dbl((D.hrows + 1) * P->M2))) || (rc = D.d_r.ensure(dbl(D.hrows * P->M2)))) return rc;
     D.s0 = s0;
+    D.hboff = hboff;
+    D.voff = voff;
     D.na = na;
     D.ka = ka;
     D.ok = true;
