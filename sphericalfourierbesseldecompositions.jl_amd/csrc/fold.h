@@ -174,7 +174,7 @@ template <typename R> static int fold_synthesis(sfb_plan* P, const double* d_cot
         const int rc = direct_alias(P, 2 * nq, ld, st, 2 * F.neven);
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(k_fold_synth<R>, dim3(gx, nblk(K, 32), (unsigned)(L + 1)), dim3(256), 0, st, K, P->niter, nq, ld,
+    hipLaunchKernelGGL(k_fold_synth<R>, dim3(nblk(F.neven, 64) + nblk(nq - F.neven, 64), nblk(K, 32), (unsigned)(L + 1)), dim3(256), 0, st, K, P->niter, nq, ld,
                        F.d_m.as<FoldM>(), F.d_cols.as<FoldCol>(), F.neven, D.d_lamPT.as<double>(), D.d_GZ.as<double>(),
                        F.d_gzoff.as<int64_t>(), D.d_r.as<double>(), d_cot, P->d_X0.as<R>());
     LAUNCH_CHECK();

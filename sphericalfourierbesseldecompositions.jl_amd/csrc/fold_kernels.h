@@ -299,9 +299,9 @@ __global__ __launch_bounds__(256) void k_fold_coth(int32_t J, int32_t ncol, int6
     }
 }
 
-// X_m[k] = (Lam P_J)[k][l] b_m + sum_h GZ[h][k] r_h, m <= mtop.  A block takes one m, 64 columns and
-// 32 ring pairs, a wave 8 of them (the table entries of a wave's ring pairs are wave-uniform).
-// Bound: X written once.
+// X_m[k] = (Lam P_J)[k][l] b_m + sum_h GZ[h][k] r_h, m <= mtop.  A block takes one m, 64 columns of one
+// l parity and 32 ring pairs, a wave 8 of them: the aliasing tables' entries are wave-uniform
+// (scalar loads; per-lane loads of them ran 548 us at nside 128).  Bound: X written once.
 template <typename R>
 __global__ __launch_bounds__(256) void k_fold_synth(int32_t K, int32_t J, int32_t ncol, int64_t ld,
                                                     const FoldM* __restrict__ fm, const FoldCol* __restrict__ cols,
@@ -310,14 +310,15 @@ __global__ __launch_bounds__(256) void k_fold_synth(int32_t K, int32_t J, int32_
                                                     const double* __restrict__ r, const double* __restrict__ cot,
                                                     R* __restrict__ X)
 {
-    const int m = blockIdx.z, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int m = blockIdx.z, lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const FoldM M = fm[m];
-    const int c = blockIdx.x * 64 + lane;
+    const int te = (neven + 63) >> 6;  // tiles of the even maps, then of the odd ones
+    const int pi = (int)blockIdx.x >= te;
+    const int c = (pi ? neven + ((int)blockIdx.x - te) * 64 : (int)blockIdx.x * 64) + lane;
     const int k0 = blockIdx.y * 32 + wv * 8;
-    if (c >= ncol || k0 + 8 <= M.kc || k0 >= K) return;
+    if (c >= (pi ? ncol : neven) || k0 + 8 <= M.kc || k0 >= K) return;
     const FoldCol C = cols[c];
     if (m > C.mtop) return;
-    const int pi = c >= neven;
     double re[8], im[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) re[u] = im[u] = 0.0;
@@ -337,18 +338,27 @@ __global__ __launch_bounds__(256) void k_fold_synth(int32_t K, int32_t J, int32_
                 im[u] = t[u] * b.y;
             }
     }
-    if (M.na > 0) {
+    if (M.na > 0 && M.nb[pi] > 0) {  // ((lmax, odd) has no l, hence no table)
         const double2* rr = (const double2*)(r + (int64_t)J * M.s0 * ld) + c;
         const double* gz = GZ + gzoff[2 * m + ((m + pi) & 1)] + k0;
+        const int ku = min(8, K - k0);  // (K is even; 8 except on grids of fewer ring pairs)
         for (int e = 0; e < J * M.na; ++e) {
             const double2 v = rr[(int64_t)e * (ld >> 1)];
+            const double* w = gz + (int64_t)e * K;
+            if (ku == 8) {
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (k0 + u < K) {
-                    const double w = gz[(int64_t)e * K + u];
-                    re[u] = fma(w, v.x, re[u]);
-                    im[u] = fma(w, v.y, im[u]);
+                for (int u = 0; u < 8; ++u) {
+                    re[u] = fma(w[u], v.x, re[u]);
+                    im[u] = fma(w[u], v.y, im[u]);
                 }
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (u < ku) {
+                        re[u] = fma(w[u], v.x, re[u]);
+                        im[u] = fma(w[u], v.y, im[u]);
+                    }
+            }
         }
     }
     typedef typename Vec2T<R>::T R2;
@@ -562,4 +572,122 @@ __global__ __launch_bounds__(256) void k_phi_ipolar4_fold(const R* __restrict__ 
     if (j1 < ni)
 #pragma unroll
         for (int ss = 0; ss < 4; ++ss) o[4 * j1 + ss] = sc * acc[1][ss];
+}
+
+// Per galaxy and map range blockIdx.y (whole knot groups): part = (sum_q g_q(r) dbar_q, sum_q g'_q(r)
+// dbar_q) on folded delta-bar maps and uniform knots.  Galaxies grouped by folded pixel (a
+// wave's delta-bar loads fall on a few lines); their segment slot and t are found from the radii
+// once per knot group, then NM maps' records are staged in LDS at a time.
+// Value and slope come from one Horner chain (5 fma); the slopes of a group share the segment's
+// 1/h, applied once to their sum.  Outside the knots the pseudo-records' slopes are 0.  R = float: FP32 records,
+// delta-bar and products, FP64 sums.  Bound: the random 16-byte record reads from LDS.
+constexpr int VF_GPT = 6;
+template <typename R, int NM>
+__global__ __launch_bounds__(1024) void k_vjp_fold(int64_t N, int64_t npf, int32_t cap, const double* __restrict__ r_s,
+                                                   const uint32_t* __restrict__ pix_s,
+                                                   const GroupInfo* __restrict__ groups,
+                                                   const double* __restrict__ gx, const double* __restrict__ grh,
+                                                   const int32_t* __restrict__ vgs, const int32_t* __restrict__ vgm,
+                                                   const int2* __restrict__ vrange, const MapInfo* __restrict__ maps,
+                                                   const typename Vec4T<R>::T* __restrict__ rec4,
+                                                   const R* __restrict__ dbar, double2* __restrict__ part)
+{
+    typedef typename Vec4T<R>::T R4;
+    extern __shared__ double4 vf_raw[];
+    R4* tb = (R4*)vf_raw;  // NM tables of cap + 1 records, one slot up: y_first, segments, y_last
+    const int64_t k0 = (int64_t)blockIdx.x * (1024 * VF_GPT) + threadIdx.x;
+    double r[VF_GPT], aw[VF_GPT], ar[VF_GPT];
+    R t[VF_GPT];
+    int ii[VF_GPT];
+    uint32_t pf[VF_GPT], south = 0;
+#pragma unroll
+    for (int u = 0; u < VF_GPT; ++u) {
+        const int64_t k = min(k0 + 1024 * u, N - 1);  // past the end: computed and dropped
+        r[u] = r_s[k];
+        pf[u] = pix_s[k] >> 1;
+        south |= (pix_s[k] & 1u) << u;
+        aw[u] = ar[u] = 0.0;
+    }
+    const int2 rg = vrange[blockIdx.y];
+    for (int g = rg.x; g < rg.y; ++g) {
+        const GroupInfo G = groups[g];
+        const double ainv = G.invdx, c0 = -G.xfirst * G.invdx, top = (double)(G.nk - 1);
+        double gr[VF_GPT];
+#pragma unroll
+        for (int u = 0; u < VF_GPT; ++u) {
+            // the end knots belong to the end segments (their slopes), outside is flat
+            const double v = fma(r[u], ainv, c0), fl = fmin(fmax(floor(v), 0.0), top - 1.0);
+            const bool below = r[u] < G.xfirst, above = r[u] > G.xlast;
+            double tt = v - fl;
+            int i = (int)fl;  // NaN: segment 0, t NaN
+            if (sizeof(R) == 8 && r[u] == r[u]) {
+                // the caller's knots and the correctly rounded t of k_seg_t (the uniform grid's t
+                // is off by the knots' own rounding, 1e-13)
+                const double* xs = gx + G.xoff;
+                double x0 = xs[i], x1 = xs[i + 1];
+                if (r[u] < x0 && i > 0) {
+                    x1 = x0;
+                    x0 = xs[--i];
+                } else if (r[u] >= x1 && i < G.nk - 2) {
+                    x0 = x1;
+                    x1 = xs[++i + 1];
+                }
+                const double h = x1 - x0, n = r[u] - x0, y = grh[G.xoff + i], q0 = n * y;
+                tt = fma(fma(-h, q0, n), y, q0);
+            }
+            ii[u] = below ? 0 : (above ? G.nk : i + 1);
+            t[u] = below || above ? (R)0 : (R)tt;
+            gr[u] = 0.0;
+        }
+        for (int j = vgs[g]; j < vgs[g + 1]; j += NM) {
+            R dd[NM][VF_GPT];
+            int nm = min(NM, vgs[g + 1] - j);
+#pragma unroll
+            for (int v = 0; v < NM; ++v) {
+                const int q = vgm[min(j + v, vgs[g + 1] - 1)];
+                const R* dq = dbar + (int64_t)q * npf;
+#pragma unroll
+                for (int u = 0; u < VF_GPT; ++u) dd[v][u] = dq[pf[u]];
+            }
+            __syncthreads();  // the previous maps' records are no longer read
+#pragma unroll
+            for (int v = 0; v < NM; ++v)
+                if (v < nm) {
+                    const MapInfo m = maps[vgm[j + v]];
+                    const R4* rq = rec4 + m.koff + vgm[j + v];
+                    for (int e = threadIdx.x; e <= m.nk; e += blockDim.x)
+                        lds_rec_put(tb + v * (cap + 1), cap + 1, e < m.nk - 1 ? e + 1 : (e == m.nk - 1 ? 0 : e), rq[e]);
+                }
+            __syncthreads();
+#pragma unroll
+            for (int v = 0; v < NM; ++v) {
+                if (v >= nm) break;
+                const uint32_t flip = (maps[vgm[j + v]].l & 1) ? south : 0u;
+#pragma unroll
+                for (int u = 0; u < VF_GPT; ++u) {
+                    const R4 c = lds_rec_get(tb + v * (cap + 1), cap + 1, ii[u]);  // (d, c, b, a)
+                    const R x = t[u];
+                    const R p1 = fma(x, c.w, c.z), p2 = fma(x, p1, c.y);
+                    const R val = fma(x, p2, c.x);
+                    const R slope = fma(x, fma(x, c.w, p1), p2);
+                    const R d = ((flip >> u) & 1u) ? -dd[v][u] : dd[v][u];
+                    if (sizeof(R) == 8) {
+                        aw[u] = fma((double)val, (double)d, aw[u]);
+                        gr[u] = fma((double)slope, (double)d, gr[u]);
+                    } else {
+                        aw[u] += (double)(val * d);
+                        gr[u] += (double)(slope * d);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < VF_GPT; ++u)
+            ar[u] = fma(gr[u], sizeof(R) == 8 ? grh[G.xoff + min(max(ii[u] - 1, 0), G.nk - 2)] : ainv, ar[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < VF_GPT; ++u) {
+        const int64_t k = k0 + 1024 * u;
+        if (k < N) part[(int64_t)blockIdx.y * N + k] = make_double2(aw[u], ar[u]);
+    }
 }

@@ -4870,82 +4870,115 @@ extern "C" int sfb_cat2amln_vjp_device(sfb_plan* P, int64_t N, const double* d_r
     hipStream_t st = stream ? (hipStream_t)stream : P->stream;
     if (N == 0) return SFB_OK;
     int rc;
-    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, CAT_ANY, false))) return rc;
     const int32_t nq = (int32_t)P->nmaps, L = (int32_t)P->lmax;
-    // mixed precision (the plan's SFB_PREC_MIXED): FP32 Jacobi recursion, synthesis GEMM,
-    // ring synthesis, delta-bar maps and per-galaxy products, FP64 sums; it needs the
-    // knot-group gather (the records in LDS), else the adjoint runs in FP64
+    // mixed precision (the plan's SFB_PREC_MIXED): FP32 ring synthesis, delta-bar maps and
+    // per-galaxy products, FP64 sums; it needs the knot-group gather (the records in LDS), else
+    // the adjoint runs in FP64
     const size_t shv64 = 32 * (size_t)(P->tbl_cap + 1) + 16 * (size_t)P->tbl_cap;
     const size_t shv32 = 16 * (size_t)(P->tbl_cap + 1) + 16 * (size_t)P->tbl_cap;
     const bool grouped = P->sell_ok && P->nvrange > 0;
     const bool f32 = P->precision != SFB_PREC_FP64 && grouped && (int64_t)shv32 <= P->lds_max;
+    // folded hemispheres on uniform knots (records in LDS by P->fold.ok); the split-BF16
+    // precisions keep the iterated refinement whose products they select
+    const size_t one = (f32 ? 16 : 32) * (size_t)(P->tbl_cap + 1);
+    const bool fold = P->fold.ok && P->seg_uniform && grouped && (int64_t)one <= P->lds_max &&
+                      (P->precision == SFB_PREC_FP64 || P->precision == SFB_PREC_MIXED);
+    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, CAT_ANY, false, fold))) return rc;
     PhaseTimer tj(P, SFB_PHASE_ADJOINT, st);
-    hipLaunchKernelGGL(k_fill_f64, dim3(nblk(P->a_size, 256)), dim3(256), 0, st, P->d_a.as<double>(), P->a_size, 0.0);
-    LAUNCH_CHECK();
-    if (f32)
-        hipLaunchKernelGGL(k_unpack_cot<float>, dim3(nblk(nq, 256), (unsigned)(L + 1)), dim3(256), 0, st, d_cot,
-                           P->d_aoff.as<int64_t>(), P->d_maps.as<MapInfo>(), P->d_outbase.as<int64_t>(), nq, P->M2,
-                           P->d_a.as<float>());
-    else
-        hipLaunchKernelGGL(k_unpack_cot<double>, dim3(nblk(nq, 256), (unsigned)(L + 1)), dim3(256), 0, st, d_cot,
-                           P->d_aoff.as<int64_t>(), P->d_maps.as<MapInfo>(), P->d_outbase.as<int64_t>(), nq, P->M2,
-                           P->d_a.as<double>());
-    LAUNCH_CHECK();
-    const bool prof = P->prof;
-    P->prof = false;  // the adjoint's stages are timed as one phase
-    const bool direct = !f32 && P->dir.ok;
-    rc = direct ? direct_synthesis(P, 2 * nq, P->M2, st) : jacobi_stage(P, nq, st, f32);
-    P->prof = prof;
-    if (rc) return rc;
-    // dbar = dOmega S a_final on every pixel of every map
-    const int slot = (P->a_final == P->d_a.as<double>()) ? 0 : (P->a_final == P->d_a1.as<double>() ? 1 : 2);
-    const unsigned nbat = (unsigned)(2 * (L + 1));
-    if (f32)
-        launch_gemm(P->d_desc_synf32.as<GemmDesc>() + slot * nbat, nbat, 2 * nq, P->K, 1.0, 0.0, st, true, true, true);
-    else if (!direct)
-        launch_gemm(P->d_desc_synf.as<GemmDesc>() + slot * nbat, nbat, 2 * nq, P->K, 1.0, 0.0, st);
-    LAUNCH_CHECK();
     const double domega = 4.0 * kPi / (double)P->npix;
-    if ((rc = phi_synthesis(P, nq, domega, st, f32))) return rc;
-    // per-galaxy sums over the maps, in ranges of maps, then the ordered reduction
     int32_t ngroups;
-    if (f32 || (grouped && (int64_t)shv64 <= P->lds_max)) {
-        // knot groups: the segment search once per group and galaxy
+    if (fold) {
         ngroups = P->nvrange;
         if ((rc = P->d_part.ensure(sizeof(double2) * (size_t)ngroups * (size_t)N))) return rc;
-        const dim3 gv(nblk(N, 1024 * VJ_GPT), (unsigned)ngroups);
+        // two record tables per stage while two blocks still share a CU's LDS
+        const bool two = 4 * one <= (size_t)P->lds_max;
+        const size_t shm = two ? 2 * one : one;
+        const dim3 gv(nblk(N, 1024 * VF_GPT), (unsigned)ngroups);
+        auto go = [&](auto kern, const auto* rec4, const auto* dbar) -> int {
+            HIP_TRY(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+            hipLaunchKernelGGL(kern, gv, dim3(1024), shm, st, N, P->fold.npf, P->tbl_cap, P->d_rs.as<double>(),
+                               P->d_pixkey2.as<uint32_t>(), P->d_groups.as<GroupInfo>(), P->d_gx.as<double>(),
+                               P->d_grh.as<double>(), P->d_vgs.as<int32_t>(), P->d_vgm.as<int32_t>(), P->d_vrange.as<int2>(), P->d_maps.as<MapInfo>(), rec4, dbar,
+                               P->d_part.as<double2>());
+            LAUNCH_CHECK();
+            return SFB_OK;
+        };
         if (f32) {
-            HIP_TRY(hipFuncSetAttribute((const void*)k_vjp_it<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)shv32));
-            hipLaunchKernelGGL(k_vjp_it<float>, gv, dim3(1024), shv32, st, N, P->npix, P->tbl_cap,
-                               P->d_rs.as<double>(), P->d_pixkey2.as<uint32_t>(), P->d_groups.as<GroupInfo>(),
-                               P->d_gx.as<double>(), P->d_grh.as<double>(), P->d_vgs.as<int32_t>(),
-                               P->d_vgm.as<int32_t>(), P->d_vrange.as<int2>(), P->d_maps.as<MapInfo>(),
-                               P->d_rec4f.as<float4>(), P->d_delta.as<float>(), P->d_part.as<double2>());
+            if ((rc = fold_synthesis<float>(P, d_cot, domega, st))) return rc;
+            rc = two ? go(k_vjp_fold<float, 2>, P->d_rec4f.as<float4>(), P->d_delta.as<float>())
+                     : go(k_vjp_fold<float, 1>, P->d_rec4f.as<float4>(), P->d_delta.as<float>());
         } else {
-            HIP_TRY(hipFuncSetAttribute((const void*)k_vjp_it<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)shv64));
-            hipLaunchKernelGGL(k_vjp_it<double>, gv, dim3(1024), shv64, st, N, P->npix, P->tbl_cap,
-                               P->d_rs.as<double>(), P->d_pixkey2.as<uint32_t>(), P->d_groups.as<GroupInfo>(),
-                               P->d_gx.as<double>(), P->d_grh.as<double>(), P->d_vgs.as<int32_t>(),
-                               P->d_vgm.as<int32_t>(), P->d_vrange.as<int2>(), P->d_maps.as<MapInfo>(),
-                               P->d_rec4.as<double4>(), P->d_delta.as<double>(), P->d_part.as<double2>());
+            if ((rc = fold_synthesis<double>(P, d_cot, domega, st))) return rc;
+            rc = two ? go(k_vjp_fold<double, 2>, P->d_rec4.as<double4>(), P->d_delta.as<double>())
+                     : go(k_vjp_fold<double, 1>, P->d_rec4.as<double4>(), P->d_delta.as<double>());
         }
-        LAUNCH_CHECK();
+        if (rc) return rc;
     } else {
-        const int32_t MG = (nq + 31) / 32;
-        ngroups = (nq + MG - 1) / MG;
-        if ((rc = P->d_part.ensure(sizeof(double2) * (size_t)ngroups * (size_t)N))) return rc;
-        const bool lds_tables = (int64_t)P->tbl_cap * 32 <= P->lds_max;
-        const size_t shg = lds_tables ? (size_t)P->tbl_cap * 32 : 0;
-        if (lds_tables)
-            HIP_TRY(hipFuncSetAttribute((const void*)k_vjp_gather, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        (int)shg));
-        hipLaunchKernelGGL(k_vjp_gather, dim3(nblk(N, 1024 * VG_GPT), (unsigned)ngroups), dim3(1024), shg, st, N,
-                           P->npix, P->d_rs.as<double>(), P->d_pixkey2.as<uint32_t>(), P->d_maps.as<MapInfo>(),
-                           P->d_rec.as<double4>(), nq, MG, lds_tables, P->d_delta.as<double>(),
-                           P->d_part.as<double2>());
+        hipLaunchKernelGGL(k_fill_f64, dim3(nblk(P->a_size, 256)), dim3(256), 0, st, P->d_a.as<double>(), P->a_size, 0.0);
         LAUNCH_CHECK();
+        if (f32)
+            hipLaunchKernelGGL(k_unpack_cot<float>, dim3(nblk(nq, 256), (unsigned)(L + 1)), dim3(256), 0, st, d_cot,
+                               P->d_aoff.as<int64_t>(), P->d_maps.as<MapInfo>(), P->d_outbase.as<int64_t>(), nq, P->M2,
+                               P->d_a.as<float>());
+        else
+            hipLaunchKernelGGL(k_unpack_cot<double>, dim3(nblk(nq, 256), (unsigned)(L + 1)), dim3(256), 0, st, d_cot,
+                               P->d_aoff.as<int64_t>(), P->d_maps.as<MapInfo>(), P->d_outbase.as<int64_t>(), nq, P->M2,
+                               P->d_a.as<double>());
+        LAUNCH_CHECK();
+        const bool prof = P->prof;
+        P->prof = false;  // the adjoint's stages are timed as one phase
+        const bool direct = !f32 && P->dir.ok;
+        rc = direct ? direct_synthesis(P, 2 * nq, P->M2, st) : jacobi_stage(P, nq, st, f32);
+        P->prof = prof;
+        if (rc) return rc;
+        // dbar = dOmega S a_final on every pixel of every map
+        const int slot = (P->a_final == P->d_a.as<double>()) ? 0 : (P->a_final == P->d_a1.as<double>() ? 1 : 2);
+        const unsigned nbat = (unsigned)(2 * (L + 1));
+        if (f32)
+            launch_gemm(P->d_desc_synf32.as<GemmDesc>() + slot * nbat, nbat, 2 * nq, P->K, 1.0, 0.0, st, true, true, true);
+        else if (!direct)
+            launch_gemm(P->d_desc_synf.as<GemmDesc>() + slot * nbat, nbat, 2 * nq, P->K, 1.0, 0.0, st);
+        LAUNCH_CHECK();
+        if ((rc = phi_synthesis(P, nq, domega, st, f32))) return rc;
+        // per-galaxy sums over the maps, in ranges of maps, then the ordered reduction
+        if (f32 || (grouped && (int64_t)shv64 <= P->lds_max)) {
+            // knot groups: the segment search once per group and galaxy
+            ngroups = P->nvrange;
+            if ((rc = P->d_part.ensure(sizeof(double2) * (size_t)ngroups * (size_t)N))) return rc;
+            const dim3 gv(nblk(N, 1024 * VJ_GPT), (unsigned)ngroups);
+            if (f32) {
+                HIP_TRY(hipFuncSetAttribute((const void*)k_vjp_it<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            (int)shv32));
+                hipLaunchKernelGGL(k_vjp_it<float>, gv, dim3(1024), shv32, st, N, P->npix, P->tbl_cap,
+                                   P->d_rs.as<double>(), P->d_pixkey2.as<uint32_t>(), P->d_groups.as<GroupInfo>(),
+                                   P->d_gx.as<double>(), P->d_grh.as<double>(), P->d_vgs.as<int32_t>(),
+                                   P->d_vgm.as<int32_t>(), P->d_vrange.as<int2>(), P->d_maps.as<MapInfo>(),
+                                   P->d_rec4f.as<float4>(), P->d_delta.as<float>(), P->d_part.as<double2>());
+            } else {
+                HIP_TRY(hipFuncSetAttribute((const void*)k_vjp_it<double>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            (int)shv64));
+                hipLaunchKernelGGL(k_vjp_it<double>, gv, dim3(1024), shv64, st, N, P->npix, P->tbl_cap,
+                                   P->d_rs.as<double>(), P->d_pixkey2.as<uint32_t>(), P->d_groups.as<GroupInfo>(),
+                                   P->d_gx.as<double>(), P->d_grh.as<double>(), P->d_vgs.as<int32_t>(),
+                                   P->d_vgm.as<int32_t>(), P->d_vrange.as<int2>(), P->d_maps.as<MapInfo>(),
+                                   P->d_rec4.as<double4>(), P->d_delta.as<double>(), P->d_part.as<double2>());
+            }
+            LAUNCH_CHECK();
+        } else {
+            const int32_t MG = (nq + 31) / 32;
+            ngroups = (nq + MG - 1) / MG;
+            if ((rc = P->d_part.ensure(sizeof(double2) * (size_t)ngroups * (size_t)N))) return rc;
+            const bool lds_tables = (int64_t)P->tbl_cap * 32 <= P->lds_max;
+            const size_t shg = lds_tables ? (size_t)P->tbl_cap * 32 : 0;
+            if (lds_tables)
+                HIP_TRY(hipFuncSetAttribute((const void*)k_vjp_gather, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                            (int)shg));
+            hipLaunchKernelGGL(k_vjp_gather, dim3(nblk(N, 1024 * VG_GPT), (unsigned)ngroups), dim3(1024), shg, st, N,
+                               P->npix, P->d_rs.as<double>(), P->d_pixkey2.as<uint32_t>(), P->d_maps.as<MapInfo>(),
+                               P->d_rec.as<double4>(), nq, MG, lds_tables, P->d_delta.as<double>(),
+                               P->d_part.as<double2>());
+            LAUNCH_CHECK();
+        }
     }
     const double inv = 1.0 / (nbar * domega);
     hipLaunchKernelGGL(k_vjp_reduce, dim3(nblk(N, 256)), dim3(256), 0, st, N, ngroups, P->d_part.as<double2>(),

@@ -58,3 +58,30 @@ def test_fp64_against_oracle(nside, nl, niter, n, sky, dense):
                 rms = np.sqrt(np.mean(np.abs(ref[s]) ** 2))
                 assert np.max(np.abs(got[s] - ref[s])) <= 1e-10 * rms, (nn + 1, l)
                 i += l + 1
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-11), ("mixed", 3e-6)])
+@pytest.mark.parametrize("nside,n", [(8, 1), (8, 6143), (16, 6145), (32, 30001)])
+def test_adjoint_against_the_unfolded_path(nside, n, precision, tol, monkeypatch):
+    """Gradients on folded maps against the unfolded gather (SFB_SEG_SEARCH=1), with radii on the
+    end knots (whose slopes count), outside them (flat), on inner knots, and southern galaxies;
+    n around a block's 6144 galaxies.  FP64 differs by the rounding of t (1e-12 of a value's
+    slope), mixed by FP32 rounding in the ring transforms (the adjoint's 1e-6)."""
+    print("fold adjoint", nside, n, precision, flush=True)
+    am = S.AnlmModes(0.7 * nside / 1000.0, 500.0, 1000.0, nside=nside)
+    rng = np.random.default_rng(n)
+    cat = catalogue(rng, n, "full")
+    edge = np.array([500.0, 1000.0, np.nextafter(500, 0), np.nextafter(1000, 2000), am.knot_x[7], am.knot_x[-3]])
+    cat[0, : min(n, 60)] = np.resize(edge, min(n, 60))
+    w = rng.uniform(0.5, 1.5, n)
+    plan = S.Plan(am, precision=precision)
+    monkeypatch.setenv("SFB_SEG_SEARCH", "1")
+    ref_plan = S.Plan(am, precision=precision)
+    monkeypatch.delenv("SFB_SEG_SEARCH")
+    c = rng.normal(size=plan.nlmsize) + 1j * rng.normal(size=plan.nlmsize)
+    got, ref = plan.cat2amln_vjp(cat, 1e-5, c, w), ref_plan.cat2amln_vjp(cat, 1e-5, c, w)
+    for g, r in zip(got[:2], ref[:2]):
+        rms = np.sqrt(np.mean(r ** 2))
+        assert np.max(np.abs(g - r)) <= tol * rms * (10 if n == 1 else 1)
+    out = (cat[0] < 500.0) | (cat[0] > 1000.0)
+    assert np.all(got[0][out] == 0.0)
