@@ -151,24 +151,26 @@ __global__ __launch_bounds__(256) void k_phi_polar4_fold(const double* __restric
     double2* twi = (double2*)(D + TQ * ld1);   // (cos, -sin)(2 pi v/i)
     for (int e = threadIdx.x; e < ni; e += blockDim.x) twi[e] = make_double2(twl[8 * e].x, -twl[8 * e].y);
     const int nv = npr >> 2;
-    for (int e = threadIdx.x; e < TQ * nv; e += blockDim.x) {
-        const int ql = e / nv, j4 = e - ql * nv;
-        const int64_t p = Rg.start_n + 4 * j4;
-        double4 v = make_double4(0.0, 0.0, 0.0, 0.0);
-        if (c0 + ql < ncol) {
-            const double* dq = delta + (int64_t)cols[c0 + ql].q * npf;
-            if (perm) {
-                const uint4 sl = *(const uint4*)(perm + p);
-                v = make_double4(dq[sl.x], dq[sl.y], dq[sl.z], dq[sl.w]);
-            } else {
-                v = make_double4(dq[p], dq[p + 1], dq[p + 2], dq[p + 3]);
-            }
+    for (int e0 = threadIdx.x; e0 < TQ * nv; e0 += PH_UL * blockDim.x) {  // PH_UL fours in flight
+        double4 v[PH_UL];
+        uint4 sl[PH_UL];
+#pragma unroll
+        for (int u = 0; u < PH_UL; ++u) {
+            const int e = min(e0 + u * (int)blockDim.x, TQ * nv - 1), p = (int)Rg.start_n + 4 * (e % nv);
+            sl[u] = make_uint4(p, p + 1, p + 2, p + 3);
+            if (perm) sl[u] = *(const uint4*)(perm + p);
         }
-        double* d = D + ql * ld1 + 4 * j4;
-        d[0] = v.x;
-        d[1] = v.y;
-        d[2] = v.z;
-        d[3] = v.w;
+#pragma unroll
+        for (int u = 0; u < PH_UL; ++u) {
+            const int e = min(e0 + u * (int)blockDim.x, TQ * nv - 1);
+            const double* dq = delta + (int64_t)cols[min(c0 + e / nv, ncol - 1)].q * npf;
+            v[u] = make_double4(dq[sl[u].x], dq[sl[u].y], dq[sl[u].z], dq[sl[u].w]);
+        }
+#pragma unroll
+        for (int u = 0; u < PH_UL; ++u) {
+            const int e = e0 + u * blockDim.x;
+            if (e < TQ * nv) *(double4*)(D + (e / nv) * ld1 + 4 * (e % nv)) = v[u];
+        }
     }
     __syncthreads();
     {

@@ -2901,7 +2901,7 @@ struct PinBuf {
 // Tables and launch lists of the refined map2alm as one operator (sht_direct.h).
 struct DirectSht {
     bool ok = false;               // the folded form applies (else jacobi_stage iterates)
-    int32_t S = 0, ct = 2;         // aliasing states; columns per k_alias_solve block
+    int32_t S = 0, nterm = 0;      // aliasing states and couplings
     int32_t n_ana = 0, n_fix = 0, n_syn = 0, n_sfix = 0;  // batches of each launch
     int32_t maxN = 1, maxNs = 1, maxNf = 1;
     int64_t hrows = 0;

@@ -7,12 +7,12 @@
 // replace and a column's states no longer fit in LDS: the iterated form stays (jacobi_stage).
 constexpr int32_t DIRECT_MAX_NITER = 8, DIRECT_MAX_NAL = 48, DIRECT_MAX_STATES = 1536;
 
-// Columns per k_alias_solve block: as many as keep a block within half a CU's LDS (more
-// columns read the Q tables and couplings fewer times), at least 2.
-static inline int32_t direct_alias_ct(int64_t S, int32_t J, int64_t lds_max)
+// Columns per k_alias_solve block: 8 (64-byte rows) for many columns, 4 for few (twice the
+// blocks), fewer when the states do not fit.
+static inline int32_t direct_alias_ct(const DirectSht& D, int32_t J, int32_t cols, int64_t lds_max)
 {
-    int32_t ct = 32;
-    while (ct > 2 && (J + 1) * S * ct * 8 > std::min<int64_t>(lds_max, 81920)) ct /= 2;
+    int32_t ct = cols >= 2048 ? 8 : 4;
+    while (ct > 1 && (int64_t)alias_lds(D.S, J, ct, D.nterm) > lds_max) ct /= 2;
     return ct;
 }
 
@@ -38,7 +38,7 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
                 for (int64_t mp = m - ((m + L) / npr) * npr; mp <= L; mp += npr) {
                     if (mp == m) continue;
                     const int64_t ma = mp < 0 ? -mp : mp;
-                    if (!(domega * npr * wk * rowmax[(size_t)(m * K + k)] * rowmax[(size_t)(ma * K + k)] > 1e-20))
+                    if (!(domega * npr * wk * rowmax[(size_t)(m * K + k)] * rowmax[(size_t)(ma * K + k)] > 1e-18))
                         continue;
                     const double sgn = ((((mp - m) / npr) * sh) & 1) ? -1.0 : 1.0;
                     const double c = -npr * wk * sgn;
@@ -56,9 +56,7 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
     }
     const int32_t S = s0[(size_t)L + 1];
     if (J > DIRECT_MAX_NITER || S > DIRECT_MAX_STATES) return SFB_OK;
-    if ((J + 1) * (int64_t)S * 2 * 8 > P->lds_max) return SFB_OK;
     D.S = S;
-    D.ct = direct_alias_ct(std::max(S, 1), J, P->lds_max);
     std::vector<AliasState> st((size_t)std::max(S, 1));
     for (int64_t m = 0; m <= L; ++m)
         for (int32_t a = 0; a < na[(size_t)m]; ++a)
@@ -83,6 +81,8 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
         st[(size_t)s].e1 = (int32_t)terms.size();
     }
     if (terms.empty()) terms.push_back({0, 0, 0.0, 0.0});
+    D.nterm = (int32_t)terms.size();
+    if ((int64_t)alias_lds(S, J, 1, D.nterm) > P->lds_max) return SFB_OK;
     // table offsets per block b = (m, parity)
     const int64_t nbat = 2 * (L + 1);
     std::vector<int64_t> hboff((size_t)nbat + 1, 0), voff((size_t)nbat + 1, 0), qoff((size_t)nbat + 1, 0);
@@ -322,11 +322,12 @@ static int direct_alias(sfb_plan* P, int32_t cols, int64_t ld, hipStream_t st, i
 {
     DirectSht& D = P->dir;
     const int32_t J = P->niter;
-    const size_t shm = sizeof(double) * (size_t)(J + 1) * (size_t)D.S * (size_t)D.ct;
+    const int32_t ct = direct_alias_ct(D, J, cols, P->lds_max);
+    const size_t shm = alias_lds(D.S, J, ct, D.nterm);
     HIP_TRY(hipFuncSetAttribute((const void*)k_alias_solve, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-    hipLaunchKernelGGL(k_alias_solve, dim3(nblk(cols, D.ct), split < 0 ? 2u : 1u), dim3(1024), shm, st, D.S, J, (int32_t)P->lmax, D.ct, cols,
-                       split, D.d_st.as<AliasState>(), D.d_term.as<AliasTerm>(), D.d_Q.as<double>(),
-                       D.d_qoff.as<int64_t>(), D.d_h.as<double>(), D.d_r.as<double>(), ld);
+    hipLaunchKernelGGL(k_alias_solve, dim3(nblk(cols, ct), split < 0 ? 2u : 1u), dim3(1024), shm, st, D.S, J,
+                       (int32_t)P->lmax, ct, cols, split, D.d_st.as<AliasState>(), D.nterm, D.d_term.as<AliasTerm>(),
+                       D.d_Q.as<double>(), D.d_qoff.as<int64_t>(), D.d_h.as<double>(), D.d_r.as<double>(), ld);
     LAUNCH_CHECK();
     return SFB_OK;
 }

@@ -14,7 +14,8 @@
 // Which (ring pair, m) alias: lambda_lm falls off steeply beyond m ~ l sin(theta), and m and
 // m' >= npr - m cannot both be inside it on a polar ring, so the product of the two lambdas
 // is negligible on all but the first few ring pairs.  A pair of states is kept when
-// dOmega npr mult max_l |lambda_lm| max_l' |lambda_l'm'| > 1e-20 (the entry of A S it makes).
+// dOmega npr mult max_l |lambda_lm| max_l' |lambda_l'm'| > 1e-18 (the entry of A S it makes, whose
+// diagonal is ~1: what is dropped stays below an FP64 rounding of the coefficients).
 #pragma once
 
 // One batch of the row-addressed GEMM: C[crow + n][i] = alpha sum_k A[arow + k][i] B[k][n]
@@ -98,49 +99,72 @@ struct AliasTerm {
 // Columns alternate real and imaginary parts.  A column belongs to the sector of its l parity
 // sg (parity of (m, l) blocks: (m + sg) & 1): sector blockIdx.y for split < 0, where sector sg's
 // rows start at sg J S; else columns below split are of sector 0, the rest of sector 1, and the
-// rows are shared.  Row of (s, j): J s0 + j na + a.  The states of CT columns stay in LDS over
-// the J steps; a thread walks states at a fixed column.  What bounds it is the chain of 2 J
-// dependent phases over a few hundred states, not bytes (h and r are a few MB).
-__global__ __launch_bounds__(1024) void k_alias_solve(int32_t S, int32_t J, int32_t L, int32_t CT, int32_t cols, int32_t split,
-                                                      const AliasState* __restrict__ st,
+// rows are shared.  Row of (s, j): J s0 + j na + a.  The values of CT columns (a power of two)
+// stay in LDS over the J steps, with the states and couplings beside them, so that after one round
+// of loads only the Q rows come from L2.  What bounds it is the chain of 2 J dependent phases
+// over a few hundred states, not bytes (states, couplings and h read phase by phase: 115 us for
+// 5028 columns and 441 states, 28 us for 320 columns).
+__host__ __device__ inline size_t alias_lds(int32_t S, int32_t J, int32_t CT, int32_t nterm)
+{
+    return sizeof(double) * (size_t)(J + 1) * (size_t)S * (size_t)CT + sizeof(AliasTerm) * (size_t)nterm +
+           sizeof(AliasState) * (size_t)S;
+}
+__global__ __launch_bounds__(1024) void k_alias_solve(int32_t S, int32_t J, int32_t L, int32_t CT, int32_t cols,
+                                                      int32_t split, const AliasState* __restrict__ st, int32_t nterm,
                                                       const AliasTerm* __restrict__ term,
                                                       const double* __restrict__ Q, const int64_t* __restrict__ qoff,
                                                       const double* __restrict__ h, double* __restrict__ r, int64_t ld)
 {
-    extern __shared__ double alias_lds[];
-    double* g = alias_lds;                      // [S][CT]
-    double* rr = alias_lds + (int64_t)S * CT;   // [J][S][CT]
-    const int c = threadIdx.x % CT, w0 = threadIdx.x / CT, nw = blockDim.x / CT;
+    extern __shared__ double alias_mem[];
+    double* g = alias_mem;                     // [S][CT]
+    double* rr = g + (int64_t)S * CT;          // [J][S][CT]: h_j, then r_j
+    AliasTerm* tm = (AliasTerm*)(rr + (int64_t)J * S * CT);
+    AliasState* sl = (AliasState*)(tm + nterm);
+    const int c = threadIdx.x & (CT - 1), w0 = threadIdx.x / CT, nw = blockDim.x / CT;
     const int col = blockIdx.x * CT + c;
     const bool live = col < cols;
     const int sg = split < 0 ? (int)blockIdx.y : (col < split ? 0 : 1);
     const int64_t row0 = split < 0 ? (int64_t)sg * J * S : 0;
-    const int64_t cc = live ? col : 0;
+    const double* hc = h + row0 * ld + (live ? col : 0);
+    for (int e = threadIdx.x; e < nterm; e += blockDim.x) tm[e] = term[e];
+    for (int e = threadIdx.x; e < S; e += blockDim.x) sl[e] = st[e];
+    for (int s = w0; s < S; s += nw) {
+        const AliasState a = st[s];
+        const bool some = live && !(a.m == L && ((a.m + sg) & 1));  // (lmax, odd) has no l: its h is never written
+        for (int j = 0; j < J; ++j)
+            rr[((int64_t)j * S + s) * CT + c] = some ? hc[((int64_t)J * a.s0 + j * a.na + a.a) * ld] : 0.0;
+    }
+    __syncthreads();
     for (int j = 0; j < J; ++j) {
         for (int s = w0; s < S; s += nw) {
-            const AliasState a = st[s];
+            const AliasState a = sl[s];
             const int par = (a.m + sg) & 1;
-            const bool some = live && !(a.m == L && par == 1);  // (lmax, odd) has no l: its h is never written
-            double v = some ? h[(row0 + (int64_t)J * a.s0 + j * a.na + a.a) * ld + cc] : 0.0;
-            const double* q = Q + qoff[2 * a.m + par];
-            for (int i = 0; some && i < j; ++i) {
-                const double* qr = q + ((int64_t)(j - 1 - i) * a.na + a.a) * a.na;
-                const double* ri = rr + ((int64_t)i * S + a.s0) * CT + c;
-                for (int e = 0; e < a.na; ++e) v = fma(qr[e], ri[e * CT], v);
+            double v = rr[((int64_t)j * S + s) * CT + c];
+            if (!(a.m == L && par == 1)) {
+                const double* q = Q + qoff[2 * a.m + par] + (int64_t)a.a * a.na;
+                for (int i = 0; i < j; ++i) {
+                    const double* qr = q + (int64_t)(j - 1 - i) * a.na * a.na;
+                    const double* ri = rr + ((int64_t)i * S + a.s0) * CT + c;
+#pragma unroll 4
+                    for (int e = 0; e < a.na; ++e) v = fma(qr[e], ri[e * CT], v);
+                }
             }
             g[s * CT + c] = v;
         }
         __syncthreads();
         for (int s = w0; s < S; s += nw) {
-            const AliasState a = st[s];
+            const int e0 = sl[s].e0, e1 = sl[s].e1;
             double v = 0.0;
-            for (int e = a.e0; e < a.e1; ++e) {
-                const AliasTerm t = term[e];
-                v = fma((col & 1) ? t.cim : t.cre, g[t.s * CT + c], v);
-            }
+            for (int e = e0; e < e1; ++e) v = fma((col & 1) ? tm[e].cim : tm[e].cre, g[tm[e].s * CT + c], v);
             rr[((int64_t)j * S + s) * CT + c] = v;
-            if (live) r[(row0 + (int64_t)J * a.s0 + j * a.na + a.a) * ld + cc] = v;
         }
         __syncthreads();
+    }
+    if (!live) return;
+    double* rc = r + row0 * ld + col;
+    for (int s = w0; s < S; s += nw) {
+        const AliasState a = sl[s];
+        for (int j = 0; j < J; ++j)
+            rc[((int64_t)J * a.s0 + j * a.na + a.a) * ld] = rr[((int64_t)j * S + s) * CT + c];
     }
 }
