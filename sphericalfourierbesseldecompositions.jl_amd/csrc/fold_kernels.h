@@ -173,21 +173,9 @@ __global__ __launch_bounds__(256) void k_phi_polar4_fold(const double* __restric
         }
     }
     __syncthreads();
-    {
-        const int MT = p4_mt(ni), ntb = tq / 2, msplit = 4 / ntb;
-        const int wv = threadIdx.x >> 6, nt = wv % ntb, mpart = wv / ntb;
-        const int mtw = (MT + msplit - 1) / msplit;
-        switch (mtw) {
-            case 1: p4_product<double, 1>(D, twi, ni, ld1, nt, mpart, msplit); break;
-            case 2: p4_product<double, 2>(D, twi, ni, ld1, nt, mpart, msplit); break;
-            case 3: p4_product<double, 3>(D, twi, ni, ld1, nt, mpart, msplit); break;
-            case 4: p4_product<double, 4>(D, twi, ni, ld1, nt, mpart, msplit); break;
-            case 5: if (MTWMAX > 4) p4_product<double, MTWMAX < 5 ? 4 : 5>(D, twi, ni, ld1, nt, mpart, msplit); break;
-            case 6: if (MTWMAX > 4) p4_product<double, MTWMAX < 6 ? 4 : 6>(D, twi, ni, ld1, nt, mpart, msplit); break;
-            case 7: if (MTWMAX > 4) p4_product<double, MTWMAX < 7 ? 4 : 7>(D, twi, ni, ld1, nt, mpart, msplit); break;
-            default: if (MTWMAX > 4) p4_product<double, MTWMAX>(D, twi, ni, ld1, nt, mpart, msplit); break;
-        }
-    }
+    p4_fold_samples(D, TQ, ni, ld1);
+    __syncthreads();
+    p4_product_tiles<MTWMAX>(D, twi, ni, ld1, tq);
     __syncthreads();
     const int Lk = mall[k];
     const int nkf = min(Lk, npr / 2) + 1;
@@ -248,6 +236,7 @@ __global__ __launch_bounds__(256) void k_fold_rows(int32_t K, int32_t J, int64_t
     }
     const double2* rr = (const double2*)(r + (int64_t)J * M.s0 * ld) + c;
     const double* z = ZB + M.v[pi] + j;
+#pragma unroll 4
     for (int h = wv; h < J * M.na; h += 4) {
         const double2 v = rr[(int64_t)h * ld2];
         const double w = z[(int64_t)h * nb];

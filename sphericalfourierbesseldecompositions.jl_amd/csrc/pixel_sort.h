@@ -12,6 +12,7 @@
 constexpr int PS_CROWD = 512;     // galaxies per pixel the pairwise rank takes
 constexpr int PS_MEAN = 96;       // mean galaxies per pixel above which the radix sorts run at once
 constexpr int PS_CHUNK = 2048;    // pixels per scan block
+constexpr int PS_SMALL = 32;      // scan blocks up to which each adds up the counts before it itself
 
 __global__ __launch_bounds__(256) void k_zero_counts(int64_t npix, int32_t* __restrict__ cnt, int32_t* __restrict__ flag)
 {
@@ -61,21 +62,28 @@ __global__ __launch_bounds__(256) void k_count_sums(int64_t npix, const int32_t*
     if (threadIdx.x == 0) sums[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-// pstart[p] = galaxies before pixel p; pstart[npix] = N
+// pstart[p] = galaxies before pixel p; pstart[npix] = N.  sums NULL (small grids, one launch
+// less): a block adds up the counts before its chunk itself, and checks its own for crowding.
 __global__ __launch_bounds__(256) void k_count_scan(int64_t npix, int32_t N, const int32_t* __restrict__ cnt,
-                                                    const int32_t* __restrict__ sums, int32_t* __restrict__ pstart)
+                                                    const int32_t* __restrict__ sums, int32_t* __restrict__ pstart,
+                                                    int32_t* __restrict__ flag)
 {
     __shared__ int32_t part[256];
     constexpr int PT = PS_CHUNK / 256;
     const int t = threadIdx.x;
     int32_t before = 0;
-    for (int b = t; b < (int)blockIdx.x; b += 256) before += sums[b];
+    if (sums)
+        for (int b = t; b < (int)blockIdx.x; b += 256) before += sums[b];
+    else
+#pragma unroll 8
+        for (int p = t; p < (int)blockIdx.x * PS_CHUNK; p += 256) before += cnt[p];
     const int64_t p0 = (int64_t)blockIdx.x * PS_CHUNK + t * PT;
     int32_t c[PT], s = 0;
 #pragma unroll
     for (int u = 0; u < PT; ++u) {
         c[u] = p0 + u < npix ? cnt[p0 + u] : 0;
         s += c[u];
+        if (!sums && flag && c[u] > PS_CROWD) atomicOr(flag + 2, 2);
     }
     // the chunk's offset: the sum of `before` over the block
     for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
@@ -161,54 +169,88 @@ __global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restri
     w_s[f] = me.w;
 }
 
-// Slices of the sliced layout from the counts: one block per window of SELL_SIGMA pixels sorts
-// them by (count descending, pixel) in LDS and writes the slices' lanes, widths and emptiest
-// lanes (what a radix sort of (window, count) keys and a pass over its result gave).
+// Slices of the sliced layout from the counts: one block per window of SELL_SIGMA pixels orders
+// them by count (descending) with a counting sort in LDS and writes the slices' lanes, widths and
+// emptiest lanes.  Pixels of one count come in any order: a pixel's sum does not depend on its
+// slot, and the slices' widths only on the counts' order.  (A bitonic sort of (count, pixel) keys,
+// 55 barriers, ran 11 us; it stays for windows with a pixel of 1024 galaxies or more.)
 __global__ __launch_bounds__(1024) void k_sell_window(int64_t npix, int32_t nslice, const int32_t* __restrict__ pstart,
                                                       int64_t* __restrict__ width, uint32_t* __restrict__ invperm,
                                                       int2* __restrict__ pinfo, int32_t* __restrict__ smin)
 {
     static_assert(SELL_SIGMA == 1024, "one thread per pixel of a window");
-    __shared__ uint32_t key[1024];
-    __shared__ int32_t cnt[1024];
-    const int t = threadIdx.x;
+    __shared__ int32_t bin[1024];   // pixels per bin (bin 0: the largest counts), then the bins' starts
+    __shared__ int32_t wsum[16];
+    __shared__ int32_t big;         // the window's largest count
+    __shared__ int2 lane_pc[1024];  // (pixel, count) by position
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
     const int64_t p0 = (int64_t)blockIdx.x * 1024;
     const bool in = p0 + t < npix;
     const int32_t c0 = in ? pstart[p0 + t + 1] - pstart[p0 + t] : 0;
-    cnt[t] = c0;
-    key[t] = in ? ((uint32_t)(0xffff - min(c0, 0xffff)) << 10) | (uint32_t)t : 0xffffffffu;
+    bin[t] = 0;
+    lane_pc[t] = make_int2(0, 0);  // lanes past the last pixel: no pixel, no galaxies
+    if (t == 0) big = 0;
     __syncthreads();
-    for (int k = 2; k <= 1024; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            const int o = t ^ j;
-            if (o > t) {
-                const uint32_t a = key[t], b = key[o];
-                if ((a > b) == ((t & k) == 0)) {
-                    key[t] = b;
-                    key[o] = a;
-                }
-            }
-            __syncthreads();
+    int32_t mx = c0;
+    for (int o = 32; o > 0; o >>= 1) mx = max(mx, __shfl_xor(mx, o, 64));
+    if (lane == 0) atomicMax(&big, mx);
+    __syncthreads();
+    if (big < 1024) {  // a bin per count
+        const int32_t b = big - c0;
+        int32_t rank = 0;
+        if (in) rank = atomicAdd(&bin[b], 1);
+        __syncthreads();
+        const int32_t n = bin[t];
+        int32_t inc = n;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int32_t v = __shfl_up(inc, o, 64);
+            if (lane >= o) inc += v;
         }
+        if (lane == 63) wsum[wv] = inc;
+        __syncthreads();
+        int32_t base = 0;
+        for (int i = 0; i < wv; ++i) base += wsum[i];
+        bin[t] = base + inc - n;
+        __syncthreads();
+        if (in) {
+            const int32_t at = bin[b] + rank;
+            lane_pc[at] = make_int2((int)(p0 + t), c0);
+            invperm[p0 + t] = (uint32_t)(p0 + at);
+        }
+    } else {  // crowded: (count, pixel) keys by a bitonic sort
+        uint32_t* key = (uint32_t*)bin;
+        key[t] = in ? ((uint32_t)(0x1fffff - min(c0, 0x1fffff)) << 10) | (uint32_t)t : 0xffffffffu;
+        __syncthreads();
+        for (int k = 2; k <= 1024; k <<= 1)
+            for (int j = k >> 1; j > 0; j >>= 1) {
+                const int o = t ^ j;
+                if (o > t) {
+                    const uint32_t a = key[t], b = key[o];
+                    if ((a > b) == ((t & k) == 0)) {
+                        key[t] = b;
+                        key[o] = a;
+                    }
+                }
+                __syncthreads();
+            }
+        if (key[t] != 0xffffffffu) {
+            const int l = (int)(key[t] & 1023u);
+            lane_pc[t] = make_int2((int)(p0 + l), pstart[p0 + l + 1] - pstart[p0 + l]);
+            invperm[p0 + l] = (uint32_t)(p0 + t);
+        }
+    }
+    __syncthreads();
     const int64_t e = p0 + t;
     const int32_t s = (int32_t)(e >> 6);
     if (s >= nslice) return;  // whole wavefronts leave together
-    const uint32_t kk = key[t];
-    int32_t c = 0;
-    if (kk != 0xffffffffu) {
-        const int l = (int)(kk & 1023u);
-        c = cnt[l];
-        invperm[p0 + l] = (uint32_t)e;
-        pinfo[e] = make_int2((int)(p0 + l), c);
-    } else {  // lanes past the last pixel: no pixel, no galaxies
-        pinfo[e] = make_int2(0, 0);
-    }
-    int32_t cmin = c;
+    const int2 pc = lane_pc[t];
+    pinfo[e] = pc;
+    int32_t c = pc.y, cmin = pc.y;
     for (int o = 32; o > 0; o >>= 1) {
         c = max(c, __shfl_xor(c, o, 64));
         cmin = min(cmin, __shfl_xor(cmin, o, 64));
     }
-    if ((t & 63) == 0) {
+    if (lane == 0) {
         width[s] = 64 * (int64_t)c;
         smin[s] = cmin;
     }

@@ -1520,7 +1520,7 @@ template <> struct MfmaT<true> {
 // into FP64 sums every four k-steps (16 samples): a length-i FP32 sum errs by ~sqrt(i/2)
 // ulp, 1e-6 of the coefficients at nside 256, the mixed path's whole error budget.  Y
 // overwrites the staged samples after the product.
-__host__ __device__ inline int p4_mt(int ni) { return (2 * (ni / 2 + 1) + 15) / 16; }
+__host__ __device__ inline int p4_mt(int ni) { return 2 * ((ni / 2 + 1 + 15) / 16); }
 // row tiles per wave at most, for the rings of an nside (i < nside)
 __host__ __device__ inline int p4_mtwmax(int64_t nside) { return p4_mt((int)(nside > 1 ? nside - 1 : 1)) <= 16 ? 4 : 8; }
 // maps per block: 8 while a wave holds every row tile, then 4 and 2
@@ -1610,6 +1610,89 @@ __device__ __forceinline__ void p4_product(R* __restrict__ D, const typename Vec
         }
 }
 
+// The FP64 product on the samples' even and odd parts, half the k-steps: cos rows take
+// x_j + x_{i-j}, sin rows x_j - x_{i-j}, j <= i/2 (a row tile is all cos or all sin).  D holds the
+// samples; they are folded in place first (even part at j, odd part at i - j), Y overwrites them.
+template <int MTW>
+__device__ __forceinline__ void p4_product_sym(double* __restrict__ D, const double2* __restrict__ twi, int ni, int ld,
+                                               int nt, int mpart, int msplit)
+{
+    typedef MfmaT<false> M;
+    const int lane = threadIdx.x & 63, nu = ni / 2 + 1, ntc = (nu + 15) / 16;
+    const int c = 16 * nt + (lane & 15);
+    const double* bcol = D + (c >> 2) * ld + (c & 3);
+    int idx[MTW], stp[MTW];
+    bool sn[MTW];
+#pragma unroll
+    for (int mi = 0; mi < MTW; ++mi) {
+        const int t = mpart + mi * msplit;
+        sn[mi] = t >= ntc;
+        const int u = 16 * (sn[mi] ? t - ntc : t) + (lane & 15);  // rows past nu are computed and dropped
+        stp[mi] = (4 * u) % ni;
+        idx[mi] = (u * (lane >> 4)) % ni;
+    }
+    const double* tw1 = (const double*)twi;  // (cos, -sin) pairs
+    M::V acc[MTW];
+#pragma unroll
+    for (int mi = 0; mi < MTW; ++mi) acc[mi] = M::zero();
+    for (int j0 = 0; j0 < nu; j0 += 8) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int j = j0 + 4 * s + (lane >> 4);
+            const double be = j < nu ? bcol[4 * j] : 0.0;
+            const double bo = (j < nu && j > 0 && 2 * j != ni) ? bcol[4 * (ni - j)] : 0.0;
+#pragma unroll
+            for (int mi = 0; mi < MTW; ++mi) {
+                acc[mi] = M::mma(tw1[2 * idx[mi] + (sn[mi] ? 1 : 0)], sn[mi] ? bo : be, acc[mi]);
+                const unsigned nx = (unsigned)(idx[mi] + stp[mi]);
+                idx[mi] = (int)min(nx, nx - (unsigned)ni);
+            }
+        }
+    }
+    __syncthreads();  // every sample read; Y overwrites them
+#pragma unroll
+    for (int mi = 0; mi < MTW; ++mi)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+            const int t = mpart + mi * msplit;
+            const int u = 16 * (sn[mi] ? t - ntc : t) + M::row(lane, v);
+            if (u < nu && t < 2 * ntc) D[(c >> 2) * ld + 2 * ((c & 3) * nu + u) + (sn[mi] ? 1 : 0)] = acc[mi][v];
+        }
+}
+
+// Folds the samples of nf sequences for p4_product_sym (all threads; barriers by the caller).
+__device__ __forceinline__ void p4_fold_samples(double* __restrict__ D, int nf, int ni, int ld)
+{
+    const int h = (ni - 1) / 2;  // pairs (j, i - j), 1 <= j <= h
+    for (int e = threadIdx.x; e < nf * 4 * h; e += blockDim.x) {
+        const int f = e / (4 * h), r = e - f * 4 * h, j = 1 + (r >> 2), s = r & 3;
+        double* d = D + f * ld + s;
+        const double a = d[4 * j], b = d[4 * (ni - j)];
+        d[4 * j] = a + b;
+        d[4 * (ni - j)] = a - b;
+    }
+}
+
+// p4_product_sym over a block's tiles: tq / 2 column tiles, the row tiles split over the rest.
+template <int MTWMAX>
+__device__ __forceinline__ void p4_product_tiles(double* __restrict__ D, const double2* __restrict__ twi, int ni, int ld,
+                                                 int tq)
+{
+    const int MT = p4_mt(ni), ntb = tq / 2, msplit = 4 / ntb;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), nt = wv % ntb, mpart = wv / ntb;
+    const int mtw = (MT + msplit - 1) / msplit;  // row tiles per wave (<= MTWMAX)
+    switch (mtw) {
+        case 1: p4_product_sym<1>(D, twi, ni, ld, nt, mpart, msplit); break;
+        case 2: p4_product_sym<2>(D, twi, ni, ld, nt, mpart, msplit); break;
+        case 3: p4_product_sym<3>(D, twi, ni, ld, nt, mpart, msplit); break;
+        case 4: p4_product_sym<4>(D, twi, ni, ld, nt, mpart, msplit); break;
+        case 5: if (MTWMAX > 4) p4_product_sym<MTWMAX < 5 ? 4 : 5>(D, twi, ni, ld, nt, mpart, msplit); break;
+        case 6: if (MTWMAX > 4) p4_product_sym<MTWMAX < 6 ? 4 : 6>(D, twi, ni, ld, nt, mpart, msplit); break;
+        case 7: if (MTWMAX > 4) p4_product_sym<MTWMAX < 7 ? 4 : 7>(D, twi, ni, ld, nt, mpart, msplit); break;
+        default: if (MTWMAX > 4) p4_product_sym<MTWMAX>(D, twi, ni, ld, nt, mpart, msplit); break;
+    }
+}
+
 template <typename R, int MTWMAX>
 __global__ __launch_bounds__(256) void k_phi_polar4(const R* __restrict__ delta, int64_t npix, int32_t nq,
                                                     int64_t M2, int32_t K, int32_t L,
@@ -1689,8 +1772,12 @@ __global__ __launch_bounds__(256) void k_phi_polar4(const R* __restrict__ delta,
     }
     __syncthreads();
     // the product: waves split the column tiles (TQ / 2 of 16 columns) and the row tiles
-    {
-        const int MT = p4_mt(ni), ntb = TQ / 2, msplit = 4 / ntb;
+    if constexpr (sizeof(R) == 8) {
+        p4_fold_samples(D, 2 * TQ, ni, ld);
+        __syncthreads();
+        p4_product_tiles<MTWMAX>(D, twi, ni, ld, TQ);
+    } else {
+        const int MT = (2 * nu + 15) / 16, ntb = TQ / 2, msplit = 4 / ntb;
         const int wv = threadIdx.x >> 6, nt = wv % ntb, mpart = wv / ntb;
         const int mtw = (MT + msplit - 1) / msplit;  // row tiles per wave (<= MTWMAX)
         switch (mtw) {
@@ -3861,11 +3948,14 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         hipLaunchKernelGGL((fold ? k_count<true> : k_count<false>), dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, cnt,
                            P->d_keyr.as<uint2>(), P->d_flag.as<int32_t>());
         LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_count_sums, dim3(nb), dim3(256), 0, st, np, cnt, sums,
-                           order == CAT_ANY ? nullptr : P->d_flag.as<int32_t>());
-        LAUNCH_CHECK();
-        hipLaunchKernelGGL(k_count_scan, dim3(nb), dim3(256), 0, st, np, (int32_t)N, cnt, sums,
-                           P->d_pstart.as<int32_t>());
+        int32_t* crowd = order == CAT_ANY ? nullptr : P->d_flag.as<int32_t>();
+        const bool small = nb <= (unsigned)PS_SMALL;
+        if (!small) {
+            hipLaunchKernelGGL(k_count_sums, dim3(nb), dim3(256), 0, st, np, cnt, sums, crowd);
+            LAUNCH_CHECK();
+        }
+        hipLaunchKernelGGL(k_count_scan, dim3(nb), dim3(256), 0, st, np, (int32_t)N, cnt,
+                           small ? (const int32_t*)nullptr : sums, P->d_pstart.as<int32_t>(), crowd);
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_place, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_keyr.as<uint2>(),
                            P->d_pstart.as<int32_t>(), d_rtp, d_w, sh, P->d_sorttmp.as<CatSlot>());
@@ -4119,8 +4209,9 @@ static int scatter_stage(sfb_plan* P, double nbar, int32_t win_kind, const doubl
         if (!onfly && ((rc = P->d_it_i.ensure(sizeof(uint16_t) * (size_t)(T * P->ngroup))) ||
                        (rc = P->d_it_t.ensure(sizeof(double) * (size_t)(T * P->ngroup)))))
             return rc;
-        // 64 slot ranges per group; LDS holds the group's knots and 1/h
-        const dim3 gseg(64, (unsigned)P->ngroup);
+        // up to 64 slot ranges per group, each a block's four rounds at least (small catalogues:
+        // fewer blocks stage the group's knots and 1/h in LDS)
+        const dim3 gseg((unsigned)std::min<int64_t>(64, nblk(P->ncat, 4096)), (unsigned)P->ngroup);
         const size_t shm_seg = 2 * sizeof(double) * (size_t)P->tbl_cap;
         HIP_TRY(hipFuncSetAttribute((const void*)k_seg_t<float>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                     (int)shm_seg));
