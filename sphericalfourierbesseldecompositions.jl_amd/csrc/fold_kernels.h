@@ -565,120 +565,185 @@ __global__ __launch_bounds__(256) void k_phi_ipolar4_fold(const R* __restrict__ 
         for (int ss = 0; ss < 4; ++ss) o[4 * j1 + ss] = sc * acc[1][ss];
 }
 
-// Per galaxy and map range blockIdx.y (whole knot groups): part = (sum_q g_q(r) dbar_q, sum_q g'_q(r)
-// dbar_q) on folded delta-bar maps and uniform knots.  Galaxies grouped by folded pixel (a
-// wave's delta-bar loads fall on a few lines); their segment slot and t are found from the radii
-// once per knot group, then NM maps' records are staged in LDS at a time.
+// Per galaxy and map range blockIdx.y (`step` runs of whole knot groups): part = (sum_q g_q(r) dbar_q,
+// sum_q g'_q(r) dbar_q) on folded delta-bar maps and uniform knots.  Galaxies come in radius bins,
+// by folded pixel inside a bin (a wave's delta-bar loads fall on a few lines); their segment slot
+// and t are found from the radii once per knot group.  Of each map's records only the block's
+// radial range is staged, so several maps fit in LDS at a time and each is staged from L2 for the
+// radii that need it (any order of the galaxies is right); the next map's delta-bar is loaded
+// while one is summed.
 // Value and slope come from one Horner chain (5 fma); the slopes of a group share the segment's
-// 1/h, applied once to their sum.  Outside the knots the pseudo-records' slopes are 0.  R = float: FP32 records,
-// delta-bar and products, FP64 sums.  Bound: the random 16-byte record reads from LDS.
-constexpr int VF_GPT = 6;
-template <typename R, int NM>
-__global__ __launch_bounds__(1024) void k_vjp_fold(int64_t N, int64_t npf, int32_t cap, const double* __restrict__ r_s,
-                                                   const uint32_t* __restrict__ pix_s,
-                                                   const GroupInfo* __restrict__ groups,
-                                                   const double* __restrict__ gx, const double* __restrict__ grh,
-                                                   const int32_t* __restrict__ vgs, const int32_t* __restrict__ vgm,
-                                                   const int2* __restrict__ vrange, const MapInfo* __restrict__ maps,
-                                                   const typename Vec4T<R>::T* __restrict__ rec4,
-                                                   const R* __restrict__ dbar, double2* __restrict__ part)
+// 1/h, applied once to their sum.  Outside the knots the pseudo-records' slopes are 0.  R = float:
+// FP32 records, delta-bar and products, FP64 sums.
+// Bound: VALU (82% busy in FP32, 19 instructions per galaxy and map), then the random 16-byte
+// record reads from LDS.  1e6 galaxies, 2514 maps, FP32: 1.69 ms; whole tables staged, two
+// at a time by 1024 threads, ran 2.87 ms and moved 5.4 GB past L2.
+constexpr int VF_THR = 512;         // two blocks per CU: one sums while the other stages
+constexpr int VF_MAPS = 16;          // maps per stage at most
+constexpr int VF_LDS = 78 << 10;
+constexpr int VF_BIN = 7 << 10;     // record bytes of one map in a radius bin (40 KB: 4.04 ms, 10: 2.42, 7: 2.18, 5: 2.17, 3: 2.24)
+constexpr int VF_BLOCKS = 2048;     // blocks wanted
+template <typename R> struct VfGpt { static constexpr int N = sizeof(R) == 8 ? 4 : 8; };  // galaxies per thread
+__device__ __forceinline__ float vf_flip(float d, uint32_t s) { return __uint_as_float(__float_as_uint(d) ^ s); }
+__device__ __forceinline__ double vf_flip(double d, uint32_t s)
+{
+    return __hiloint2double(__double2hiint(d) ^ (int)s, __double2loint(d));
+}
+template <typename R>
+__global__ __launch_bounds__(VF_THR, 4) void k_vjp_fold(int64_t N, int64_t npf, int32_t lds, int32_t step, int32_t nrange,
+                                                      const double* __restrict__ r_s,
+                                                      const uint32_t* __restrict__ pix_s,
+                                                      const GroupInfo* __restrict__ groups,
+                                                      const double* __restrict__ gx, const double* __restrict__ grh,
+                                                      const int32_t* __restrict__ vgs, const int32_t* __restrict__ vgm,
+                                                      const int2* __restrict__ vrange,
+                                                      const MapInfo* __restrict__ maps,
+                                                      const typename Vec4T<R>::T* __restrict__ rec4,
+                                                      const R* __restrict__ dbar, double2* __restrict__ part)
 {
     typedef typename Vec4T<R>::T R4;
-    extern __shared__ double4 vf_raw[];
-    R4* tb = (R4*)vf_raw;  // NM tables of cap + 1 records, one slot up: y_first, segments, y_last
-    const int64_t k0 = (int64_t)blockIdx.x * (1024 * VF_GPT) + threadIdx.x;
-    double r[VF_GPT], aw[VF_GPT], ar[VF_GPT];
-    R t[VF_GPT];
-    int ii[VF_GPT];
-    uint32_t pf[VF_GPT], south = 0;
+    constexpr int GPT = VfGpt<R>::N, NW = VF_THR / 64;
+    extern __shared__ double4 vf_raw[];  // lds bytes
+    R4* tb = (R4*)vf_raw;
+    __shared__ double rr[2 * NW];
+    __shared__ int64_t base[VF_MAPS];  // first record of each staged map
+    __shared__ int32_t mapq[VF_MAPS];
+    const int64_t k0 = (int64_t)blockIdx.x * (VF_THR * GPT) + threadIdx.x;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    double aw[GPT], ar[GPT];
+    uint32_t pf[GPT], south = 0;  // byte offsets of the pixels
+    double rlo = INFINITY, rhi = -INFINITY;
+    auto radius = [&](int u) { return r_s[min(k0 + VF_THR * u, N - 1)]; };  // past the end: computed and dropped
 #pragma unroll
-    for (int u = 0; u < VF_GPT; ++u) {
-        const int64_t k = min(k0 + 1024 * u, N - 1);  // past the end: computed and dropped
-        r[u] = r_s[k];
-        pf[u] = pix_s[k] >> 1;
-        south |= (pix_s[k] & 1u) << u;
+    for (int u = 0; u < GPT; ++u) {
+        const double r = radius(u);
+        const uint32_t px = pix_s[min(k0 + VF_THR * u, N - 1)];
+        pf[u] = (px >> 1) * (uint32_t)sizeof(R);
+        south |= (px & 1u) << u;
         aw[u] = ar[u] = 0.0;
+        rlo = fmin(rlo, r);  // (NaN is passed over)
+        rhi = fmax(rhi, r);
     }
-    const int2 rg = vrange[blockIdx.y];
-    for (int g = rg.x; g < rg.y; ++g) {
+    for (int o = 32; o > 0; o >>= 1) {
+        rlo = fmin(rlo, __shfl_xor(rlo, o, 64));
+        rhi = fmax(rhi, __shfl_xor(rhi, o, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        rr[threadIdx.x >> 6] = rlo;
+        rr[NW + (threadIdx.x >> 6)] = rhi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        rlo = fmin(rlo, rr[i]);
+        rhi = fmax(rhi, rr[NW + i]);
+    }
+    const int g0 = vrange[blockIdx.y * step].x, g1 = vrange[min((int)(blockIdx.y + 1) * step, nrange) - 1].y;
+    // delta-bar of the range's maps in order, one map ahead of the sums
+    const int jend = vgs[g1];
+    R dn[GPT];
+    auto load_dbar = [&](int j) {
+        const char* dq = (const char*)(dbar + (int64_t)vgm[min(j, jend - 1)] * npf);
+#pragma unroll
+        for (int u = 0; u < GPT; ++u) dn[u] = *(const R*)(dq + pf[u]);
+    };
+    load_dbar(vgs[g0]);
+    for (int g = g0; g < g1; ++g) {
         const GroupInfo G = groups[g];
         const double ainv = G.invdx, c0 = -G.xfirst * G.invdx, top = (double)(G.nk - 1);
-        double gr[VF_GPT];
-#pragma unroll
-        for (int u = 0; u < VF_GPT; ++u) {
+        // the block's slots: uniform-grid slots of its end radii, one to spare for the knots' rounding
+        // (NaN radii only: slot 0)
+        const double flo = fmin(fmax(floor(fma(rlo, ainv, c0)), -1.0), top);
+        const double fhi = fmin(fmax(floor(fma(rhi, ainv, c0)), -1.0), top);
+        const int lo = __builtin_amdgcn_readfirstlane(rlo <= rhi ? max((int)flo, 0) : 0);
+        const int hi = __builtin_amdgcn_readfirstlane(rlo <= rhi ? min((int)fhi + 2, G.nk) : 0);
+        const int nrec = hi - lo + 1;  // (nk + 1 records always fit)
+        const int fit = min(VF_MAPS, lds / (nrec * (int)sizeof(R4)));
+        // segment slot (0 and nk: outside) and t of a radius
+        auto locate = [&](double r, double& t) -> int {
             // the end knots belong to the end segments (their slopes), outside is flat
-            const double v = fma(r[u], ainv, c0), fl = fmin(fmax(floor(v), 0.0), top - 1.0);
-            const bool below = r[u] < G.xfirst, above = r[u] > G.xlast;
-            double tt = v - fl;
+            const double v = fma(r, ainv, c0), fl = fmin(fmax(floor(v), 0.0), top - 1.0);
             int i = (int)fl;  // NaN: segment 0, t NaN
-            if (sizeof(R) == 8 && r[u] == r[u]) {
+            t = v - fl;
+            if (sizeof(R) == 8 && r == r) {
                 // the caller's knots and the correctly rounded t of k_seg_t (the uniform grid's t
                 // is off by the knots' own rounding, 1e-13)
                 const double* xs = gx + G.xoff;
                 double x0 = xs[i], x1 = xs[i + 1];
-                if (r[u] < x0 && i > 0) {
+                if (r < x0 && i > 0) {
                     x1 = x0;
                     x0 = xs[--i];
-                } else if (r[u] >= x1 && i < G.nk - 2) {
+                } else if (r >= x1 && i < G.nk - 2) {
                     x0 = x1;
                     x1 = xs[++i + 1];
                 }
-                const double h = x1 - x0, n = r[u] - x0, y = grh[G.xoff + i], q0 = n * y;
-                tt = fma(fma(-h, q0, n), y, q0);
+                const double h = x1 - x0, n = r - x0, y = grh[G.xoff + i], q0 = n * y;
+                t = fma(fma(-h, q0, n), y, q0);
             }
-            ii[u] = below ? 0 : (above ? G.nk : i + 1);
-            t[u] = below || above ? (R)0 : (R)tt;
+            if (r < G.xfirst || r > G.xlast) t = 0.0;
+            return r < G.xfirst ? 0 : (r > G.xlast ? G.nk : i + 1);
+        };
+        int ii[GPT];
+        R t[GPT];
+        double gr[GPT];
+#pragma unroll
+        for (int u = 0; u < GPT; ++u) {
+            double tt;
+            ii[u] = min(max(locate(radius(u), tt) - lo, 0), nrec - 1);  // (clamped: NaN)
+            t[u] = (R)tt;
             gr[u] = 0.0;
         }
-        for (int j = vgs[g]; j < vgs[g + 1]; j += NM) {
-            R dd[NM][VF_GPT];
-            int nm = min(NM, vgs[g + 1] - j);
-#pragma unroll
-            for (int v = 0; v < NM; ++v) {
-                const int q = vgm[min(j + v, vgs[g + 1] - 1)];
-                const R* dq = dbar + (int64_t)q * npf;
-#pragma unroll
-                for (int u = 0; u < VF_GPT; ++u) dd[v][u] = dq[pf[u]];
-            }
+        for (int j = vgs[g]; j < vgs[g + 1]; j += fit) {
+            const int nm = min(fit, vgs[g + 1] - j);
             __syncthreads();  // the previous maps' records are no longer read
-#pragma unroll
-            for (int v = 0; v < NM; ++v)
-                if (v < nm) {
-                    const MapInfo m = maps[vgm[j + v]];
-                    const R4* rq = rec4 + m.koff + vgm[j + v];
-                    for (int e = threadIdx.x; e <= m.nk; e += blockDim.x)
-                        lds_rec_put(tb + v * (cap + 1), cap + 1, e < m.nk - 1 ? e + 1 : (e == m.nk - 1 ? 0 : e), rq[e]);
-                }
+            if ((int)threadIdx.x < nm) {
+                const int q = vgm[j + threadIdx.x];
+                base[threadIdx.x] = maps[q].koff + q;
+                mapq[threadIdx.x] = maps[q].l & 1;
+            }
             __syncthreads();
+            const int nch = (nrec + 63) >> 6;  // a wave copies 64 records of one map at a time
+            for (int c = wave; c < nm * nch; c += NW) {
+                const int v = c / nch, k = (c - v * nch) * 64 + lane, sl = lo + k;
+                // slot 0 holds y_first (record nk - 1), 1 .. nk - 1 the segments, nk y_last
+                const int64_t bq = base[v];
+                const R4* rq = rec4 + (((int64_t)__builtin_amdgcn_readfirstlane((int)(bq >> 32)) << 32) |
+                                       (uint32_t)__builtin_amdgcn_readfirstlane((int)bq));
+                if (k < nrec) lds_rec_put(tb + v * nrec, nrec, k, rq[sl == 0 ? G.nk - 1 : (sl == G.nk ? sl : sl - 1)]);
+            }
+            __syncthreads();
+            for (int v = 0; v < nm; ++v) {
+                const int mq = __builtin_amdgcn_readfirstlane(mapq[v]);
+                const uint32_t flip = (mq & 1) ? south : 0u;  // odd l: southern galaxies take -dbar
+                R d[GPT];
 #pragma unroll
-            for (int v = 0; v < NM; ++v) {
-                if (v >= nm) break;
-                const uint32_t flip = (maps[vgm[j + v]].l & 1) ? south : 0u;
+                for (int u = 0; u < GPT; ++u) d[u] = vf_flip(dn[u], (flip >> u) << 31);
+                load_dbar(j + v + 1);  // (a range's maps are consecutive)
+                const R4* tv = tb + v * nrec;
 #pragma unroll
-                for (int u = 0; u < VF_GPT; ++u) {
-                    const R4 c = lds_rec_get(tb + v * (cap + 1), cap + 1, ii[u]);  // (d, c, b, a)
+                for (int u = 0; u < GPT; ++u) {
+                    const R4 c = lds_rec_get(tv, nrec, ii[u]);  // (d, c, b, a)
                     const R x = t[u];
                     const R p1 = fma(x, c.w, c.z), p2 = fma(x, p1, c.y);
                     const R val = fma(x, p2, c.x);
                     const R slope = fma(x, fma(x, c.w, p1), p2);
-                    const R d = ((flip >> u) & 1u) ? -dd[v][u] : dd[v][u];
                     if (sizeof(R) == 8) {
-                        aw[u] = fma((double)val, (double)d, aw[u]);
-                        gr[u] = fma((double)slope, (double)d, gr[u]);
+                        aw[u] = fma((double)val, (double)d[u], aw[u]);
+                        gr[u] = fma((double)slope, (double)d[u], gr[u]);
                     } else {
-                        aw[u] += (double)(val * d);
-                        gr[u] += (double)(slope * d);
+                        aw[u] += (double)(val * d[u]);
+                        gr[u] += (double)(slope * d[u]);
                     }
                 }
             }
         }
 #pragma unroll
-        for (int u = 0; u < VF_GPT; ++u)
-            ar[u] = fma(gr[u], sizeof(R) == 8 ? grh[G.xoff + min(max(ii[u] - 1, 0), G.nk - 2)] : ainv, ar[u]);
+        for (int u = 0; u < GPT; ++u)
+            ar[u] = fma(gr[u], sizeof(R) == 8 ? grh[G.xoff + min(max(ii[u] + lo - 1, 0), G.nk - 2)] : ainv, ar[u]);
     }
 #pragma unroll
-    for (int u = 0; u < VF_GPT; ++u) {
-        const int64_t k = k0 + 1024 * u;
+    for (int u = 0; u < GPT; ++u) {
+        const int64_t k = k0 + VF_THR * u;
         if (k < N) part[(int64_t)blockIdx.y * N + k] = make_double2(aw[u], ar[u]);
     }
 }

@@ -21,12 +21,20 @@ __global__ __launch_bounds__(256) void k_zero_counts(int64_t npix, int32_t* __re
     if (i < 4) flag[i] = 0;
 }
 
+// Radius bins in front of the pixels (bin major; n <= 1: none), for consumers that want a block's
+// galaxies in a narrow radial range.  The bin of a galaxy only orders the list.
+struct RadBins {
+    int32_t n;
+    uint32_t np2;      // folded pixels with the hemisphere bit: 2 npf per bin
+    double r0, inv;    // bin = (r - r0) inv, clamped
+};
+
 // pixel (FOLD: folded, with the hemisphere in bit 0) and arrival rank of every galaxy.
 // flag[1] |= 1 when an angle is not finite (the reference's floor(Int, NaN) throws).
 template <bool FOLD>
 __global__ __launch_bounds__(256) void k_count(int64_t N, const double* __restrict__ rtp, int64_t nside,
                                                int32_t* __restrict__ cnt, uint2* __restrict__ pr,
-                                               int32_t* __restrict__ flag)
+                                               int32_t* __restrict__ flag, RadBins rb)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
@@ -38,7 +46,8 @@ __global__ __launch_bounds__(256) void k_count(int64_t N, const double* __restri
     } else {
         atomicOr(flag + 1, 1);
     }
-    const uint32_t f = FOLD ? fold_pixel(p, nside) : (uint32_t)p;
+    uint32_t f = FOLD ? fold_pixel(p, nside) : (uint32_t)p;
+    if (FOLD && rb.n > 1) f += rb.np2 * (uint32_t)fmin(fmax((rtp[3 * i] - rb.r0) * rb.inv, 0.0), (double)(rb.n - 1));
     pr[i] = make_uint2(f, (uint32_t)atomicAdd(cnt + (FOLD ? f >> 1 : f), 1));
 }
 
@@ -118,7 +127,8 @@ struct alignas(32) CatSlot {
 
 __global__ __launch_bounds__(256) void k_place(int64_t N, const uint2* __restrict__ pr,
                                                const int32_t* __restrict__ pstart, const double* __restrict__ rtp,
-                                               const double* __restrict__ w, int32_t sh, CatSlot* __restrict__ slot)
+                                               const double* __restrict__ w, int32_t sh, CatSlot* __restrict__ slot,
+                                               uint32_t np2)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= N) return;
@@ -127,7 +137,7 @@ __global__ __launch_bounds__(256) void k_place(int64_t N, const uint2* __restric
     c.r = rtp[3 * i];
     c.w = w ? w[i] : 1.0;
     c.i = (uint32_t)i;
-    c.pix = q.x;
+    c.pix = np2 ? q.x % np2 : q.x;  // without the radius bin
     slot[(int64_t)pstart[q.x >> sh] + q.y] = c;
 }
 

@@ -3108,6 +3108,7 @@ struct sfb_plan {
     DevBuf d_pinfo, d_pwin;  // per slice lane: (pixel, count), separable window factor
     DevBuf d_vgm, d_vgs, d_vrange;  // adjoint gather: group-ordered maps, group starts, map ranges
     int32_t nvrange = 0;
+    double r_first = 0.0, r_last = 1.0;  // the outermost knots of all maps (radius bins)
     // knot groups (maps with bit-identical knots) and the shared segment search
     int32_t ngroup = 0, nk_max_group = 0;
     // every group's knots uniform to 1e-9 of their spacing: the mixed-path scatter finds
@@ -3240,6 +3241,8 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
     for (int64_t qq = 0; qq < P->nmaps; ++qq) {
         int64_t o = knot_off[qq], nk = knot_off[qq + 1] - knot_off[qq];
         P->tbl_cap = std::max<int32_t>(P->tbl_cap, (int32_t)nk);
+        P->r_first = qq ? std::min(P->r_first, kx[o]) : kx[o];
+        P->r_last = qq ? std::max(P->r_last, kx[o + nk - 1]) : kx[o + nk - 1];
         for (int64_t i = 0; i < nk; ++i) {
             double a = 0.0;
             if (i + 1 < nk) {
@@ -3906,18 +3909,21 @@ static int64_t sell_bound(const sfb_plan* P, int64_t N, int64_t np)
 // Groups the catalogue by pixel: cat_idx, pstart, and pixel, r and w in that order; slots: also
 // the sliced layout sr, sw (soff, pinfo) when the records fit in LDS (the per-map scatter reads
 // it; the shells' spread and the adjoint's gather do not).  fold: by folded pixel (fold_pixel).
+// nbin > 1 (fold, CAT_ANY, no slots): in radius bins, by pixel inside a bin.
 static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const double* d_w, hipStream_t st,
-                         CatOrder order, bool slots, bool fold = false)
+                         CatOrder order, bool slots, bool fold = false, int32_t nbin = 1)
 {
     int rc;
     const int64_t np = fold ? P->fold.npf : P->npix;
+    const int64_t ncell = np * nbin;  // counters
+    const RadBins rb{nbin, (uint32_t)(2 * np), P->r_first, (double)nbin / (P->r_last - P->r_first)};
     const int32_t sh = fold ? 1 : 0;  // folded pixels carry the hemisphere in bit 0
     P->cat_np = np;
     P->cat_fold = fold;
     if (N > 0x7fffffff) return fail(SFB_ERR_ARG, "N > 2^31-1 galaxies");
     P->ncat = N;
     P->unit_w = d_w == nullptr;
-    if ((rc = P->d_pstart.ensure(sizeof(int32_t) * (size_t)(P->npix + 1)))) return rc;
+    if ((rc = P->d_pstart.ensure(sizeof(int32_t) * (size_t)(std::max(P->npix, ncell) + 1)))) return rc;
     if (N == 0) {
         hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P->d_flag.as<int32_t>(), 4, 0);
         LAUNCH_CHECK();
@@ -3936,29 +3942,30 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         return rc;
     PhaseTimer timer(P, SFB_PHASE_CATALOG, st);
     if (!P->crowded && N <= PS_MEAN * np) {
-        const unsigned nb = nblk(np, PS_CHUNK);
-        if ((rc = P->d_cnt.ensure(sizeof(int32_t) * ((size_t)np + nb))) ||
+        const unsigned nb = nblk(ncell, PS_CHUNK);
+        if ((rc = P->d_cnt.ensure(sizeof(int32_t) * ((size_t)ncell + nb))) ||
             (rc = P->d_sorttmp.ensure(sizeof(CatSlot) * n)))
             return rc;
         int32_t* cnt = P->d_cnt.as<int32_t>();
-        int32_t* sums = cnt + np;
-        hipLaunchKernelGGL(k_zero_counts, dim3(nblk(np, 256)), dim3(256), 0, st, np, cnt,
+        int32_t* sums = cnt + ncell;
+        hipLaunchKernelGGL(k_zero_counts, dim3(nblk(ncell, 256)), dim3(256), 0, st, ncell, cnt,
                            P->d_flag.as<int32_t>());
         LAUNCH_CHECK();
         hipLaunchKernelGGL((fold ? k_count<true> : k_count<false>), dim3(nblk(N, 256)), dim3(256), 0, st, N, d_rtp, P->nside, cnt,
-                           P->d_keyr.as<uint2>(), P->d_flag.as<int32_t>());
+                           P->d_keyr.as<uint2>(), P->d_flag.as<int32_t>(), rb);
         LAUNCH_CHECK();
         int32_t* crowd = order == CAT_ANY ? nullptr : P->d_flag.as<int32_t>();
         const bool small = nb <= (unsigned)PS_SMALL;
         if (!small) {
-            hipLaunchKernelGGL(k_count_sums, dim3(nb), dim3(256), 0, st, np, cnt, sums, crowd);
+            hipLaunchKernelGGL(k_count_sums, dim3(nb), dim3(256), 0, st, ncell, cnt, sums, crowd);
             LAUNCH_CHECK();
         }
-        hipLaunchKernelGGL(k_count_scan, dim3(nb), dim3(256), 0, st, np, (int32_t)N, cnt,
+        hipLaunchKernelGGL(k_count_scan, dim3(nb), dim3(256), 0, st, ncell, (int32_t)N, cnt,
                            small ? (const int32_t*)nullptr : sums, P->d_pstart.as<int32_t>(), crowd);
         LAUNCH_CHECK();
         hipLaunchKernelGGL(k_place, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_keyr.as<uint2>(),
-                           P->d_pstart.as<int32_t>(), d_rtp, d_w, sh, P->d_sorttmp.as<CatSlot>());
+                           P->d_pstart.as<int32_t>(), d_rtp, d_w, sh, P->d_sorttmp.as<CatSlot>(),
+                           nbin > 1 ? rb.np2 : 0u);
         LAUNCH_CHECK();
         auto rank = [&](auto kern) -> int {
             hipLaunchKernelGGL(kern, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_sorttmp.as<CatSlot>(),
@@ -4972,36 +4979,43 @@ extern "C" int sfb_cat2amln_vjp_device(sfb_plan* P, int64_t N, const double* d_r
     // folded hemispheres on uniform knots (records in LDS by P->fold.ok); the split-BF16
     // precisions keep the iterated refinement whose products they select
     const size_t one = (f32 ? 16 : 32) * (size_t)(P->tbl_cap + 1);
-    const bool fold = P->fold.ok && P->seg_uniform && grouped && (int64_t)one <= P->lds_max &&
+    const bool fold = P->fold.ok && P->seg_uniform && grouped && (int64_t)one + 512 <= P->lds_max &&
                       (P->precision == SFB_PREC_FP64 || P->precision == SFB_PREC_MIXED);
-    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, CAT_ANY, false, fold))) return rc;
+    // radius bins: a bin's records of a map take at most VF_BIN bytes of LDS
+    // (no more counters than 4 N: they are cleared and scanned)
+    const int64_t bmax = std::min<int64_t>(16, 4 * N / std::max<int64_t>(1, P->fold.npf));
+    const int32_t nbin =
+        fold ? (int32_t)std::max<int64_t>(1, std::min<int64_t>(bmax, nblk((int64_t)one, VF_BIN))) : 1;
+    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, CAT_ANY, false, fold, nbin))) return rc;
     PhaseTimer tj(P, SFB_PHASE_ADJOINT, st);
     const double domega = 4.0 * kPi / (double)P->npix;
     int32_t ngroups;
     if (fold) {
-        ngroups = P->nvrange;
+        // map ranges: as few as fill the chip (each writes and re-reads 16 B per galaxy)
+        const int64_t nb = nblk(N, VF_THR * (f32 ? VfGpt<float>::N : VfGpt<double>::N));
+        int32_t step = 1;
+        while (step < P->nvrange && nb * ((P->nvrange + 2 * step - 1) / (2 * step)) >= VF_BLOCKS) step *= 2;
+        ngroups = (P->nvrange + step - 1) / step;
         if ((rc = P->d_part.ensure(sizeof(double2) * (size_t)ngroups * (size_t)N))) return rc;
-        // two record tables per stage while two blocks still share a CU's LDS
-        const bool two = 4 * one <= (size_t)P->lds_max;
-        const size_t shm = two ? 2 * one : one;
-        const dim3 gv(nblk(N, 1024 * VF_GPT), (unsigned)ngroups);
+        // a whole map's records (any radial range), or the budget
+        const size_t shm = std::min((size_t)P->lds_max - 512, std::max(one, (size_t)VF_LDS));
+        const dim3 gv((unsigned)nb, (unsigned)ngroups);
         auto go = [&](auto kern, const auto* rec4, const auto* dbar) -> int {
             HIP_TRY(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-            hipLaunchKernelGGL(kern, gv, dim3(1024), shm, st, N, P->fold.npf, P->tbl_cap, P->d_rs.as<double>(),
-                               P->d_pixkey2.as<uint32_t>(), P->d_groups.as<GroupInfo>(), P->d_gx.as<double>(),
-                               P->d_grh.as<double>(), P->d_vgs.as<int32_t>(), P->d_vgm.as<int32_t>(), P->d_vrange.as<int2>(), P->d_maps.as<MapInfo>(), rec4, dbar,
-                               P->d_part.as<double2>());
+            hipLaunchKernelGGL(kern, gv, dim3(VF_THR), shm, st, N, P->fold.npf, (int32_t)shm, step,
+                               P->nvrange, P->d_rs.as<double>(), P->d_pixkey2.as<uint32_t>(),
+                               P->d_groups.as<GroupInfo>(), P->d_gx.as<double>(), P->d_grh.as<double>(),
+                               P->d_vgs.as<int32_t>(), P->d_vgm.as<int32_t>(), P->d_vrange.as<int2>(),
+                               P->d_maps.as<MapInfo>(), rec4, dbar, P->d_part.as<double2>());
             LAUNCH_CHECK();
             return SFB_OK;
         };
         if (f32) {
             if ((rc = fold_synthesis<float>(P, d_cot, domega, st))) return rc;
-            rc = two ? go(k_vjp_fold<float, 2>, P->d_rec4f.as<float4>(), P->d_delta.as<float>())
-                     : go(k_vjp_fold<float, 1>, P->d_rec4f.as<float4>(), P->d_delta.as<float>());
+            rc = go(k_vjp_fold<float>, P->d_rec4f.as<float4>(), P->d_delta.as<float>());
         } else {
             if ((rc = fold_synthesis<double>(P, d_cot, domega, st))) return rc;
-            rc = two ? go(k_vjp_fold<double, 2>, P->d_rec4.as<double4>(), P->d_delta.as<double>())
-                     : go(k_vjp_fold<double, 1>, P->d_rec4.as<double4>(), P->d_delta.as<double>());
+            rc = go(k_vjp_fold<double>, P->d_rec4.as<double4>(), P->d_delta.as<double>());
         }
         if (rc) return rc;
     } else {
