@@ -48,8 +48,7 @@ static int fold_tables(sfb_plan* P)
     for (size_t c = 0; c < qs.size(); ++c) {
         const MapInfo& mi = P->maps[(size_t)qs[c]];
         F.neven += !(mi.l & 1);
-        cols[c] = {qs[c], mi.l, std::max<int32_t>(mi.l, mal), 0, P->out_base[(size_t)qs[c]]};
-        cols[c].j = (int32_t)c - ((mi.l & 1) ? F.neven : 0);
+        cols[c] = {qs[c], mi.l, std::max<int32_t>(mi.l, mal), P->out_base[(size_t)qs[c]]};
     }
     std::vector<FoldM> fm((size_t)(L + 1));
     F.maxcnt = 1;

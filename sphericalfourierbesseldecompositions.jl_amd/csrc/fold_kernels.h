@@ -17,7 +17,6 @@
 struct FoldCol {
     int32_t q, l;     // the map and its l
     int32_t mtop;     // X kept for m <= mtop: max(l, largest aliasing m)
-    int32_t j;        // position in its parity's run
     int64_t out;      // index of a_{nl0}
 };
 // Per m: the analysis tables of the two l parities (block (m, par = (l + m) & 1)).
@@ -65,7 +64,8 @@ __device__ __forceinline__ void store_fold1(double* __restrict__ X, int64_t ld, 
 }
 
 // Equatorial ring pairs of folded maps: k_phi_fft with one sequence per map (TQ columns per
-// block).  X[(m K + k) ld + 2 c].
+// block).  X[(m K + k) ld + 2 c].  Bound: FP64 butterflies (VALU 49% busy) and their LDS passes (42%).
+// nside 128, 2514 maps: 561 us (unfolded, two sequences per map: 1.10 ms).
 __global__ __launch_bounds__(512) void k_phi_fft_fold(const double* __restrict__ delta, int64_t npf, int32_t ncol,
                                                       int64_t ld, int32_t K, const RingDev* __restrict__ rings,
                                                       const double2* __restrict__ tw, double* __restrict__ X,
@@ -126,7 +126,9 @@ __global__ __launch_bounds__(512) void k_phi_fft_fold(const double* __restrict__
 }
 
 // Polar ring pairs of folded maps: k_phi_polar4 with one sequence per map (twice its maps per
-// block for the same tiles).
+// block for the same tiles).  Bound: VALU (57%: gathers, indexes, X stores) around the MFMA product, which
+// takes even and odd sample parts (p4_product_sym).  nside 128, 2514 maps: 501 us (597 with the
+// whole product, 1.20 ms unfolded).
 template <int MTWMAX>
 __global__ __launch_bounds__(256) void k_phi_polar4_fold(const double* __restrict__ delta, int64_t npf, int32_t ncol,
                                                          int64_t ld, int32_t K, const RingDev* __restrict__ rings,
@@ -206,7 +208,8 @@ __global__ __launch_bounds__(256) void k_phi_polar4_fold(const double* __restric
 // a_lm of every map and m <= l from the ring coefficients and the aliasing steps' values r, and
 // its place in the a_nlm vector.  A block takes one m, one l parity and 64 columns, its four waves
 // a quarter of the ring pairs each (eight rows of X in flight per thread).  Bound: X read once
-// (16 B per column, m <= l and ring pair).
+// (16 B per column, m <= l and ring pair).  nside 128, 2514 maps: 125 us; a product for every l' of
+// each map in its place ran 680 us.
 __global__ __launch_bounds__(256) void k_fold_rows(int32_t K, int32_t J, int64_t ld, const FoldM* __restrict__ fm,
                                                    const FoldCol* __restrict__ cols, int32_t neven,
                                                    const double* __restrict__ lam, const double* __restrict__ ZB,
@@ -260,7 +263,7 @@ __global__ __launch_bounds__(256) void k_fold_rows(int32_t K, int32_t J, int64_t
 // ---- the transposed direction (adjoint): cotangent -> folded delta-bar maps ------------------
 
 // h of the aliasing steps from the cotangent b = D_half c: h[s, j] = (U_j^T b)[state], b only at
-// row l.  Zero where m > l.
+// row l.  Zero where m > l.  13 us at nside 128 (h written once; launch and latency).
 __global__ __launch_bounds__(256) void k_fold_coth(int32_t J, int32_t ncol, int64_t ld, const FoldM* __restrict__ fm,
                                                    const FoldCol* __restrict__ cols, int32_t neven,
                                                    const double* __restrict__ UB, const double* __restrict__ cot,
@@ -293,6 +296,7 @@ __global__ __launch_bounds__(256) void k_fold_coth(int32_t J, int32_t ncol, int6
 // X_m[k] = (Lam P_J)[k][l] b_m + sum_h GZ[h][k] r_h, m <= mtop.  A block takes one m, 64 columns of one
 // l parity and 32 ring pairs, a wave 8 of them: the aliasing tables' entries are wave-uniform
 // (scalar loads; per-lane loads of them ran 548 us at nside 128).  Bound: X written once.
+// nside 128, 2514 maps, FP32 X: 221 us (synthesis of every l' by products: 1.69 ms with the refinement).
 template <typename R>
 __global__ __launch_bounds__(256) void k_fold_synth(int32_t K, int32_t J, int32_t ncol, int64_t ld,
                                                     const FoldM* __restrict__ fm, const FoldCol* __restrict__ cols,
@@ -364,6 +368,7 @@ __global__ __launch_bounds__(256) void k_fold_synth(int32_t K, int32_t J, int32_
 }
 
 // Equatorial ring pairs, inverse: k_phi_ifft with one sequence per map; out[q][f] in pixel order.
+// Bound as k_phi_fft_fold.  nside 128, 2514 maps, FP32: 415 us (unfolded 1.09 ms).
 template <typename R>
 __global__ __launch_bounds__(512) void k_phi_ifft_fold(const R* __restrict__ X, int64_t npf, int32_t ncol, int64_t ld,
                                                        int32_t K, int32_t L, const RingDev* __restrict__ rings,
@@ -451,7 +456,8 @@ __global__ __launch_bounds__(512) void k_phi_ifft_fold(const R* __restrict__ X, 
     }
 }
 
-// Polar ring pairs, inverse: k_phi_ipolar4 with one sequence per map.
+// Polar ring pairs, inverse: k_phi_ipolar4 with one sequence per map.  Bound: the direct length-i DFTs
+// (VALU) and their LDS reads (79% busy).  nside 128, 2514 maps, FP32: 505 us (unfolded 1.44 ms).
 template <typename R>
 __global__ __launch_bounds__(256) void k_phi_ipolar4_fold(const R* __restrict__ X, int64_t npf, int32_t ncol, int64_t ld,
                                                           int32_t K, const RingDev* __restrict__ rings,

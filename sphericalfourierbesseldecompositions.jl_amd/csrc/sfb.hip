@@ -2,26 +2,23 @@
 // (src/cat2anlm.jl:257-310 in hsgg/SphericalFourierBesselDecompositions.jl 0.5.19).
 //
 // Pipeline of one call (all on one HIP stream):
-//   k_prep        ang2pix (ring scheme) + sortable r key per galaxy
-//   rocprim       stable radix sort by r, then stable radix sort by pixel
-//                 -> galaxies grouped by pixel, r-ordered inside a pixel, which is
-//                 the reference's summation order (sortout, cat2anlm.jl:50-71)
-//   k_gather      r, w in that order; k_pixel_start: first galaxy of every pixel;
-//                 k_sell_*: sliced layout (one wavefront lane per pixel)
-//   k_seg_t       per knot group (maps with identical knots) and galaxy: spline
-//                 segment i and t = (r - x_i)/h, correctly rounded
-//   k_scatter_it  delta[q][p] = (sum_{i in p} w_i g_q(r_i)) * 1/(nbar dOmega) - W_q(p)
-//                 with the reference's spline formula and rounding (cat2anlm.jl:284-291)
-//   k_phi_fft / k_phi_polar4
-//                 per ring pair (north k, south 4 nside-2-k): F_m = sum_j delta_j e^{-i m phi_j},
-//                 stored as E = F_N + F_S and O = F_N - F_S for m = 0..lmax
-//   Legendre      a_{l m} = dOmega sum_k lambda_lm(theta_k) (E or O by parity of l+m):
-//                 one batched FP64 MFMA GEMM per (m, parity) -- rows = (map, re/im),
-//                 K = ring pairs, columns = l
-//   niter times   synthesis G = a Lambda^T on the aliasing rings, k_alias: minus the
-//                 DFT of the synthesised short rings' aliases, a <- b + a (I - C0) +
-//                 dOmega R Lambda  (Healpix map2alm! niter loop, src/healpix_helpers.jl:50-56)
-//   k_pack        anlm[getidx(n,l,m)] = a^{(n,l)}_{l m}, m = 0..l, plus a non-finite flag
+//   pixel_sort.h  ang2pix (ring scheme), counting sort by pixel and a fixed order inside each pixel
+//                 (the reference's summation order on the FP64 path, sortout, cat2anlm.jl:50-71); stable
+//                 rocprim radix sorts where a pixel is crowded; k_sell_*: sliced layout (one
+//                 wavefront lane per pixel)
+//   FP64, on maps folded onto one hemisphere (fold.h):
+//     k_seg_t       per knot group (maps with identical knots) and galaxy: spline segment i and
+//                   t = (r - x_i)/h, correctly rounded
+//     k_scatter_it  delta[q][p] = (sum_{i in p} w_i g_q(r_i)) * 1/(nbar dOmega) - W_q(p)
+//                   with the reference's spline formula and rounding (cat2anlm.jl:284-291)
+//     k_phi_fft_fold / k_phi_polar4_fold   per ring pair F_m = sum_j delta_j e^{-i m phi_j}
+//     k_fold_rows   a_lm of map (n, l) as a dot product over ring pairs with the analysis table
+//                   that holds the niter refinements (Healpix map2alm!, src/healpix_helpers.jl:50-56;
+//                   sht_direct.h), into anlm[getidx(n,l,m)]
+//   mixed precision, separable windows: the same transforms in FP64 on ~160 radial shells instead
+//     of one map per (n, l) (shells.h)
+//   otherwise (dense mixed windows, split-BF16, tables or grids that those refuse): per-map scatter,
+//     k_phi_fft / k_phi_polar4, k_gemm_tall and niter Jacobi steps with k_alias, k_pack
 #include <hip/hip_runtime.h>
 
 #include <rocprim/device/device_radix_sort.hpp>
@@ -2714,27 +2711,40 @@ __global__ void k_wrl_sep(int32_t nmax, int32_t L, int64_t nr, const double* __r
 }
 
 // field2anlm: out[n,l,m] += sum_s dr r_s^2 g_nl(r_s) a^{(s)}_{l m} over the shells s of
-// this chunk (maps of the SHT), in the a layout of the Legendre step
-__global__ void k_field_contract(int32_t nmaps, int32_t Q, int64_t s0, int64_t nr, const double* __restrict__ r,
-                                 double dr, const double* __restrict__ gtab, const MapInfo* __restrict__ maps,
-                                 const int64_t* __restrict__ aoff, const int64_t* __restrict__ out_base, int64_t M2,
-                                 const double* __restrict__ a, double* __restrict__ out)
+// this chunk (maps of the SHT), in the a layout of the Legendre step.  Half a wavefront per (map, m), its
+// lanes along s, so that g's and a's rows are read coalesced (a lane per map, walking g with a stride of
+// nr and a by itself, ran 24.5 us at 75 shells and 344 maps; now 6.8).  Bound: latency at small grids, a's rows from L2 at large ones.
+constexpr int FC_W = 32;
+__global__ __launch_bounds__(256) void k_field_contract(int32_t nmaps, int32_t Q, int64_t s0, int64_t nr,
+                                                        const double* __restrict__ r, double dr,
+                                                        const double* __restrict__ gtab,
+                                                        const MapInfo* __restrict__ maps,
+                                                        const int64_t* __restrict__ aoff,
+                                                        const int64_t* __restrict__ out_base, int64_t M2,
+                                                        const double* __restrict__ a, double* __restrict__ out)
 {
-    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    const int q = blockIdx.x * (256 / FC_W) + threadIdx.x / FC_W, lane = threadIdx.x % FC_W;
     const int m = blockIdx.y;
     if (q >= nmaps) return;
     const int l = maps[q].l;
-    if (m > l) return;
+    if (m > l) return;  // (a half leaves as a whole)
     const int par = (l - m) & 1, j = (l - m) >> 1;
-    const double* src = a + (aoff[m * 2 + par] + j) * M2;
-    const double* g = gtab + (int64_t)q * nr;
+    const double2* src = (const double2*)(a + (aoff[m * 2 + par] + j) * M2);
+    const double* g = gtab + (int64_t)q * nr + s0;
     double sr = 0.0, si = 0.0;
-    for (int s = 0; s < Q; ++s) {
+#pragma unroll 4
+    for (int s = lane; s < Q; s += FC_W) {
         const double rs = r[s0 + s];
-        const double w = g[s0 + s] * rs * rs * dr;
-        sr += w * src[2 * s];
-        si += w * src[2 * s + 1];
+        const double w = g[s] * rs * rs * dr;
+        const double2 v = src[s];
+        sr += w * v.x;
+        si += w * v.y;
     }
+    for (int o = FC_W / 2; o > 0; o >>= 1) {
+        sr += __shfl_xor(sr, o, FC_W);
+        si += __shfl_xor(si, o, FC_W);
+    }
+    if (lane) return;
     out[2 * (out_base[q] + m)] += sr;
     out[2 * (out_base[q] + m) + 1] += si;
 }
@@ -5436,7 +5446,7 @@ extern "C" int sfb_field2anlm_device(sfb_plan* P, int64_t nr, const double* d_r,
         LAUNCH_CHECK();
         P->delta_perm = nullptr;  // the field's shells in pixel order
         if ((rc = sht_stage(P, Q, st, false))) return rc;
-        hipLaunchKernelGGL(k_field_contract, dim3(nblk(P->nmaps, 256), (unsigned)(P->lmax + 1)), dim3(256), 0, st,
+        hipLaunchKernelGGL(k_field_contract, dim3(nblk(P->nmaps, 256 / FC_W), (unsigned)(P->lmax + 1)), dim3(256), 0, st,
                            (int32_t)P->nmaps, Q, s0, nr, d_r, dr, P->d_gtab.as<double>(), P->d_maps.as<MapInfo>(),
                            P->d_aoff.as<int64_t>(), P->d_outbase.as<int64_t>(), P->a_ld, P->a_final, d_out);
         LAUNCH_CHECK();
