@@ -43,12 +43,13 @@ extern "C" {
 #define SFB_ERR_NOMEM 6      /* host allocation failed */
 
 #define SFB_PREC_FP64 0      /* plain path: reference method, FP64 throughout */
-#define SFB_PREC_MIXED 1     /* FP32 spline values, delta maps and phi-transform; the first Legendre
-                                analysis on FP64 MFMA over FP32 ring coefficients, the Jacobi passes
-                                on FP32 MFMA (FP32 iterate and aliasing buffers); FP64 setup, segment
-                                search, pixel sums, lambda tables, GEMM epilogues, aliasing sums and
-                                the l = 0 maps' monopoles.  Every (n,l) block within 1e-6 of FP64. */
-#define SFB_PREC_BF16X3 2    /* SFB_PREC_MIXED with the Jacobi GEMMs on bf16 MFMA: each FP32 operand split
+#define SFB_PREC_MIXED 1     /* separable windows: the splines represented on a common radial basis to
+                                half an FP32 unit, everything else in FP64.  Dense windows (and splines
+                                the basis does not represent): FP32 spline values, delta maps and ring
+                                coefficients, the first Legendre analysis on FP64 MFMA, the Jacobi passes
+                                on FP32 MFMA; FP64 setup, pixel sums, epilogues, aliasing sums and the
+                                l = 0 maps' monopoles.  Every (n,l) block within 1e-6 of FP64. */
+#define SFB_PREC_BF16X3 2    /* the FP32-map path with the Jacobi GEMMs on bf16 MFMA: each FP32 operand split
                                 into hi + mid + lo bf16 terms, six products, FP32 accumulation */
 #define SFB_PREC_BF16X2 3    /* the same with hi + lo terms, three products (~2^-16 per product; the
                                 Jacobi steps only correct the FP64-MFMA first analysis, so every
@@ -219,8 +220,8 @@ int sfb_amln2clnn_cross(sfb_plan* pa, sfb_plan* pb, int64_t nlnn, const int64_t*
  * a is affine in the window with dL/dW[p, l, n] = -dbar_{nl}(p), the synthesised
  * cotangent map this function forms internally, but no entry point hands it out.
  * A non-finite angle is an error (SFB_ERR_ARG), as in the forward call.  With a plan of
- * SFB_PREC_MIXED the adjoint runs in FP32 (Jacobi recursion, synthesis, delta-bar maps,
- * per-galaxy products) with FP64 sums over the maps; otherwise in FP64.
+ * SFB_PREC_MIXED the adjoint's synthesis, delta-bar maps and per-galaxy products run in FP32
+ * with FP64 sums over the maps; otherwise in FP64.
  * g'(r) is the spline derivative of src/Splines.jl:367-377
  * (derivative(gnl, n, l, r), src/GNLs.jl:110).  No counterpart in the reference,
  * which has no derivative of cat2amln; it backs the ChainRulesCore.rrule of the
@@ -261,13 +262,13 @@ int sfb_anlm2field_device(sfb_plan* p, int64_t nr, const double* d_r, const doub
 
 /* ---- per-phase timing ------------------------------------------------------ */
 
-#define SFB_PHASE_CATALOG 0    /* ang2pix, the two stable sorts, gathers, pixel segments */
-#define SFB_PHASE_SCATTER 1    /* spline evaluation + ordered per-pixel sums -> delta maps */
+#define SFB_PHASE_CATALOG 0    /* ang2pix, grouping by pixel, sliced layout */
+#define SFB_PHASE_SCATTER 1    /* ordered per-pixel sums -> delta maps (mixed: shell maps) */
 #define SFB_PHASE_PHI 2        /* phi-transform of the rings with 4 nside pixels (one FFT kernel) */
-#define SFB_PHASE_ANALYSIS 3   /* Legendre analysis GEMMs (1 + niter launches) */
-#define SFB_PHASE_SYNTHESIS 4  /* Legendre synthesis GEMMs (niter launches) */
-#define SFB_PHASE_RESIDUAL 5   /* ring-Fourier residual with aliasing (niter launches) */
-#define SFB_PHASE_PACK 6       /* a_nlm packing and the non-finite check */
+#define SFB_PHASE_ANALYSIS 3   /* Legendre analysis (one launch with the folded tables; else 1 + niter) */
+#define SFB_PHASE_SYNTHESIS 4  /* Legendre synthesis GEMMs (iterated refinement only: niter launches) */
+#define SFB_PHASE_RESIDUAL 5   /* aliasing of short rings (folded: one solve; else niter launches) */
+#define SFB_PHASE_PACK 6       /* a_nlm packing (mixed: radial contraction) and the non-finite check */
 #define SFB_PHASE_SEGMENT 7    /* per knot group and galaxy: spline segment and t (shared by the group's maps) */
 #define SFB_PHASE_MONOPOLE 8   /* mixed precision: FP64 monopole correction of the l = 0 maps */
 #define SFB_PHASE_ADJOINT 9    /* sfb_cat2amln_vjp(_device) after its catalogue stage */
@@ -297,7 +298,7 @@ int sfb_ang2pix_ring(int32_t device, int64_t nside, int64_t N, const double* the
 
 /* The delta map of map q (the (n,l) pair in map order) as the reference forms it
  * before map2alm (src/cat2anlm.jl:284-291), length npix: FP64 and bit-exact on an
- * SFB_PREC_FP64 plan; on the other precisions the FP32 map their scatter writes,
+ * SFB_PREC_FP64 plan; on the other precisions the FP32 map of the per-map scatter,
  * widened to double. */
 int sfb_delta_map(sfb_plan* p, int64_t N, const double* rtp, const double* w, double nbar,
                   int32_t win_kind, const double* win_a, const double* win_b, int64_t q,

@@ -457,7 +457,7 @@ __global__ __launch_bounds__(512) void k_phi_ifft_fold(const R* __restrict__ X, 
 }
 
 // Polar ring pairs, inverse: k_phi_ipolar4 with one sequence per map.  Bound: the direct length-i DFTs
-// (VALU) and their LDS reads (79% busy).  nside 128, 2514 maps, FP32: 505 us (unfolded 1.44 ms).
+// (VALU) and their LDS reads (79% busy).  nside 128, 2514 maps, FP32: 415 us (unfolded 1.44 ms).
 template <typename R>
 __global__ __launch_bounds__(256) void k_phi_ipolar4_fold(const R* __restrict__ X, int64_t npf, int32_t ncol, int64_t ld,
                                                           int32_t K, const RingDev* __restrict__ rings,
@@ -541,34 +541,15 @@ __global__ __launch_bounds__(256) void k_phi_ipolar4_fold(const R* __restrict__ 
     if (e >= TQ * njp) return;
     const int f = e / njp, jp = e - f * njp, c = c0 + f;
     if (c >= ncol) return;
-    const int j0 = 2 * jp, j1 = j0 + 1;
-    const R2* vf = V + f * 4 * nu;
-    R acc[2][4];
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int ss = 0; ss < 4; ++ss) acc[a][ss] = 0;
-    int i0 = 0, i1 = 0;
-    for (int u = 0; u < nu; ++u) {
-        const R2 w0 = twi[i0], w1 = twi[i1];
-#pragma unroll
-        for (int ss = 0; ss < 4; ++ss) {
-            const R2 v = vf[ss * nu + u];
-            acc[0][ss] = fma(v.x, w0.x, fma(-v.y, w0.y, acc[0][ss]));
-            acc[1][ss] = fma(v.x, w1.x, fma(-v.y, w1.y, acc[1][ss]));
-        }
-        i0 += j0;
-        if (i0 >= ni) i0 -= ni;
-        i1 += j1;
-        if (i1 >= ni) i1 -= ni;
-    }
+    R y0[4], y1[4];
+    const int j1 = ip4_outputs<R>(V + f * 4 * nu, twi, ni, nu, jp, y0, y1);
     const R sc = (R)scale;
     R* o = out + (int64_t)cols[c].q * npf + Rg.start_n;
 #pragma unroll
-    for (int ss = 0; ss < 4; ++ss) o[4 * j0 + ss] = sc * acc[0][ss];
-    if (j1 < ni)
+    for (int ss = 0; ss < 4; ++ss) o[4 * jp + ss] = sc * y0[ss];
+    if (j1 >= 0)
 #pragma unroll
-        for (int ss = 0; ss < 4; ++ss) o[4 * j1 + ss] = sc * acc[1][ss];
+        for (int ss = 0; ss < 4; ++ss) o[4 * j1 + ss] = sc * y1[ss];
 }
 
 // Per galaxy and map range blockIdx.y (`step` runs of whole knot groups): part = (sum_q g_q(r) dbar_q,

@@ -36,7 +36,8 @@ __device__ __forceinline__ double rcp64(double d)
 // boundary extrapolation), NaN passes through.
 // Bound: the tile's HBM write (npix nc 8 B, once) and the latency of a block's phases, hence
 // small blocks, four to a CU (32 pixels, 256 threads and tabulated reciprocals, two blocks to a
-// CU, ran 121 us at N = 1e6, nside 128, nc 159 and 1025 us at 4e6, nside 256, nc 219).
+// CU, ran 121 us at N = 1e6, nside 128, nc 159 and 1025 us at 4e6, nside 256, nc 219; now 109
+// and 515 us, 2.3 and 2.7 TB/s of the maps' write).
 __global__ __launch_bounds__(SH_NT) void k_shell_spread(int64_t npix, int32_t nc, const double* __restrict__ knots,
                                                         const int32_t* __restrict__ pstart,
                                                         const double* __restrict__ r_s, const double* __restrict__ w_s,
@@ -111,7 +112,8 @@ __global__ __launch_bounds__(SH_NT) void k_shell_spread(int64_t npix, int32_t nc
 // exact spline sums sum_i w_i g_n0(r_i), FP64.  A block takes two n and one share of the galaxies:
 // their (y, y'') at the knots in LDS, the segment from the uniform knots (the scatter's rule;
 // shells only exist on such knots).  Bound by r and w from L2, once per pair of n, and the two
-// random 16-byte reads per value (one n per block and 32-byte records: 482 us at 4e6, 48 n).
+// random 16-byte reads per value (LDS 68% busy).  352 us at 4e6, 48 n (one n per block and 32-byte
+// records: 482 us).
 constexpr int SM_N = 2, SM_U = 4;
 __global__ __launch_bounds__(1024) void k_shell_mono(int64_t N, int32_t nmx, const double* __restrict__ r,
                                                      const double* __restrict__ w, const MapInfo* __restrict__ maps,
@@ -179,7 +181,7 @@ __global__ __launch_bounds__(1024) void k_shell_mono(int64_t N, int32_t nmx, con
 // coefficients of the shell maps (a layout, row stride ld, shell s at 2 s).  A block takes one
 // l and SC_M values of m: their Z rows stay in LDS, and 32 lanes take the maps of this l (lq,
 // cnt of them from l0) over gamma by shell, gt[l0 nc + s cnt + j].  A few MB and 0.1 GFLOP:
-// latency-bound.  The monopoles (l = 0: a wave per map) add c00 inv (exact sum - sum_s gamma_s
+// latency-bound, 35 us at nside 128 (159 shells, 116 345 coefficients), 112 us at nside 256.  The monopoles (l = 0: a wave per map) add c00 inv (exact sum - sum_s gamma_s
 // T_s), T_s = sum_p D_s(p) (at tsum[2 s]): the refinements pass an error of the first
 // analysis' monopole to a_00 one to one.
 constexpr int SC_M = 8;

@@ -28,7 +28,9 @@ struct RowGemm {
     int32_t col0, ncol;
 };
 
-// The GEMM of k_gemm_tall<FP64> on RowGemm batches (load-bound like it: 3 waves per SIMD).
+// The GEMM of k_gemm_tall<FP64> on RowGemm batches (load-bound like it: 3 waves per SIMD).  One call with
+// the folded table takes the place of the analysis and 2 niter refinement products.  159 shells, nside 128:
+// 64 us; 219 shells, nside 256: 287 us.
 __global__ __launch_bounds__(256, 3) void k_gemm_rows(const RowGemm* __restrict__ descs, int32_t cols,
                                                       const double* __restrict__ A, int64_t lda, double* C0,
                                                       int64_t ldc0, double* C1, int64_t ldc1, double alpha, double beta)
@@ -103,7 +105,7 @@ struct AliasTerm {
 // stay in LDS over the J steps, with the states and couplings beside them, so that after one round
 // of loads only the Q rows come from L2.  What bounds it is the chain of 2 J dependent phases
 // over a few hundred states, not bytes (states, couplings and h read phase by phase: 115 us for
-// 5028 columns and 441 states, 28 us for 320 columns).
+// 5028 columns and 441 states, 28 us for 320 columns; now 78 and 20 us).
 __host__ __device__ inline size_t alias_lds(int32_t S, int32_t J, int32_t CT, int32_t nterm)
 {
     return sizeof(double) * (size_t)(J + 1) * (size_t)S * (size_t)CT + sizeof(AliasTerm) * (size_t)nterm +
