@@ -457,7 +457,7 @@ __global__ __launch_bounds__(512) void k_phi_ifft_fold(const R* __restrict__ X, 
 }
 
 // Polar ring pairs, inverse: k_phi_ipolar4 with one sequence per map.  Bound: the direct length-i DFTs
-// (VALU) and their LDS reads (79% busy).  nside 128, 2514 maps, FP32: 415 us (unfolded 1.44 ms).
+// (VALU) and their LDS reads (79% busy).  nside 128, 2514 maps, FP32: 345 us (unfolded 1.44 ms).
 template <typename R>
 __global__ __launch_bounds__(256) void k_phi_ipolar4_fold(const R* __restrict__ X, int64_t npf, int32_t ncol, int64_t ld,
                                                           int32_t K, const RingDev* __restrict__ rings,
@@ -516,25 +516,9 @@ __global__ __launch_bounds__(256) void k_phi_ipolar4_fold(const R* __restrict__ 
         }
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < TQ * 4 * nu; e += blockDim.x) {
-        const int f = e / (4 * nu), rr = e - f * 4 * nu;
-        const int ss = rr / nu, u = rr - ss * nu;
-        const R2* xf = Xb + f * npr;
-        R vr = 0, vi = 0;
-#pragma unroll
-        for (int t = 0; t < 4; ++t) {
-            const int bb = u + t * ni;
-            const R2 x = xf[bb];
-            const double2 w64 = twl[((unsigned)(2 * bb) * (unsigned)ss) % (unsigned)n2];
-            const R wx = (R)w64.x, wy = (R)w64.y;
-            vr += x.x * wx - x.y * wy;
-            vi += x.x * wy + x.y * wx;
-        }
-        const R hv = (u == 0 || 2 * u == ni) ? (R)0.5 : (R)1;
-        R2 v;
-        v.x = hv * vr;
-        v.y = hv * vi;
-        V[e] = v;
+    for (int e = threadIdx.x; e < TQ * nu; e += blockDim.x) {
+        const int f = e / nu, u = e - f * nu;
+        ip4_radix<R>(Xb + f * npr, twl, ni, nu, u, V + f * 4 * nu);
     }
     __syncthreads();
     const int e = threadIdx.x;
