@@ -5022,8 +5022,9 @@ extern "C" int sfb_cat2amln_vjp_device(sfb_plan* P, int64_t N, const double* d_r
     const bool fold = P->fold.ok && P->seg_uniform && grouped && (int64_t)one + 512 <= P->lds_max &&
                       (P->precision == SFB_PREC_FP64 || P->precision == SFB_PREC_MIXED);
     // radius bins: a bin's records of a map take at most VF_BIN bytes of LDS
-    // (no more counters than 4 N: they are cleared and scanned)
-    const int64_t bmax = std::min<int64_t>(16, 4 * N / std::max<int64_t>(1, P->fold.npf));
+    // (no more counters than 4 N: they are cleared and scanned; bin and folded pixel in 31 bits)
+    const int64_t npf1 = std::max<int64_t>(1, P->fold.npf);
+    const int64_t bmax = std::min<int64_t>({16, 4 * N / npf1, 0x7fffffff / (2 * npf1)});
     const int32_t nbin =
         fold ? (int32_t)std::max<int64_t>(1, std::min<int64_t>(bmax, nblk((int64_t)one, VF_BIN))) : 1;
     if ((rc = catalog_stage(P, N, d_rtp, d_w, st, CAT_ANY, false, fold, nbin))) return rc;
