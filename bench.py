@@ -45,11 +45,14 @@ import numpy as np  # noqa: E402
 METRIC = "cat2amln Mgal/s at N=1e6,kmax=0.1,nside=128: mixed vs FP64 GPU, max rel err"
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
-FP32_PEAK_TFLOPS = 157.3
 
-# phase -> the kernel it brackets (the roofline is taken for single-kernel phases)
-PHASE_KERNEL = {"scatter": "k_scatter_it", "segment": "k_seg_t", "phi": "k_phi_fft", "phi_polar": "k_phi_polar4",
-                "analysis": "k_gemm_tall", "synthesis": "k_gemm_tall", "residual": "k_alias"}
+# phase -> the kernel it brackets (the roofline is taken for single-kernel phases): FP64 on folded
+# hemispheres, mixed on radial shells
+PHASE_KERNEL = {
+    "fp64": {"scatter": "k_scatter_it", "segment": "k_seg_t", "phi": "k_phi_fft_fold", "phi_polar": "k_phi_polar4_fold",
+             "analysis": "k_fold_rows"},
+    "mixed": {"scatter": "k_shell_spread", "phi": "k_phi_fft", "phi_polar": "k_phi_polar4", "analysis": "k_gemm_rows"},
+}
 
 
 def log(*a):
@@ -120,37 +123,53 @@ def errors(a, ref, am, qs=None):
             "worst_block_nl": [worst[1], worst[2]], "blocks": len(blk_max), "modes": int(rel.size)}
 
 
+def shell_count(am):
+    """Functions of the mixed path's radial basis (degree-9 B-splines on csrc/radial.cpp's breaks)."""
+    lo, hi = am.knot_x[am.knot_off[0]], am.knot_x[am.knot_off[1] - 1]
+    H = (hi - lo) / (float(np.diff(am.knot_off).max()) - 1.0)
+    half, n = 0.0, 0
+    while half < 0.5 * (hi - lo):
+        half += min(20.0 * H, max(0.5 * H, 0.3 * half))
+        n += 1
+    return 2 * n + 9
+
+
 def algorithmic_work(am, N, f32=False, ngroup=None):
-    """Per-launch algorithmic bytes / flops of each single-kernel phase (f32: the mixed path's
-    FP32 delta maps and ring coefficients)."""
+    """Per-launch algorithmic bytes / flops of each single-kernel phase: one FP64 map per (n, l), folded
+    onto one hemisphere, or (f32, the mixed path) one full-sky FP64 map per radial shell."""
     L, nside = am.lmax, am.nside
     npix, K, nmaps = 12 * nside * nside, 2 * nside, am.nmaps
-    M2 = 2 * nmaps
-    vb = 4 if f32 else 8
-    nlm_pairs = (L + 1) * (L + 2) // 2  # sum over (m, parity) of the l count
-    delta_bytes = nmaps * npix * vb
-    x_bytes = (L + 1) * 2 * K * M2 * vb
-    a_bytes = nlm_pairs * M2 * 8
-    # rings with 4 nside pixels: ring pairs nside-1 .. 2 nside-1 (2 nside + 1 rings)
-    k_eq0 = nside - 1
-    npix_eq = (2 * nside + 1) * 4 * nside
+    npix_eq = (2 * nside + 1) * 4 * nside  # rings with 4 nside pixels
+    k_eq0 = nside - 1                      # their ring pairs: nside-1 .. 2 nside-1
+    nlm_pairs = (L + 1) * (L + 2) // 2     # sum over (m, parity) of the l count
+    if f32:
+        ns = shell_count(am)
+        x_bytes = (L + 1) * 2 * K * 2 * ns * 8
+        x_eq = x_bytes * (K - k_eq0) // K
+        return {
+            # per galaxy r and w read, the shells' maps written once
+            "scatter": {"bytes": ns * npix * 8 + N * 16 + (npix + 1) * 4, "flops": 20.0 * N * 10},
+            "phi": {"bytes": ns * npix_eq * 8 + x_eq, "flops": 0.0},
+            "phi_polar": {"bytes": ns * (npix - npix_eq) * 8 + (x_bytes - x_eq), "flops": 0.0},
+            # a = X (folded table), N/S ring-pair symmetry: 2 flop x rows x K x sum n_b
+            "analysis": {"bytes": x_bytes + nlm_pairs * 2 * ns * 8, "flops": 2.0 * 2 * ns * K * nlm_pairs},
+        }
+    npf = 6 * nside * nside + 2 * nside    # northern and equatorial pixels
+    npf_eq = nside * 4 * nside + 4 * nside
+    # rows l only: per map and ring pair the coefficients m <= l of one parity pair
+    x_bytes = sum((2 * (l + 1)) * K * 8 * int(np.sum(am.lmax_n >= l)) for l in range(L + 1))
     x_eq = x_bytes * (K - k_eq0) // K
     if ngroup is None:
         ngroup = len({am.knot_x[am.knot_off[q]:am.knot_off[q + 1]].tobytes() for q in range(am.nmaps)})
     return {
-        # delta maps written once; per pixel its slice entry and window factor read once; per
-        # galaxy its radius read once (mixed path: segment and t found from it on the uniform
-        # knots) or its 16-bit segment and t (FP64 path)
-        "scatter": {"bytes": delta_bytes + N * (8 if f32 else 2 + vb) + (npix + 1) * 4 + npix * 8,
-                    "flops": 10.0 * N * nmaps},
+        # folded delta maps written once; per pixel its slice entry and window factors read once; per
+        # galaxy its 16-bit segment and t
+        "scatter": {"bytes": nmaps * npf * 8 + N * 10 + npf * 28, "flops": 10.0 * N * nmaps},
         # per knot group and galaxy: r read, (16-bit segment, t) written
-        "segment": {"bytes": ngroup * N * (8 + 2 + vb), "flops": 0.0},
-        "phi": {"bytes": nmaps * npix_eq * vb + x_eq, "flops": 0.0},
-        "phi_polar": {"bytes": nmaps * (npix - npix_eq) * vb + (x_bytes - x_eq), "flops": 0.0},
-        # a = dOmega * X Lambda with N/S ring-pair symmetry: 2 flop x rows x K x sum n_b
-        "analysis": {"bytes": x_bytes + a_bytes, "flops": 2.0 * M2 * K * nlm_pairs},
-        "synthesis": {"bytes": x_bytes + a_bytes, "flops": 2.0 * M2 * K * nlm_pairs},
-        "residual": {"bytes": 3 * x_bytes, "flops": 0.0},
+        "segment": {"bytes": ngroup * N * 18, "flops": 0.0},
+        "phi": {"bytes": nmaps * npf_eq * 8 + x_eq, "flops": 0.0},
+        "phi_polar": {"bytes": nmaps * (npf - npf_eq) * 8 + (x_bytes - x_eq), "flops": 0.0},
+        "analysis": {"bytes": x_bytes, "flops": x_bytes / 4.0},
     }
 
 
@@ -360,15 +379,15 @@ def main():
     dom = max(single, key=lambda k: single[k]["ms_per_launch"])
     w = work[dom]
     t_launch = ph[dom]["ms_per_launch"] * 1e-3
-    if dom in ("analysis", "synthesis"):
+    if dom == "analysis":
         achieved = w["flops"] / t_launch / 1e12
-        roof = {"bound": "mfma", "achieved": achieved, "peak": FP32_PEAK_TFLOPS, "unit": "TFLOP/s",
-                "frac": achieved / FP32_PEAK_TFLOPS, "traffic": None}
+        roof = {"bound": "mfma", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
+                "frac": achieved / FP64_PEAK_TFLOPS, "traffic": None}
     else:
         achieved = w["bytes"] / t_launch / 1e9
         roof = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": achieved / HBM_PEAK_GBS, "traffic": None}
-    roof.update({"kernel": PHASE_KERNEL.get(dom, dom), "phase": dom, "algorithmic_bytes_per_launch": w["bytes"],
+    roof.update({"kernel": PHASE_KERNEL[head].get(dom, dom), "phase": dom, "algorithmic_bytes_per_launch": w["bytes"],
                  "launch_ms": t_launch * 1e3})
     tpath = os.path.join(ROOT, "profiles", "hbm_traffic.json")
     if os.path.exists(tpath):
