@@ -29,6 +29,33 @@ struct RadBins {
     double r0, inv;    // bin = (r - r0) inv, clamped
 };
 
+// Arrival rank in a cell.  Atomics on one address take 7 ns each, one after another, so where
+// several lanes of a wavefront share a cell (a crowded or an ordered catalogue; four lanes are
+// tried) one lane adds for all of its cell.
+__device__ __forceinline__ uint32_t arrival_rank(int32_t* __restrict__ cnt, uint32_t cell)
+{
+    const uint64_t live = __ballot(1);
+    const int lane = threadIdx.x & 63, nl = __popcll(live);  // lanes 0 .. nl - 1
+    bool shared = false;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cell, (j * nl) >> 2);
+        shared |= __popcll(__ballot(cell == c)) > 1;
+    }
+    if (!shared) return (uint32_t)atomicAdd(cnt + cell, 1);
+    uint64_t mine = 0;
+    for (uint64_t todo = live; todo;) {
+        const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)cell, __ffsll((unsigned long long)todo) - 1);
+        const uint64_t same = __ballot(cell == c);
+        if (cell == c) mine = same;
+        todo &= ~same;
+    }
+    const int lead = __ffsll((unsigned long long)mine) - 1;
+    int32_t base = 0;
+    if (lane == lead) base = atomicAdd(cnt + cell, (int32_t)__popcll(mine));
+    return (uint32_t)(__shfl(base, lead, 64) + (int32_t)__popcll(mine & ((1ull << lane) - 1)));
+}
+
 // pixel (FOLD: folded, with the hemisphere in bit 0) and arrival rank of every galaxy.
 // flag[1] |= 1 when an angle is not finite (the reference's floor(Int, NaN) throws).
 template <bool FOLD>
@@ -48,7 +75,7 @@ __global__ __launch_bounds__(256) void k_count(int64_t N, const double* __restri
     }
     uint32_t f = FOLD ? fold_pixel(p, nside) : (uint32_t)p;
     if (FOLD && rb.n > 1) f += rb.np2 * (uint32_t)fmin(fmax((rtp[3 * i] - rb.r0) * rb.inv, 0.0), (double)(rb.n - 1));
-    pr[i] = make_uint2(f, (uint32_t)atomicAdd(cnt + (FOLD ? f >> 1 : f), 1));
+    pr[i] = make_uint2(f, arrival_rank(cnt, FOLD ? f >> 1 : f));
 }
 
 // per PS_CHUNK pixels: their galaxies, and the crowding flag
