@@ -151,8 +151,9 @@ int sfb_cat2amln_batch_device(sfb_plan* p, int32_t B, const int64_t* N_b, const 
  * batch entry points capture the whole batch into a graph and launch it, and replay that
  * graph when a later batch call repeats the same sizes, n-bar values, pointers, window kind
  * and precision (no plan buffer reallocated since).  Before a capture the largest mock runs
- * once eagerly so that no buffer grows under capture.  enable = 0 enqueues the mocks
- * directly (the default); enable < 0 leaves the setting.  *capture_ms (if not NULL)
+ * once eagerly so that no buffer grows under capture.  A batch with a mock large enough for
+ * the radix sorts (96 galaxies per pixel on average, in FP64 1024 per folded pixel) is enqueued
+ * directly.  enable = 0 enqueues the mocks directly (the default); enable < 0 leaves the setting.  *capture_ms (if not NULL)
  * receives the wall time of the last capture and instantiation. */
 int sfb_plan_set_batch_graph(sfb_plan* p, int32_t enable, double* capture_ms);
 

@@ -4,13 +4,22 @@
 // dispatches where two stable radix sorts took forty: the catalogue stage of a small call is
 // launch-bound (1e5 galaxies at nside 32: ~49 dispatches of 3-7 us each).
 //
-// The rank pass compares a pixel's galaxies pairwise, so it is for pixels of up to PS_CROWD
-// galaxies; a fuller one raises flag[2] bit 1 and the call is redone with the radix sorts
-// (which the plan then keeps).
+// The rank pass compares a pixel's galaxies pairwise.  A catalogue with many galaxies in every
+// pixel takes stable radix sorts instead (known from its size); a few crowded pixels
+// do not: their rank costs less than the sum over a pixel's galaxies in order that follows it, up
+// to PS_CROWD galaxies.  A pixel beyond raises flag[2] bit 1 and the call is redone with the
+// radix sorts.
 #pragma once
 
-constexpr int PS_CROWD = 512;     // galaxies per pixel the pairwise rank takes
-constexpr int PS_MEAN = 96;       // mean galaxies per pixel above which the radix sorts run at once
+// Mean galaxies per pixel above which the radix sorts run.  FP64 (by pixel and r, two sorts): at
+// nside 16 the call takes 684 us with counting kernels against 795 with the sorts at 768 per folded
+// pixel, 1310 against 1256 at 1536; nside 32 2765 / 3061 at 768.  Mixed (one sort, by pixel): 456 us
+// either way at 96, nside 32; 198 / 222 at 48 and 460 / 525 at 144, nside 16; 340 / 332 at 24 and
+// 1084 / 949 at 96, nside 64.
+constexpr int PS_MEAN_R = 1024, PS_MEAN = 96;
+constexpr int PS_CROWD = 1 << 20; // galaxies of one pixel that the rank takes
+constexpr int PS_WALK = 64;       // galaxies of a pixel up to which each lane walks them (call at 96 per
+                                  // pixel, nside 32 FP64: 478 us; 128: 550, 256: 534)
 constexpr int PS_CHUNK = 2048;    // pixels per scan block
 constexpr int PS_SMALL = 32;      // scan blocks up to which each adds up the counts before it itself
 
@@ -168,10 +177,39 @@ __global__ __launch_bounds__(256) void k_place(int64_t N, const uint2* __restric
     slot[(int64_t)pstart[q.x >> sh] + q.y] = c;
 }
 
+// Orders a wavefront's LDS accesses (its lanes run in step; only the compiler may reorder).
+__device__ __forceinline__ void wave_lds_sync()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Sort key of a galaxy inside its pixel, northern ones first: ORDER 1 the input index, 2 r and
+// the input index (31 bits).  No galaxy's key is the largest value.
+struct RankKey {
+    uint64_t a;
+    uint32_t b;
+};
+template <int ORDER> __device__ __forceinline__ RankKey rank_key(const CatSlot& c)
+{
+    const uint64_t south = (uint64_t)(c.pix & 1u) << 63;
+    if (ORDER == 1) return {south | c.i, 0};
+    const uint64_t k = sortable_bits(c.r);
+    return {south | k >> 1, (uint32_t)(k & 1) << 31 | c.i};
+}
+__device__ __forceinline__ bool rank_less(const RankKey& x, const RankKey& y)
+{
+    return (x.a < y.a) | ((x.a == y.a) & (x.b < y.b));
+}
+
 // order inside a pixel: 0 as placed (where any order does), 1 by input index, 2 by (r, input
 // index), the order of the reference's sums; in a folded pixel northern galaxies first, as the
 // radix sorts leave them.  Writes the sorted list of input indices, and
 // pixel, r and w in that order.
+// Bound: the scattered 32-byte writes while pixels hold a few galaxies: each lane walks its own
+// pixel's.  A wavefront that meets a crowded pixel takes its pixels one after another: its own
+// galaxies of the pixel, sorted, stay in LDS, every other galaxy finds its place among them (seven
+// LDS reads, 64 galaxies at a time), and a galaxy's rank is the sum of the places up to its own.
 template <int ORDER>
 __global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restrict__ slot,
                                               const int32_t* __restrict__ pstart, int32_t sh,
@@ -179,15 +217,16 @@ __global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restri
                                               uint32_t* __restrict__ pix_s, double* __restrict__ r_s,
                                               double* __restrict__ w_s)
 {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= N) return;
+    __shared__ uint64_t own_a[4][64];
+    __shared__ uint32_t own_b[4][64], hist[4][64];
+    const int64_t e0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, e = min(e0, N - 1);
     const CatSlot me = slot[e];
     int64_t f = e;
     if (ORDER) {
         const int32_t s0 = pstart[me.pix >> sh], s1 = pstart[(me.pix >> sh) + 1];
-        if (s1 - s0 <= PS_CROWD) {  // (fuller: the call is redone)
+        int32_t before = 0;
+        if (__ballot(s1 - s0 > PS_WALK) == 0) {
             const uint64_t k = sortable_bits(me.r);
-            int32_t before = 0;
             for (int32_t s = s0; s < s1; ++s) {
                 const uint32_t i = slot[s].i, ps = slot[s].pix;
                 if (ORDER == 2) {
@@ -197,9 +236,57 @@ __global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restri
                     before += ps < me.pix || (ps == me.pix && i < me.i);
                 }
             }
-            f = (int64_t)s0 + before;
+        } else {  // (every lane is here, those past the end without a galaxy)
+            const RankKey k = rank_key<ORDER>(me);
+            const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+            for (uint64_t todo = __ballot(e0 < N); todo;) {
+                const int l = __ffsll((unsigned long long)todo) - 1;
+                const int32_t u0 = __builtin_amdgcn_readlane(s0, l), u1 = __builtin_amdgcn_readlane(s1, l);
+                const uint64_t group = __ballot(s0 == u0 && e0 < N);
+                todo &= ~group;
+                if (u1 - u0 > PS_CROWD) continue;
+                int p = 0;  // place among the wavefront's galaxies of this pixel
+                for (uint64_t m = group; m; m &= m - 1) {
+                    const int j = __ffsll((unsigned long long)m) - 1;
+                    const RankKey o{(uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(k.a >> 32), j) << 32 |
+                                        (uint32_t)__builtin_amdgcn_readlane((int)k.a, j),
+                                    (uint32_t)__builtin_amdgcn_readlane((int)k.b, j)};
+                    p += rank_less(o, k);
+                }
+                own_a[wv][lane] = ~0ull;
+                own_b[wv][lane] = ~0u;
+                hist[wv][lane] = 0;
+                wave_lds_sync();
+                if (group >> lane & 1) {
+                    own_a[wv][p] = k.a;
+                    own_b[wv][p] = k.b;
+                }
+                wave_lds_sync();
+                CatSlot nx = slot[min(u0 + lane, u1 - 1)];
+                for (int32_t c = u0; c < u1; c += 64) {
+                    const RankKey o = rank_key<ORDER>(nx);
+                    nx = slot[min(c + 64 + lane, u1 - 1)];  // the next 64 in flight
+                    int at = 0;  // own galaxies up to o
+#pragma unroll
+                    for (int step = 32; step > 0; step >>= 1)
+                        at += rank_less(o, {own_a[wv][at + step - 1], own_b[wv][at + step - 1]}) ? 0 : step;
+                    at += !rank_less(o, {own_a[wv][at], own_b[wv][at]});
+                    if (c + lane < u1 && at < 64) atomicAdd(&hist[wv][at], 1u);
+                }
+                wave_lds_sync();
+                int32_t inc = (int32_t)hist[wv][lane];
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int32_t v = __shfl_up(inc, o, 64);
+                    if (lane >= o) inc += v;
+                }
+                inc = __shfl(inc, p, 64);
+                if (group >> lane & 1) before = inc;
+                wave_lds_sync();
+            }
         }
+        if (s1 - s0 <= PS_CROWD) f = (int64_t)s0 + before;  // (fuller: as placed, the call is redone)
     }
+    if (e0 >= N) return;
     idx[f] = me.i;
     pix_s[f] = me.pix;
     r_s[f] = me.r;

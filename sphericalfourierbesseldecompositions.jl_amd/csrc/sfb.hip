@@ -4,7 +4,7 @@
 // Pipeline of one call (all on one HIP stream):
 //   pixel_sort.h  ang2pix (ring scheme), counting sort by pixel and a fixed order inside each pixel
 //                 (the reference's summation order on the FP64 path, sortout, cat2anlm.jl:50-71); stable
-//                 rocprim radix sorts where a pixel is crowded; k_sell_*: sliced layout (one
+//                 rocprim radix sorts where every pixel is full; k_sell_*: sliced layout (one
 //                 wavefront lane per pixel)
 //   FP64, on maps folded onto one hemisphere (fold.h):
 //     k_seg_t       per knot group (maps with identical knots) and galaxy: spline segment i and
@@ -3139,8 +3139,8 @@ struct sfb_plan {
     int64_t sell_hint = 0;  // the exact slot total of a call that overflowed the bound
     DevBuf d_invperm, d_swidth, d_soff, d_sr, d_sw;
     DevBuf d_cnt;            // galaxies per pixel and per scan chunk
-    bool crowded = false;    // a catalogue crowded a pixel: group by radix sorts
     int64_t cat_np = 0;      // pixels of the last catalogue's grouping (npix, or npf folded)
+    bool radix_next = false; // a pixel was too full for the rank: the redone call takes the radix sorts
     bool cat_fold = false;   // ... with southern pixels folded onto northern ones
     DevBuf d_ss;             // folded sliced layout: 1 where a slot's galaxy is southern
     const uint32_t* cat_idx = nullptr;  // the last catalogue's input indices, by pixel
@@ -3946,6 +3946,19 @@ static int64_t sell_bound(const sfb_plan* P, int64_t N, int64_t np)
     return std::max<int64_t>(N + 64 * nwin * cmax, P->sell_hint);
 }
 
+// The grouping of a catalogue over np pixels: counting kernels, or the radix sorts.
+static bool groups_by_count(int64_t N, int64_t np, CatOrder order)
+{
+    return order == CAT_ANY || N <= (order == CAT_RADIUS ? PS_MEAN_R : PS_MEAN) * np;
+}
+
+// Scratch that only the counting kernels use.
+static int count_scratch(sfb_plan* P, int64_t N, int64_t ncell)
+{
+    int rc = P->d_cnt.ensure(sizeof(int32_t) * ((size_t)ncell + nblk(ncell, PS_CHUNK)));
+    return rc ? rc : P->d_sorttmp.ensure(sizeof(CatSlot) * (size_t)N);
+}
+
 // Groups the catalogue by pixel: cat_idx, pstart, and pixel, r and w in that order; slots: also
 // the sliced layout sr, sw (soff, pinfo) when the records fit in LDS (the per-map scatter reads
 // it; the shells' spread and the adjoint's gather do not).  fold: by folded pixel (fold_pixel).
@@ -3981,11 +3994,11 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         (rc = P->d_rs.ensure(8 * n)) || (rc = P->d_ws.ensure(8 * n)) || (rc = P->d_pixkey2.ensure(4 * n)))
         return rc;
     PhaseTimer timer(P, SFB_PHASE_CATALOG, st);
-    if (!P->crowded && N <= PS_MEAN * np) {
+    const bool radix = !groups_by_count(N, np, order) || (P->radix_next && order != CAT_ANY);
+    if (order != CAT_ANY) P->radix_next = false;
+    if (!radix) {
         const unsigned nb = nblk(ncell, PS_CHUNK);
-        if ((rc = P->d_cnt.ensure(sizeof(int32_t) * ((size_t)ncell + nb))) ||
-            (rc = P->d_sorttmp.ensure(sizeof(CatSlot) * n)))
-            return rc;
+        if ((rc = count_scratch(P, N, ncell))) return rc;
         int32_t* cnt = P->d_cnt.as<int32_t>();
         int32_t* sums = cnt + ncell;
         hipLaunchKernelGGL(k_zero_counts, dim3(nblk(ncell, 256)), dim3(256), 0, st, ncell, cnt,
@@ -4020,7 +4033,7 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         if (rc) return rc;
         P->cat_idx = P->d_idx.as<uint32_t>();
     } else {
-        // crowded pixels: stable radix sorts, by r (CAT_RADIUS) and by pixel
+        // many galaxies in every pixel: stable radix sorts, by r (CAT_RADIUS) and by pixel
         if ((rc = P->d_keyr2.ensure(8 * n)) || (rc = P->d_idx2.ensure(4 * n)) || (rc = P->d_pix.ensure(4 * n)) || (rc = P->d_pixkey.ensure(4 * n)))
             return rc;
         hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, P->d_flag.as<int32_t>(), 4, 0);
@@ -4744,10 +4757,10 @@ static int check_window(const sfb_plan* P, int32_t win_kind, const double* wa, c
 
 // After a call whose sliced layout overflowed its capacity (flag[2] bit 0): the exact slot
 // total becomes the plan's capacity hint (it only grows), for the call to be redone.  Bit 1: a
-// pixel too full for the pairwise rank; the plan groups by radix sorts from then on.
+// pixel too full for the pairwise rank; the redone call takes the radix sorts.
 static int take_slot_total(sfb_plan* P, int32_t over)
 {
-    if (over & 2) P->crowded = true;
+    if (over & 2) P->radix_next = true;
     if (!(over & 1)) return SFB_OK;
     int64_t T = 0;
     HIP_TRY(hipMemcpy(&T, P->d_soff.as<int64_t>() + P->sell_nslice, sizeof(int64_t), hipMemcpyDeviceToHost));
@@ -4808,6 +4821,30 @@ static int monopole_fix(sfb_plan* P, int64_t N, double nbar, int32_t win_kind, c
 #include "fold.h"
 #include "shells.h"
 
+// How a cat2amln call of N galaxies runs: over the radial shells, with FP32 maps, on folded
+// hemispheres, and over how many pixels its catalogue is grouped.
+struct CatRoute {
+    bool shells, f32, fold;
+    int64_t np;
+    CatOrder order() const { return shells || f32 ? CAT_INPUT : CAT_RADIUS; }
+};
+static CatRoute cat_route(const sfb_plan* P, int64_t N, int32_t win_kind)
+{
+    CatRoute c{false, false, false, P->npix};
+    // mixed path on the plan's radial basis.  It needs a window that is one map times w_ln (a
+    // dense one has a map per (n, l) anyway); the split-BF16 precisions keep the per-map
+    // pipeline, whose Jacobi products they select.
+    c.shells = P->precision == SFB_PREC_MIXED && P->shells.ok && win_kind == SFB_WIN_SEPARABLE;
+    // else FP32 spline values and delta maps, FP32 MFMA for the Jacobi passes
+    size_t shp4;
+    c.f32 = !c.shells && P->precision != SFB_PREC_FP64 && polar4_fits(P, sizeof(float), &shp4);
+    // FP64: folded hemispheres when the sliced scatter takes the catalogue (an empty one, or one
+    // beyond its 32-bit slots, goes the unfolded way)
+    c.fold = !c.shells && !c.f32 && P->fold.ok && N > 0 && sell_bound(P, N, P->fold.npf) < SELL_MAX;
+    if (c.fold) c.np = P->fold.npf;
+    return c;
+}
+
 // One cat2amln enqueued on stream st with no host synchronisation: its flags (non-finite
 // a_nlm, non-finite angle, slot overflow) are left in d_flag[0..2].
 static int cat2amln_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const double* d_w, double nbar,
@@ -4815,18 +4852,10 @@ static int cat2amln_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const d
                             hipStream_t st)
 {
     int rc;
-    // mixed path on the plan's radial basis.  It needs a window that is one map times w_ln (a
-    // dense one has a map per (n, l) anyway); the split-BF16 precisions keep the per-map
-    // pipeline, whose Jacobi products they select.
-    if (P->precision == SFB_PREC_MIXED && P->shells.ok && win_kind == SFB_WIN_SEPARABLE)
-        return shells_enqueue(P, N, d_rtp, d_w, nbar, d_win_a, d_win_b, d_out, st);
-    // else FP32 spline values and delta maps, FP32 MFMA for the Jacobi passes
-    size_t shp4;
-    const bool f32 = P->precision != SFB_PREC_FP64 && polar4_fits(P, sizeof(float), &shp4);
-    // FP64: folded hemispheres when the sliced scatter takes the catalogue (an empty one, or one
-    // beyond its 32-bit slots, goes the unfolded way)
-    const bool fold = !f32 && P->fold.ok && N > 0 && sell_bound(P, N, P->fold.npf) < SELL_MAX;
-    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, f32 ? CAT_INPUT : CAT_RADIUS, true, fold))) return rc;
+    const CatRoute route = cat_route(P, N, win_kind);
+    const bool f32 = route.f32, fold = route.fold;
+    if (route.shells) return shells_enqueue(P, N, d_rtp, d_w, nbar, d_win_a, d_win_b, d_out, st);
+    if ((rc = catalog_stage(P, N, d_rtp, d_w, st, route.order(), true, fold))) return rc;
     if ((rc = scatter_stage(P, nbar, win_kind, d_win_a, d_win_b, st, f32))) return rc;
     if (fold) return fold_analysis(P, d_out, st);
     if ((rc = sht_stage(P, (int32_t)P->nmaps, st, f32))) return rc;
@@ -5221,11 +5250,22 @@ extern "C" int sfb_cat2amln_batch_device(sfb_plan* P, int32_t B, const int64_t* 
     // Every mock is enqueued back to back with no host synchronisation; each leaves its flags
     // in d_bflag and the host reads them all once at the end.  The largest catalogue goes
     // first so that its call grows every work buffer to the batch's largest size while the
-    // stream is otherwise idle; later calls reuse them (no allocation behind queued work).
+    // stream is otherwise idle; later calls reuse them (no allocation behind queued work).  Where
+    // it takes the radix sorts and smaller ones the counting kernels, the scratch of those is
+    // laid out for the largest of them before anything is enqueued.
     std::vector<int32_t> order((size_t)B);
     for (int32_t b = 0; b < B; ++b) order[(size_t)b] = b;
     std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return N_b[x] > N_b[y]; });
     if ((rc = P->d_bflag.ensure(sizeof(int32_t) * 4 * (size_t)B))) return rc;
+    bool radix = false, counted = false;
+    for (int32_t ib = 0; ib < B && !counted; ++ib) {
+        const int64_t n = N_b[order[(size_t)ib]];
+        if (n == 0) break;
+        const CatRoute route = cat_route(P, n, win_kind);
+        counted = groups_by_count(n, route.np, route.order());
+        radix = radix || !counted;
+        if (counted && radix && (rc = count_scratch(P, n, route.np))) return rc;
+    }
     auto enqueue_all = [&]() -> int {
         for (int32_t ib = 0; ib < B; ++ib) {
             const int32_t b = order[(size_t)ib];
@@ -5243,7 +5283,8 @@ extern "C" int sfb_cat2amln_batch_device(sfb_plan* P, int32_t B, const int64_t* 
         }
         return SFB_OK;
     };
-    if (!P->batch_graph) {
+    if (!P->batch_graph || radix) {
+        // (the radix sorts clear their histograms with memsets, which stay out of a graph)
         if ((rc = enqueue_all())) return rc;
     } else {
         // One HIP graph for the whole batch: replayed when the call repeats the previous one
@@ -5311,6 +5352,7 @@ extern "C" int sfb_cat2amln_batch_device(sfb_plan* P, int32_t B, const int64_t* 
         if (f[1]) return fail(SFB_ERR_ARG, "catalogue %d: InexactError: a galaxy angle (theta or phi) is not finite", b);
         if (f[2]) {  // a crowded mock outgrew the slot bound: redone alone with exact sizes
             const int64_t n = N_b[b];
+            if (f[2] & 2) P->radix_next = true;
             if ((rc = sfb_cat2amln_device(P, n, n ? d_rtp + 3 * off[(size_t)b] : nullptr,
                                           (d_w && n) ? d_w + off[(size_t)b] : nullptr, nbar_b[b], win_kind, d_win_a,
                                           d_win_b, d_out + (int64_t)b * 2 * P->nlmsize, stream))) {
