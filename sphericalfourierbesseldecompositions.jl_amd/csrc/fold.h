@@ -12,7 +12,8 @@ static int fold_tables(sfb_plan* P)
     Fold& F = P->fold;
     const DirectSht& D = P->dir;
     F.ok = false;
-    if (!D.ok || !P->sell_ok) return SFB_OK;
+    // (a slot's radius carries the hemisphere in its sign: k_sell_fill)
+    if (!D.ok || !P->sell_ok || !(P->r_first >= 0.0)) return SFB_OK;
     const int64_t L = P->lmax, nside = P->nside;
     F.npf = 6 * nside * nside + 2 * nside;
     // launch shapes: three FFT blocks per CU while they hold more than one map

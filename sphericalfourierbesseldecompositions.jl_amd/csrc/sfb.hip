@@ -415,7 +415,7 @@ __global__ __launch_bounds__(1024) void k_scan_i64(int32_t n, const int64_t* __r
 __global__ void k_sell_fill(int64_t N, const uint32_t* __restrict__ pix_s, const int32_t* __restrict__ pstart,
                             const uint32_t* __restrict__ invperm, const int64_t* __restrict__ soff,
                             const double* __restrict__ r_s, const double* __restrict__ w_s, double* __restrict__ sr,
-                            double* __restrict__ sw, int64_t tcap, int32_t sh, uint8_t* __restrict__ ss)
+                            double* __restrict__ sw, int64_t tcap, int32_t sh)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= N) return;
@@ -424,9 +424,12 @@ __global__ void k_sell_fill(int64_t N, const uint32_t* __restrict__ pix_s, const
     const uint32_t e = invperm[p];
     const int64_t dst = soff[e >> 6] + 64 * j + (e & 63);
     if (dst >= tcap) return;
-    sr[dst] = r_s[k];
+    double r = r_s[k];
+    // folded maps: the sign marks a southern galaxy (knots start at r >= 0, where a negative
+    // radius takes the same end value as 0; NaN stays NaN)
+    if (sh) r = copysign(r < 0.0 ? 0.0 : r, pix_s[k] & 1u ? -1.0 : 1.0);
+    sr[dst] = r;
     sw[dst] = w_s[k];
-    if (sh) ss[dst] = (uint8_t)(pix_s[k] & 1u);  // folded maps: a southern galaxy
 }
 
 // padding of the T = *Tdev slots (r = -inf, w = 0: they add an exact +-0 to every pixel
@@ -475,7 +478,7 @@ __global__ __launch_bounds__(1024) void k_seg_t(int64_t Tcap, const int64_t* __r
                                                const double* __restrict__ sr,
                                                const GroupInfo* __restrict__ groups, const double* __restrict__ gx,
                                                const double* __restrict__ grh, uint16_t* __restrict__ it_i,
-                                               TT* __restrict__ it_t, const uint8_t* __restrict__ ss)
+                                               TT* __restrict__ it_t, bool fold)
 {
     extern __shared__ double sm_seg[];
     const int64_t T = min(*Tdev, Tcap);
@@ -494,18 +497,16 @@ __global__ __launch_bounds__(1024) void k_seg_t(int64_t Tcap, const int64_t* __r
     TT* ot = it_t + (int64_t)g * Tcap;
     for (int64_t eb = e0 + threadIdx.x; eb < e1; eb += 4 * (int64_t)blockDim.x) {
         double rr[4];
-        bool south[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int64_t e = eb + u * (int64_t)blockDim.x;
             rr[u] = e < e1 ? sr[e] : 0.0;
-            south[u] = ss && e < e1 && (ss[e] & 1);
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
             const int64_t e = eb + u * (int64_t)blockDim.x;
             if (e >= e1) break;
-            const double r = rr[u];
+            const double r = fold ? fabs(rr[u]) : rr[u];
             int i;
             double t;
             if (r >= G.xfirst && r <= G.xlast) {
@@ -534,9 +535,9 @@ __global__ __launch_bounds__(1024) void k_seg_t(int64_t Tcap, const int64_t* __r
                 i = 0;
                 t = r;
             }
-            // folded maps: t's sign carries the hemisphere (t >= 0 otherwise, and the boundary
-            // records' slopes are 0)
-            if (ss) t = south[u] ? -fabs(t) : fabs(t);
+            // folded maps: t's sign carries the hemisphere, as the slot's radius does (t >= 0
+            // otherwise, and the boundary records' slopes are 0)
+            if (fold) t = copysign(t, rr[u]);
             oi[e] = (uint16_t)i;
             ot[e] = (TT)t;
         }
@@ -3142,7 +3143,6 @@ struct sfb_plan {
     int64_t cat_np = 0;      // pixels of the last catalogue's grouping (npix, or npf folded)
     bool radix_next = false; // a pixel was too full for the rank: the redone call takes the radix sorts
     bool cat_fold = false;   // ... with southern pixels folded onto northern ones
-    DevBuf d_ss;             // folded sliced layout: 1 where a slot's galaxy is southern
     const uint32_t* cat_idx = nullptr;  // the last catalogue's input indices, by pixel
     DevBuf d_smin;  // per slice: the smallest galaxy count of its lanes
     DevBuf d_pinfo, d_pwin;  // per slice lane: (pixel, count), separable window factor
@@ -3892,7 +3892,7 @@ extern "C" void sfb_plan_destroy(sfb_plan* P)
                       &P->d_pix, &P->d_pixkey, &P->d_pixkey2, &P->d_rs, &P->d_ws, &P->d_pstart, &P->d_sorttmp,
                       &P->h_rtp, &P->h_w, &P->h_wa, &P->h_wb, &P->h_out,
                       &P->d_desc_synf, &P->d_part, &P->h_cot, &P->h_dr, &P->h_dw,
-                      &P->d_cnt, &P->d_ss, &P->d_invperm, &P->d_swidth, &P->d_smin, &P->d_soff,
+                      &P->d_cnt, &P->d_invperm, &P->d_swidth, &P->d_smin, &P->d_soff,
                       &P->d_sr, &P->d_sw, &P->d_groups, &P->d_gx, &P->d_grh, &P->d_rec4, &P->d_qorder,
                       &P->d_it_i, &P->d_it_t, &P->d_sblk, &P->d_sblk32, &P->d_rec4f, &P->d_swf, &P->d_pinfo,
                       &P->d_pwin, &P->d_vgm, &P->d_vgs, &P->d_vrange, &P->d_lamw, &P->d_desc_cal,
@@ -4099,7 +4099,6 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         const int64_t tcap = sell_bound(P, N, np);
         P->sell_cap = tcap;
         P->sell_fits = tcap < SELL_MAX;
-        if (fold && (rc = P->d_ss.ensure((size_t)tcap))) return rc;
         if ((rc = P->d_sr.ensure(8 * (size_t)tcap)) || (rc = P->d_sw.ensure(8 * (size_t)tcap))) return rc;
         const int64_t* Tdev = P->d_soff.as<int64_t>() + P->sell_nslice;
         hipLaunchKernelGGL(k_sell_pad, dim3(nblk(tcap, 256)), dim3(256), 0, st, tcap, Tdev, P->d_sr.as<double>(),
@@ -4108,7 +4107,7 @@ static int catalog_stage(sfb_plan* P, int64_t N, const double* d_rtp, const doub
         hipLaunchKernelGGL(k_sell_fill, dim3(nblk(N, 256)), dim3(256), 0, st, N, P->d_pixkey2.as<uint32_t>(),
                            P->d_pstart.as<int32_t>(), P->d_invperm.as<uint32_t>(), P->d_soff.as<int64_t>(),
                            P->d_rs.as<double>(), P->d_ws.as<double>(), P->d_sr.as<double>(), P->d_sw.as<double>(),
-                           tcap, sh, P->d_ss.as<uint8_t>());
+                           tcap, sh);
         LAUNCH_CHECK();
     }
     return SFB_OK;
@@ -4287,12 +4286,11 @@ static int scatter_stage(sfb_plan* P, double nbar, int32_t win_kind, const doubl
             if (!onfly)
                 hipLaunchKernelGGL(k_seg_t<float>, gseg, dim3(1024), shm_seg, st, T, Tdev, P->d_sr.as<double>(),
                                    P->d_groups.as<GroupInfo>(), P->d_gx.as<double>(), P->d_grh.as<double>(),
-                                   P->d_it_i.as<uint16_t>(), P->d_it_t.as<float>(), (const uint8_t*)nullptr);
+                                   P->d_it_i.as<uint16_t>(), P->d_it_t.as<float>(), false);
         } else {
             hipLaunchKernelGGL(k_seg_t<double>, gseg, dim3(1024), shm_seg, st, T, Tdev, P->d_sr.as<double>(),
                                P->d_groups.as<GroupInfo>(), P->d_gx.as<double>(), P->d_grh.as<double>(),
-                               P->d_it_i.as<uint16_t>(), P->d_it_t.as<double>(),
-                               P->cat_fold ? P->d_ss.as<uint8_t>() : (const uint8_t*)nullptr);
+                               P->d_it_i.as<uint16_t>(), P->d_it_t.as<double>(), P->cat_fold);
         }
         LAUNCH_CHECK();
         tseg.end();
