@@ -3068,8 +3068,10 @@ struct Shells {
     bool ok = false;
     int32_t nc = 0;  // basis functions
     DevBuf d_knots, d_gamma, d_lstart, d_lq;  // gamma by l and shell; the maps of each l
+    DevBuf d_part;                            // the spread's maps by part
     void release()
     {
+        d_part.release();
         d_knots.release();
         d_gamma.release();
         d_lstart.release();

@@ -36,11 +36,18 @@ static int shells_tables(sfb_plan* P, const sfb::RadialBasis& R, bool fitted)
     return SFB_OK;
 }
 
+// Parts of the spread's galaxy runs: blocks of 512 galaxies at least, 12 blocks per CU at most.
+static int32_t shell_parts(int64_t N, int64_t npix)
+{
+    const int64_t nb = nblk(npix, SH_PT);
+    return (int32_t)std::max<int64_t>(1, std::min<int64_t>(3072 / nb, N / (512 * nb)));
+}
+
 // One mixed cat2amln over the shells, enqueued on st (separable window).
 static int shells_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const double* d_w, double nbar,
                           const double* d_mask, const double* d_wln, double* d_out, hipStream_t st)
 {
-    const Shells& S = P->shells;
+    Shells& S = P->shells;
     const int32_t nc = S.nc, nq = nc + 1;
     int rc;
     if ((rc = catalog_stage(P, N, d_rtp, d_w, st, CAT_INPUT, false))) return rc;
@@ -48,10 +55,19 @@ static int shells_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const dou
         PhaseTimer timer(P, SFB_PHASE_SCATTER, st);
         const size_t shm = sh_lds(nc);
         HIP_TRY(hipFuncSetAttribute((const void*)k_shell_spread, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
-        hipLaunchKernelGGL(k_shell_spread, dim3(nblk(P->npix, SH_PT)), dim3(SH_NT), shm, st, P->npix, nc,
-                           S.d_knots.as<double>(), P->d_pstart.as<int32_t>(), P->d_rs.as<double>(),
-                           P->d_ws.as<double>(), d_mask, P->d_delta.as<double>());
+        const int32_t parts = shell_parts(N, P->npix);
+        const int64_t n = (int64_t)nc * P->npix;
+        if (parts > 1 && (rc = S.d_part.ensure(sizeof(double) * (size_t)(parts * n)))) return rc;
+        double* D = P->d_delta.as<double>();
+        double* to = parts > 1 ? S.d_part.as<double>() : D;
+        hipLaunchKernelGGL(k_shell_spread, dim3(nblk(P->npix, SH_PT), (unsigned)parts), dim3(SH_NT), shm, st, P->npix,
+                           nc, S.d_knots.as<double>(), P->d_pstart.as<int32_t>(), P->d_rs.as<double>(),
+                           P->d_ws.as<double>(), d_mask, to, D + n);
         LAUNCH_CHECK();
+        if (parts > 1) {
+            hipLaunchKernelGGL(k_shell_sum, dim3(nblk(n, 256)), dim3(256), 0, st, n, parts, to, D);
+            LAUNCH_CHECK();
+        }
     }
     // the l = 0 maps' exact sums: about two blocks per CU over all n while their tables leave
     // room for two, whole blocks of galaxies each
