@@ -15,8 +15,9 @@
 // nside 16 the call takes 684 us with counting kernels against 795 with the sorts at 768 per folded
 // pixel, 1310 against 1256 at 1536; nside 32 2765 / 3061 at 768.  Mixed (one sort, by pixel): 456 us
 // either way at 96, nside 32; 198 / 222 at 48 and 460 / 525 at 144, nside 16; 340 / 332 at 24 and
-// 1084 / 949 at 96, nside 64.
-constexpr int PS_MEAN_R = 1024, PS_MEAN = 96;
+// 1084 / 949 at 96, nside 64.  Any order (adjoint, in radius bins): 463 us either way at 638, nside 16
+// mixed, 1315 / 828 at 2551 (the counters' atomics); 435 / 501 and 1450 / 1163 in FP64.
+constexpr int PS_MEAN_R = 1024, PS_MEAN = 96, PS_MEAN_ANY = 640;
 constexpr int PS_CROWD = 1 << 20; // galaxies of one pixel that the rank takes
 constexpr int PS_WALK = 64;       // galaxies of a pixel up to which each lane walks them (call at 96 per
                                   // pixel, nside 32 FP64: 478 us; 128: 550, 256: 534)

@@ -3951,7 +3951,7 @@ static int64_t sell_bound(const sfb_plan* P, int64_t N, int64_t np)
 // The grouping of a catalogue over np pixels: counting kernels, or the radix sorts.
 static bool groups_by_count(int64_t N, int64_t np, CatOrder order)
 {
-    return order == CAT_ANY || N <= (order == CAT_RADIUS ? PS_MEAN_R : PS_MEAN) * np;
+    return N <= (order == CAT_RADIUS ? PS_MEAN_R : (order == CAT_INPUT ? PS_MEAN : PS_MEAN_ANY)) * np;
 }
 
 // Scratch that only the counting kernels use.

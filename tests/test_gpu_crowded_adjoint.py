@@ -55,3 +55,23 @@ def test_time(precision):
         plan.profile(False)
     print("catalogue stage, whole sky and pencil beam, ms", precision, ms, flush=True)
     assert ms[1] < 4.0 * ms[0]
+
+
+@pytest.mark.parametrize("precision,tol", [("fp64", 1e-11), ("mixed", 3e-6)])
+@pytest.mark.parametrize("n", [28 * 640, 28 * 640 + 1])
+def test_dense_sky(n, precision, tol, monkeypatch):
+    """On either side of 640 galaxies per folded pixel (nside 2: 28): counting kernels in radius bins,
+    and the radix sort without bins."""
+    print("dense adjoint", n, precision, flush=True)
+    am = S.AnlmModes.from_nl(20, 8, 500.0, 1000.0, nside=2)
+    rng = np.random.default_rng(n)
+    cat = catalogue(n, *SKY, 3)
+    w = rng.uniform(0.5, 1.5, n)
+    monkeypatch.setenv("SFB_SEG_SEARCH", "1")
+    ref_plan = S.Plan(am, precision=precision)
+    monkeypatch.delenv("SFB_SEG_SEARCH")
+    plan = S.Plan(am, precision=precision)
+    c = rng.normal(size=plan.nlmsize) + 1j * rng.normal(size=plan.nlmsize)
+    got, ref = plan.cat2amln_vjp(cat, 1e-5, c, w), ref_plan.cat2amln_vjp(cat, 1e-5, c, w)
+    for g, r in zip(got[:2], ref[:2]):
+        assert np.max(np.abs(g - r)) <= tol * np.sqrt(np.mean(r ** 2))
