@@ -114,7 +114,9 @@ void sfb_plan_destroy(sfb_plan* p);
 /* Sizes the plan works with: number of maps, getnlmsize, npix. */
 int sfb_plan_sizes(const sfb_plan* p, int64_t* nmaps, int64_t* nlmsize, int64_t* npix);
 
-/* Switches the Legendre-step precision of an existing plan (SFB_PREC_*). */
+/* Switches the precision of an existing plan (SFB_PREC_*).  What a precision alone needs (the
+ * radial basis of SFB_PREC_MIXED, the FP32 tile search) is laid out at the first switch to it,
+ * or at creation; on an error the plan keeps the precision it had. */
 int sfb_plan_set_precision(sfb_plan* p, int32_t precision);
 
 /* cat2amln(rθϕ, amodes, nbar, win_rhat_ln, weight): src/cat2anlm.jl:257-310.
@@ -284,8 +286,9 @@ int sfb_plan_profile(sfb_plan* p, int32_t enable);
  * and the number of profiled calls since sfb_plan_profile. */
 int sfb_plan_phase_times(const sfb_plan* p, double* ms, int64_t* launches, int64_t* calls);
 
-/* The phi-transform tile shapes the plan's tile search chose at creation (no reference
- * counterpart; SFB_TUNE=0 in the environment skips the search and keeps the defaults):
+/* The phi-transform tile shapes the plan's tile search chose (at creation, for FP32 maps at the
+ * first use of another precision than FP64; no reference counterpart; SFB_TUNE=0 in the
+ * environment skips the search and keeps the defaults):
  * tiles[0..5] = maps per FFT block FP64, FFT threads per block FP64, the same two for FP32,
  * maps per polar block at the largest polar ring FP64, FP32 (fixed by the ring sizes, not
  * searched); *tune_ms = the search's wall time. */

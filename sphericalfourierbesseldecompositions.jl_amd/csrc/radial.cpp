@@ -49,7 +49,7 @@ void bspline(const std::vector<double>& t, int iv, double x, double* out)
 }  // namespace
 
 static bool fit(int64_t nmaps, const int64_t* off, const double* kx, const double* ky, const double* kypp,
-                RadialBasis* R)
+                RadialBasis* R, int threads)
 {
     if (nmaps < 1) return false;
     const double lo = kx[off[0]], hi = kx[off[1] - 1];
@@ -172,8 +172,7 @@ static bool fit(int64_t nmaps, const int64_t* off, const double* kx, const doubl
             }
         }
     };
-    const int nt = (int)std::min<int64_t>(std::max(1u, std::min(16u, std::thread::hardware_concurrency())),
-                                          1 + nmaps / 16);
+    const int nt = (int)std::min<int64_t>(std::max(1, threads), 1 + nmaps / 16);
     std::vector<std::thread> th;
     try {
         for (int i = 1; i < nt; ++i) th.emplace_back(work);
@@ -186,10 +185,10 @@ static bool fit(int64_t nmaps, const int64_t* off, const double* kx, const doubl
 }
 
 bool radial_basis(int64_t nmaps, const int64_t* off, const double* kx, const double* ky, const double* kypp,
-                  RadialBasis* R)
+                  RadialBasis* R, int threads)
 {
     try {
-        return fit(nmaps, off, kx, ky, kypp, R);
+        return fit(nmaps, off, kx, ky, kypp, R, threads);
     } catch (const std::bad_alloc&) {  // without the basis the plan keeps the per-map path
         return false;
     }

@@ -35,6 +35,7 @@
 #include <new>
 #include <string>
 #include <system_error>
+#include <thread>
 #include <vector>
 
 #include "sfb_internal.h"
@@ -3066,6 +3067,7 @@ struct Fold {
 // Device tables of the mixed path's radial basis (shells.h).
 struct Shells {
     bool ok = false;
+    bool tried = false;  // built, or found not to apply (plans that never run mixed have none)
     int32_t nc = 0;  // basis functions
     DevBuf d_knots, d_gamma, d_lstart, d_lq;  // gamma by l and shell; the maps of each l
     DevBuf d_part;                            // the spread's maps by part
@@ -3089,6 +3091,7 @@ struct sfb_plan {
     int32_t TQF = 1, TQF32 = 2, logM = 1;  // phi-transform FFT tiles (FP64 / FP32)
     int32_t fft_nt = 512, fft_nt32 = 256;           // FFT threads per block (FP64 / FP32)
     double tune_ms = 0.0;                           // time the plan-time tile search took
+    bool tuned[2] = {false, false};                 // ... done for FP64 / FP32 maps
     std::vector<MapInfo> maps;
     std::vector<int64_t> out_base, lam_off;
     std::vector<int64_t> aoff;  // per (m, parity): first row of its block in the a buffers (rows of M2 values)
@@ -3793,8 +3796,9 @@ static int plan_tables(sfb_plan* P, const int64_t* lmax_n, const int64_t* knot_o
 extern "C" const char* sfb_version(void) { return "sfb_mi355x 0.1 (gfx950)"; }
 
 static int shells_tables(sfb_plan* P, const sfb::RadialBasis& R, bool fitted);  // shells.h
+static int shells_build(sfb_plan* P);
 static int fold_tables(sfb_plan* P);    // fold.h
-static int autotune_phi(sfb_plan* P);  // plan-time phi-transform tile search (defined below)
+static int autotune_phi(sfb_plan* P, bool f32);  // plan-time phi-transform tile search (defined below)
 
 extern "C" int sfb_plan_create(sfb_plan** out, int64_t nside, int64_t lmax, int64_t nmax, const int64_t* lmax_n,
                                const int64_t* knot_off, const double* knot_x, const double* knot_y,
@@ -3861,19 +3865,27 @@ extern "C" int sfb_plan_create(sfb_plan** out, int64_t nside, int64_t lmax, int6
         delete P;
         return fail(SFB_ERR_DEVICE, "hipStreamCreate failed: %s", hipGetErrorString(e));
     }
-    // the radial fit runs on host threads beside the plan's other tables
+    // What only the mixed precisions use is laid out for plans created with them, else by
+    // sfb_plan_set_precision.  The radial fit runs beside the plan's other tables, on few threads:
+    // one takes 1.4 ms at 87 maps, 4.7 at 237 and 121 at 2514, the tables 1.6, 4.4 and 248 ms.
     sfb::RadialBasis basis;
-    auto fit_basis = [&]() { return sfb::radial_basis(nmaps, knot_off, knot_x, knot_y, knot_ypp, &basis); };
+    auto fit_basis = [&]() {
+        return sfb::radial_basis(nmaps, knot_off, knot_x, knot_y, knot_ypp, &basis, nmaps < 2048 ? 2 : 4);
+    };
     std::future<bool> fit;
-    try {
-        fit = std::async(std::launch::async, fit_basis);
-    } catch (const std::system_error&) {  // no thread to spare
+    if (precision == SFB_PREC_MIXED) {
+        try {
+            fit = std::async(std::launch::async, fit_basis);
+        } catch (const std::system_error&) {  // no thread to spare: fitted below
+        }
     }
     int rc = plan_tables(P, lmax_n, knot_off, knot_x, knot_y, knot_ypp);
-    const bool fitted = fit.valid() ? fit.get() : fit_basis();
-    if (!rc) rc = shells_tables(P, basis, fitted && P->dir.ok);
+    const bool fitted = fit.valid() && fit.get();
+    if (!rc && fitted) rc = shells_tables(P, basis, P->dir.ok);
+    if (!rc && precision == SFB_PREC_MIXED && !fitted) rc = shells_build(P);
     if (!rc) rc = fold_tables(P);
-    if (!rc) rc = autotune_phi(P);
+    if (!rc) rc = autotune_phi(P, false);
+    if (!rc && precision != SFB_PREC_FP64) rc = autotune_phi(P, true);
     if (rc) {
         sfb_plan_destroy(P);
         return rc;
@@ -3926,6 +3938,11 @@ extern "C" int sfb_plan_set_precision(sfb_plan* P, int32_t precision)
 {
     if (!P) return fail(SFB_ERR_ARG, "plan is NULL");
     if (precision < SFB_PREC_FP64 || precision > SFB_PREC_BF16X2) return fail(SFB_ERR_ARG, "unknown precision %d", precision);
+    sfb::clear_error();
+    HIP_TRY(hipSetDevice(P->device));
+    int rc;
+    if (precision == SFB_PREC_MIXED && (rc = shells_build(P))) return rc;
+    if (precision != SFB_PREC_FP64 && (rc = autotune_phi(P, true))) return rc;
     P->precision = precision;
     return SFB_OK;
 }
@@ -4492,17 +4509,17 @@ static int phi_transform(sfb_plan* P, int32_t nq, hipStream_t st, bool f32, bool
     return SFB_OK;
 }
 
-// Plan-time tile search for the phi-transform.  Candidates: maps per FFT block (powers of
-// two whose LDS fits) x 256 / 512 threads, for FP64 and for FP32, then up to 32 / 64 maps per
-// polar block.  Each runs the whole transform over the first TUNE_MAPS maps of the plan's
+// Plan-time tile search for the phi-transform of FP64 maps or (plans of the other precisions) FP32
+// ones, once each.  Candidates: maps per FFT block (powers of two whose LDS fits) x 256 / 512
+// threads.  Each runs the whole transform over the first TUNE_MAPS maps of the plan's
 // (zeroed) map buffer (every map alike; 1024 maps give the grid thousands of blocks per
 // ring-pair class), once to warm up and three times timed on the plan's stream; the fastest stays.
 // Tile shapes change no arithmetic (each ring sequence is transformed alike), so the search
 // moves only the time.  SFB_TUNE=0 in the environment keeps the fixed defaults.
-static int autotune_phi(sfb_plan* P)
+static int autotune_phi(sfb_plan* P, bool f32)
 {
     const char* env = std::getenv("SFB_TUNE");
-    if (env && env[0] == '0') return SFB_OK;
+    if (P->tuned[f32] || (env && env[0] == '0')) return SFB_OK;
     const auto t_start = std::chrono::steady_clock::now();
     hipStream_t st = P->stream;
     constexpr int32_t TUNE_MAPS = 1024;
@@ -4514,15 +4531,18 @@ static int autotune_phi(sfb_plan* P)
     // SELL_SIGMA); time the tiles on that access pattern, with a fixed pseudo-random
     // permutation inside the same windows.
     DevBuf d_perm;
-    struct Release {  // the permutation buffer is freed on every return
+    struct Release {  // the permutation buffer is freed on every return; no phase is timed meanwhile
         DevBuf& b;
         sfb_plan* p;
+        bool prof;
         ~Release()
         {
             p->delta_perm = nullptr;
+            p->prof = prof;
             b.release();
         }
-    } release_perm{d_perm, P};
+    } release_perm{d_perm, P, P->prof};
+    P->prof = false;
     if (P->sell_ok && P->npix % 64 == 0) {
         std::vector<uint32_t> perm((size_t)P->npix);
         uint64_t x = 0x9E3779B97F4A7C15ull;
@@ -4563,9 +4583,9 @@ static int autotune_phi(sfb_plan* P)
         return SFB_OK;
     };
     const int64_t M = 2 * P->nside;
-    for (int f = 0; f < 2 && !rc; ++f) {
-        int32_t& tq = f ? P->TQF32 : P->TQF;
-        int32_t& nt = f ? P->fft_nt32 : P->fft_nt;
+    {
+        int32_t& tq = f32 ? P->TQF32 : P->TQF;
+        int32_t& nt = f32 ? P->fft_nt32 : P->fft_nt;
         // FFT tiles (the polar kernel's shape is fixed by the ring sizes)
         int32_t btq = tq, bnt = nt;
         float bms = 1e30f;
@@ -4576,7 +4596,7 @@ static int autotune_phi(sfb_plan* P)
                 tq = cq;
                 nt = cn;
                 float ms = 0.0f;
-                if ((rc = timed(f == 1, &ms))) break;
+                if ((rc = timed(f32, &ms))) break;
                 if (ms < bms) {
                     bms = ms;
                     btq = cq;
@@ -4590,7 +4610,8 @@ static int autotune_phi(sfb_plan* P)
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     HIP_TRY(hipStreamSynchronize(st));  // the search's work is done before d_perm is freed
-    P->tune_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
+    P->tune_ms += std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t_start).count();
+    P->tuned[f32] = !rc;
     return rc;
 }
 

@@ -44,7 +44,8 @@ double spline_deriv(int64_t n, const double* x, const double* y, const double* y
 // coefficients of map q's spline.  radial_basis returns false when the maps' knots do not share
 // their ends, the basis would exceed RADIAL_MAX functions, or a spline is further than
 // RADIAL_TOL of its largest value from its representation (half an FP32 unit: what the
-// per-map path's FP32 records lose); err is the largest such distance.
+// per-map path's FP32 records lose); err is the largest such distance.  The splines are fitted
+// by up to `threads` threads.
 constexpr int RADIAL_DEGREE = 9;
 constexpr int64_t RADIAL_MAX = 448;
 constexpr double RADIAL_TOL = 5.9604644775390625e-8;
@@ -54,7 +55,7 @@ struct RadialBasis {
     double err = 0.0;
 };
 bool radial_basis(int64_t nmaps, const int64_t* off, const double* kx, const double* ky, const double* kypp,
-                  RadialBasis* out);
+                  RadialBasis* out, int threads);
 
 // Fault injection for the error-path tests, from the environment variable SFB_FAULT:
 // "alloc" makes every device allocation fail (SFB_ERR_DEVICE), "maxevals" gives the k_nl

@@ -7,6 +7,7 @@ static int shells_tables(sfb_plan* P, const sfb::RadialBasis& R, bool fitted)
 {
     Shells& S = P->shells;
     S.ok = false;
+    S.tried = true;
     // the maps' buffers hold the shells and the mask, and the blocks' tables fit in LDS
     if (!fitted || !P->seg_uniform || R.nc + 1 > P->nmaps || (int64_t)sh_lds(R.nc) > P->lds_max ||
         16 * SM_N * (int64_t)P->tbl_cap > P->lds_max - 1024)
@@ -24,6 +25,7 @@ static int shells_tables(sfb_plan* P, const sfb::RadialBasis& R, bool fitted)
                 gt[(size_t)(l0 * R.nc + s * cnt + j)] = R.gamma[(size_t)(lq[(size_t)(l0 + j)] * (int64_t)R.nc + s)];
     }
     int r;
+    S.tried = false;  // (until every table is there)
     if ((r = S.d_knots.ensure(sizeof(double) * R.t.size())) || (r = S.d_gamma.ensure(sizeof(double) * gt.size())) ||
         (r = S.d_lstart.ensure(4 * lstart.size())) || (r = S.d_lq.ensure(4 * lq.size())))
         return r;
@@ -32,8 +34,37 @@ static int shells_tables(sfb_plan* P, const sfb::RadialBasis& R, bool fitted)
     HIP_TRY(hipMemcpy(S.d_knots.p, R.t.data(), sizeof(double) * R.t.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(S.d_gamma.p, gt.data(), sizeof(double) * gt.size(), hipMemcpyHostToDevice));
     S.nc = R.nc;
-    S.ok = true;
+    S.ok = S.tried = true;
     return SFB_OK;
+}
+
+// The basis and its tables for a plan that has none yet, from the splines it holds on the device
+// (records (x, y, y'', .) of every knot).
+static int shells_build(sfb_plan* P)
+{
+    if (P->shells.tried) return SFB_OK;
+    sfb::RadialBasis basis;
+    bool fitted = false;
+    if (P->dir.ok) {
+        try {
+            const size_t n = (size_t)(P->maps.back().koff + P->maps.back().nk);
+            std::vector<double> rec(4 * n), kx(n), ky(n), kypp(n);
+            HIP_TRY(hipMemcpy(rec.data(), P->d_rec.p, sizeof(double) * rec.size(), hipMemcpyDeviceToHost));
+            for (size_t i = 0; i < n; ++i) {
+                kx[i] = rec[4 * i];
+                ky[i] = rec[4 * i + 1];
+                kypp[i] = rec[4 * i + 2];
+            }
+            std::vector<int64_t> off;
+            for (const MapInfo& m : P->maps) off.push_back(m.koff);
+            off.push_back((int64_t)n);
+            fitted = sfb::radial_basis(P->nmaps, off.data(), kx.data(), ky.data(), kypp.data(), &basis,
+                                       (int)std::min(16u, std::thread::hardware_concurrency()));
+        } catch (const std::bad_alloc&) {
+            return fail(SFB_ERR_NOMEM, "out of host memory for the radial basis");
+        }
+    }
+    return shells_tables(P, basis, fitted);
 }
 
 // Parts of the spread's galaxy runs: blocks of 512 galaxies at least, 12 blocks per CU at most.

@@ -93,20 +93,25 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
         qoff[(size_t)b + 1] = qoff[(size_t)b] + std::max(J - 1, 0) * a * a;
     }
     int rc;
-    DevBuf V, I0, P0, P1, mm;  // plan-time scratch
-    struct Scratch {
-        DevBuf* b[5];
-        ~Scratch() { for (DevBuf* x : b) x->release(); }
-    } scratch{{&V, &I0, &P0, &P1, &mm}};
-    const size_t icb = sizeof(double) * (size_t)std::max<int64_t>(1, P->ic0_off.back());
+    struct Scratch {  // plan-time scratch, in two allocations
+        DevBuf tab, mm;
+        ~Scratch()
+        {
+            tab.release();
+            mm.release();
+        }
+    } scratch;
+    const int64_t icn = P->ic0_off.back();
     auto dbl = [](int64_t n) { return sizeof(double) * (size_t)std::max<int64_t>(1, n); };
     if ((rc = D.d_lamP.ensure(dbl(P->lam_size))) || (rc = D.d_lamPT.ensure(dbl(P->lam_size))) ||
         (rc = D.d_HB.ensure(dbl(hboff.back()))) || (rc = D.d_GZ.ensure(dbl(hboff.back()))) ||
         (rc = D.d_UB.ensure(dbl(voff.back()))) || (rc = D.d_ZB.ensure(dbl(voff.back()))) ||
         (rc = D.d_Q.ensure(dbl(qoff.back()))) || (rc = D.d_qoff.ensure(sizeof(int64_t) * qoff.size())) ||
         (rc = D.d_st.ensure(sizeof(AliasState) * st.size())) || (rc = D.d_term.ensure(sizeof(AliasTerm) * terms.size())) ||
-        (rc = V.ensure(dbl(voff.back()))) || (rc = I0.ensure(icb)) || (rc = P0.ensure(icb)) || (rc = P1.ensure(icb)))
+        (rc = scratch.tab.ensure(dbl(voff.back() + 3 * icn))))
         return rc;
+    double* const V = scratch.tab.as<double>();
+    double *const I0 = V + voff.back(), *const P0 = I0 + icn, *const P1 = P0 + icn;
     HIP_TRY(hipMemcpy(D.d_qoff.p, qoff.data(), sizeof(int64_t) * qoff.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(D.d_st.p, st.data(), sizeof(AliasState) * st.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(D.d_term.p, terms.data(), sizeof(AliasTerm) * terms.size(), hipMemcpyHostToDevice));
@@ -140,13 +145,13 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
         d.C = C; d.crs = crs; d.ccs = ccs; d.M = M; d.N = N; d.K = Kk;
     };
     // I0 = P0 = 1
-    for (DevBuf* buf : {&I0, &P0})
+    for (double* buf : {I0, P0})
         batch([&](int64_t b, SmallMM& d) {
         d.eye = 1;
         const int32_t n = n_of(b);
-        set(d, nullptr, 0, 0, nullptr, 0, 0, buf->as<double>() + P->ic0_off[(size_t)b], n, 1, n, n, 0);
+        set(d, nullptr, 0, 0, nullptr, 0, 0, buf + P->ic0_off[(size_t)b], n, 1, n, n, 0);
     });
-    double *pc = P0.as<double>(), *pn = P1.as<double>();
+    double *pc = P0, *pn = P1;
     for (int32_t j = 0; j < J; ++j) {
         const int64_t Jj = j;
         // U_j = P_j S^T and V_j = D^j S^T (V_0 = S^T), columns j na .. of the block's n x J na
@@ -157,9 +162,9 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
         });
         batch([&](int64_t b, SmallMM& d) {
             const int32_t n = n_of(b), a = a_of(b);
-            double* v = V.as<double>() + voff[(size_t)b];
+            double* v = V + voff[(size_t)b];
             if (j == 0)
-                set(d, I0.as<double>() + P->ic0_off[(size_t)b], n, 1, lam(b) + k_of(b) * n, 1, n, v,
+                set(d, I0 + P->ic0_off[(size_t)b], n, 1, lam(b) + k_of(b) * n, 1, n, v,
                 (int64_t)J * a, 1, n, a, n);
             else
                 set(d, P->d_ic0.as<double>() + P->ic0_off[(size_t)b], n, 1, v + (Jj - 1) * a, (int64_t)J * a, 1,
@@ -195,24 +200,25 @@ static int direct_tables(sfb_plan* P, const std::vector<RingDev>& rd, const std:
         batch([&](int64_t b, SmallMM& d) {
             const int32_t n = n_of(b), a = a_of(b);
             d.alpha = domega;
-            set(d, V.as<double>() + voff[(size_t)b] + jr * a, 1, (int64_t)J * a,
-                I0.as<double>() + P->ic0_off[(size_t)b], n, 1,
+            set(d, V + voff[(size_t)b] + jr * a, 1, (int64_t)J * a,
+                I0 + P->ic0_off[(size_t)b], n, 1,
                 D.d_ZB.as<double>() + voff[(size_t)b] + (int64_t)j * a * n, n, 1, a, n, n);
         });
         batch([&](int64_t b, SmallMM& d) {
             const int32_t n = n_of(b), a = a_of(b);
             d.alpha = domega;
-            set(d, V.as<double>() + voff[(size_t)b] + jr * a, 1, (int64_t)J * a, lam(b), 1, n,
+            set(d, V + voff[(size_t)b] + jr * a, 1, (int64_t)J * a, lam(b), 1, n,
                 D.d_GZ.as<double>() + hboff[(size_t)b] + (int64_t)j * a * K, K, 1, a, K, n);
         });
         if (j + 1 < J) batch([&](int64_t b, SmallMM& d) {  // Q_j = dOmega S V_j
             const int32_t n = n_of(b), a = a_of(b);
             d.alpha = domega;
-            set(d, lam(b) + k_of(b) * n, n, 1, V.as<double>() + voff[(size_t)b] + (int64_t)j * a,
+            set(d, lam(b) + k_of(b) * n, n, 1, V + voff[(size_t)b] + (int64_t)j * a,
                 (int64_t)J * a, 1, D.d_Q.as<double>() + qoff[(size_t)b] + (int64_t)j * a * a, a,
                 1, a, a, n);
         });
     }
+    DevBuf& mm = scratch.mm;
     if ((rc = mm.ensure(sizeof(SmallMM) * std::max<size_t>(1, all.size())))) return rc;
     if (!all.empty()) HIP_TRY(hipMemcpy(mm.p, all.data(), sizeof(SmallMM) * all.size(), hipMemcpyHostToDevice));
     for (const Launch& l : launches) {
