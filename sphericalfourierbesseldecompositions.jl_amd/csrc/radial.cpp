@@ -12,8 +12,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <exception>
 #include <new>
-#include <system_error>
 #include <thread>
 
 #include "sfb_internal.h"
@@ -174,9 +174,10 @@ static bool fit(int64_t nmaps, const int64_t* off, const double* kx, const doubl
     };
     const int nt = (int)std::min<int64_t>(std::max(1, threads), 1 + nmaps / 16);
     std::vector<std::thread> th;
+    th.reserve((size_t)nt);  // (a failure here leaves no thread behind)
     try {
         for (int i = 1; i < nt; ++i) th.emplace_back(work);
-    } catch (const std::system_error&) {  // fewer threads than asked for: this one does the rest
+    } catch (const std::exception&) {  // no thread or no memory for one: the others do the rest
     }
     work();
     for (std::thread& x : th) x.join();

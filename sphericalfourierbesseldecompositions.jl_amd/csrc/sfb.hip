@@ -30,11 +30,11 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <future>
 #include <mutex>
 #include <new>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -3876,7 +3876,7 @@ extern "C" int sfb_plan_create(sfb_plan** out, int64_t nside, int64_t lmax, int6
     if (precision == SFB_PREC_MIXED) {
         try {
             fit = std::async(std::launch::async, fit_basis);
-        } catch (const std::system_error&) {  // no thread to spare: fitted below
+        } catch (const std::exception&) {  // no thread or no memory for one: fitted below
         }
     }
     int rc = plan_tables(P, lmax_n, knot_off, knot_x, knot_y, knot_ypp);
