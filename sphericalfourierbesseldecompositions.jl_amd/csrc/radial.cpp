@@ -52,11 +52,13 @@ static bool fit(int64_t nmaps, const int64_t* off, const double* kx, const doubl
                 RadialBasis* R, int threads)
 {
     if (nmaps < 1) return false;
+    for (int64_t q = 0; q < nmaps; ++q)  // (this runs beside the plan's own checks of the tables)
+        if (off[q + 1] - off[q] < 4) return false;
     const double lo = kx[off[0]], hi = kx[off[1] - 1];
     double H = hi - lo;
     for (int64_t q = 0; q < nmaps; ++q) {
         const int64_t nk = off[q + 1] - off[q];
-        if (nk < 4 || kx[off[q]] != lo || kx[off[q + 1] - 1] != hi) return false;
+        if (kx[off[q]] != lo || kx[off[q + 1] - 1] != hi) return false;
         H = std::min(H, (hi - lo) / (double)(nk - 1));
     }
     const double len = hi - lo;

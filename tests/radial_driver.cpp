@@ -1,5 +1,8 @@
-// radial_basis under failing allocations (tests/test_radial_basis.py).
+// radial_basis under failing allocations and odd knot offsets (tests/test_radial_basis.py).
 //   fail FILE     allocation k = 1, 2, .. throws until a call needs no more: prints the count
+//   empty         maps without knots, their table behind an unreadable page: prints the result
+#include <sys/mman.h>
+
 #include <atomic>
 #include <cstdio>
 #include <cstdlib>
@@ -21,6 +24,16 @@ void operator delete(void* p, std::size_t) noexcept { std::free(p); }
 
 int main(int argc, char** argv)
 {
+    if (argc > 1 && !std::strcmp(argv[1], "empty")) {
+        char* m = (char*)mmap(nullptr, 3 * 4096, PROT_READ | PROT_WRITE, MAP_PRIVATE | MAP_ANONYMOUS, -1, 0);
+        if (m == (char*)MAP_FAILED || mprotect(m, 4096, PROT_NONE) || mprotect(m + 2 * 4096, 4096, PROT_NONE)) return 2;
+        const double* x = (const double*)(m + 4096);
+        const int64_t off[3] = {0, 0, 0}, end[2] = {512, 512};
+        sfb::RadialBasis R;
+        const bool a = sfb::radial_basis(2, off, x, x, x, &R, 4), b = sfb::radial_basis(1, end, x, x, x, &R, 4);
+        std::printf("%d %d\n", a, b);
+        return 0;
+    }
     if (argc < 3) return 2;
     FILE* f = std::fopen(argv[2], "rb");
     if (!f) return 2;

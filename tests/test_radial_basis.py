@@ -1,6 +1,6 @@
 """The host fit of the mixed path's radial basis (csrc/radial.cpp) on its own, on the CPU: an allocation
 that fails at any point, those for its threads included, gives `no basis` and never ends the
-process."""
+process; tables without knots are turned down before anything is read."""
 import os
 import subprocess
 
@@ -43,3 +43,9 @@ def test_allocation_failures(driver, tmp_path):
     assert r.returncode == 0, (r.returncode, r.stderr[-300:])
     tried, ok, nc = map(int, r.stdout.split())
     assert tried > 10 and ok == 1 and nc > 20
+
+
+def test_tables_without_knots(driver):
+    r = driver("empty")
+    assert r.returncode == 0, r.returncode
+    assert r.stdout.split() == ["0", "0"]
