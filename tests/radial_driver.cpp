@@ -1,5 +1,6 @@
 // radial_basis under failing allocations and odd knot offsets (tests/test_radial_basis.py).
 //   fail FILE     allocation k = 1, 2, .. throws until a call needs no more: prints the count
+//   count FILE    prints the number of basis functions
 //   empty         maps without knots, their table behind an unreadable page: prints the result
 #include <sys/mman.h>
 
@@ -44,6 +45,12 @@ int main(int argc, char** argv)
     if (std::fread(off.data(), 8, off.size(), f) != off.size() || std::fread(t.data(), 8, t.size(), f) != t.size()) return 2;
     std::fclose(f);
     const double *x = t.data(), *y = x + n[1], *ypp = y + n[1];
+    if (!std::strcmp(argv[1], "count")) {
+        sfb::RadialBasis R;
+        const bool ok = sfb::radial_basis(n[0], off.data(), x, y, ypp, &R, 4);
+        std::printf("%d %d\n", ok, R.nc);
+        return 0;
+    }
     for (long k = 0;; ++k) {
         sfb::RadialBasis R;
         g_left = k;

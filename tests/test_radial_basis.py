@@ -1,8 +1,10 @@
 """The host fit of the mixed path's radial basis (csrc/radial.cpp) on its own, on the CPU: an allocation
 that fails at any point, those for its threads included, gives `no basis` and never ends the
-process; tables without knots are turned down before anything is read."""
+process; tables without knots are turned down before anything is read; and bench.py's count of
+the basis functions is the one the fit makes."""
 import os
 import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -49,3 +51,23 @@ def test_tables_without_knots(driver):
     r = driver("empty")
     assert r.returncode == 0, r.returncode
     assert r.stdout.split() == ["0", "0"]
+
+
+@pytest.mark.parametrize("kmax,rmin,rmax,nside", [(0.03, 500.0, 1000.0, 16), (0.05, 500.0, 1000.0, 32),
+                                                  (0.1, 500.0, 1500.0, 128)])
+def test_bench_counts_the_same_functions(driver, tmp_path, kmax, rmin, rmax, nside):
+    sys.path.insert(0, ROOT)
+    import bench
+
+    am = S.AnlmModes(kmax, rmin, rmax, nside=nside)
+    # (the finest table sets the breaks; the others only have to share its ends)
+    q = int(np.argmax(np.diff(am.knot_off)))
+    lo, hi = am.knot_off[q], am.knot_off[q + 1]
+    with open(tmp_path / "t", "wb") as f:
+        np.array([1, hi - lo, 0, hi - lo], dtype=np.int64).tofile(f)
+        for a in (am.knot_x, am.knot_y, am.knot_ypp):
+            np.asarray(a[lo:hi], dtype=np.float64).tofile(f)
+    r = driver("count", str(tmp_path / "t"))
+    assert r.returncode == 0
+    ok, nc = map(int, r.stdout.split())
+    assert ok == 1 and nc == bench.shell_count(am)
