@@ -4703,7 +4703,7 @@ static int sht_stage(sfb_plan* P, int32_t nq, hipStream_t st, bool f32 = false, 
 // block does not fit in LDS); equatorial ones: the inverse FFT (the direct sum where its
 // block does not fit).
 template <typename R>
-static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st, int64_t ld)
+static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st)
 {
     const int32_t K = P->K, L = (int32_t)P->lmax;
     const InvShapes S = inv_shapes(P->nside, L, P->lds_max);  // sized for FP64: FP32 blocks use less
@@ -4715,7 +4715,7 @@ static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st
         const int32_t ntile = (int32_t)((nq + S.tqmin - 1) / S.tqmin);
         const int64_t units = (int64_t)S.nip4 * ntile;
         hipLaunchKernelGGL(k_phi_ipolar4<R>, dim3((unsigned)(32 * ((units + 31) / 32))), dim3(256), S.shq, st, X,
-                           P->npix, nq, ld, K, L, P->d_rings.as<RingDev>(), P->d_tw.as<double2>(), scale, out,
+                           P->npix, nq, P->M2, K, L, P->d_rings.as<RingDev>(), P->d_tw.as<double2>(), scale, out,
                            IP_TQMAX, P->d_mall.as<int32_t>(), S.nip4, ntile);
         LAUNCH_CHECK();
     }
@@ -4724,7 +4724,7 @@ static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st
         const size_t shs = sizeof(double2) * 2 * TQS * (size_t)(L + 1);
         HIP_TRY(hipFuncSetAttribute((const void*)k_phi_synth<R>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shs));
         hipLaunchKernelGGL(k_phi_synth<R>, dim3((unsigned)(S.k_eq0 - S.nip4), nblk(nq, TQS)), dim3(256), shs, st, X,
-                           P->npix, nq, ld, K, L, P->d_rings.as<RingDev>(), scale, out, TQS,
+                           P->npix, nq, P->M2, K, L, P->d_rings.as<RingDev>(), scale, out, TQS,
                            P->d_mall.as<int32_t>(), S.nip4);
         LAUNCH_CHECK();
     }
@@ -4732,18 +4732,16 @@ static int phi_synthesis_t(sfb_plan* P, int32_t nq, double scale, hipStream_t st
         HIP_TRY(hipFuncSetAttribute((const void*)k_phi_ifft<R>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)S.shi));
         const int64_t units = (int64_t)(K - S.k_eq0) * nblk(nq, S.tqi);
         hipLaunchKernelGGL(k_phi_ifft<R>, dim3((unsigned)(32 * ((units + 31) / 32))), dim3(512), S.shi, st, X,
-                           P->npix, nq, ld, K, L, P->d_rings.as<RingDev>(), P->d_tw.as<double2>(), scale, out,
+                           P->npix, nq, P->M2, K, L, P->d_rings.as<RingDev>(), P->d_tw.as<double2>(), scale, out,
                            S.tqi, S.k_eq0, P->logM, P->d_mall.as<int32_t>());
         LAUNCH_CHECK();
     }
     return SFB_OK;
 }
 
-static int phi_synthesis(sfb_plan* P, int32_t nq, double scale, hipStream_t st, bool f32 = false,
-                         int64_t ld = 0)
+static int phi_synthesis(sfb_plan* P, int32_t nq, double scale, hipStream_t st, bool f32 = false)
 {
-    if (!ld) ld = P->M2;
-    return f32 ? phi_synthesis_t<float>(P, nq, scale, st, ld) : phi_synthesis_t<double>(P, nq, scale, st, ld);
+    return f32 ? phi_synthesis_t<float>(P, nq, scale, st) : phi_synthesis_t<double>(P, nq, scale, st);
 }
 
 // Launch shapes of the ring transforms for a geometry (host arithmetic, no device).
