@@ -552,8 +552,11 @@ __global__ __launch_bounds__(256) void k_phi_ipolar4_fold(const R* __restrict__ 
 constexpr int VF_THR = 512;         // two blocks per CU: one sums while the other stages
 constexpr int VF_MAPS = 16;          // maps per stage at most
 constexpr int VF_LDS = 78 << 10;
-constexpr int VF_BIN = 7 << 10;     // record bytes of one map in a radius bin (40 KB: 4.04 ms, 10: 2.42, 7: 2.18, 5: 2.17, 3: 2.24)
-constexpr int VF_BLOCKS = 2048;     // blocks wanted
+constexpr int VF_BIN = 7 << 10;     // record bytes of one map in a radius bin (1e6 galaxies, 2514 maps, FP32: one
+                                    // bin of 40 KB 3.18 ms, 10: 1.92, 7: 1.80, 5: 1.80; 2e5, 344 maps, FP64:
+                                    // 153, 127, 125 and 124 us)
+constexpr int VF_BLOCKS = 2048;     // blocks wanted (with the reduction of their sums, the same cases: 1024 1.98 ms
+                                    // and 130 us, 2048 1.88 and 141, 4096 1.92 and 142)
 template <typename R> struct VfGpt { static constexpr int N = sizeof(R) == 8 ? 4 : 8; };  // galaxies per thread
 __device__ __forceinline__ float vf_flip(float d, uint32_t s) { return __uint_as_float(__float_as_uint(d) ^ s); }
 __device__ __forceinline__ double vf_flip(double d, uint32_t s)

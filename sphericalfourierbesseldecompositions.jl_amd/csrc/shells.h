@@ -67,11 +67,13 @@ static int shells_build(sfb_plan* P)
     return shells_tables(P, basis, fitted);
 }
 
-// Parts of the spread's galaxy runs: blocks of 512 galaxies at least, 12 blocks per CU at most.
+// Parts of the spread's galaxy runs: blocks of 256 galaxies at least, 12 blocks per CU at most.  Spread
+// at nside 16 with blocks of 256 / 512 / 1024 at least: 52 / 87 / 196 us for 3e5 galaxies, 508 / 509 / 506
+// for 4e6; at nside 32, 1e6: 108 / 113 / 180 (the sum of the parts takes 5 to 7).
 static int32_t shell_parts(int64_t N, int64_t npix)
 {
     const int64_t nb = nblk(npix, SH_PT);
-    return (int32_t)std::max<int64_t>(1, std::min<int64_t>(3072 / nb, N / (512 * nb)));
+    return (int32_t)std::max<int64_t>(1, std::min<int64_t>(3072 / nb, N / (256 * nb)));
 }
 
 // One mixed cat2amln over the shells, enqueued on st (separable window).

@@ -7,11 +7,11 @@
 // replace and a column's states no longer fit in LDS: the iterated form stays (jacobi_stage).
 constexpr int32_t DIRECT_MAX_NITER = 8, DIRECT_MAX_NAL = 48, DIRECT_MAX_STATES = 1536;
 
-// Columns per k_alias_solve block: 8 (64-byte rows) for many columns, 4 for few (twice the
-// blocks), fewer when the states do not fit.
-static inline int32_t direct_alias_ct(const DirectSht& D, int32_t J, int32_t cols, int64_t lds_max)
+// Columns per k_alias_solve block: 4 (8: 80 us against 77 for 5028 columns at nside 128, 25 against 20
+// for 320, 28 against 20 at nside 32), fewer when the states do not fit.
+static inline int32_t direct_alias_ct(const DirectSht& D, int32_t J, int64_t lds_max)
 {
-    int32_t ct = cols >= 2048 ? 8 : 4;
+    int32_t ct = 4;
     while (ct > 1 && (int64_t)alias_lds(D.S, J, ct, D.nterm) > lds_max) ct /= 2;
     return ct;
 }
@@ -328,7 +328,7 @@ static int direct_alias(sfb_plan* P, int32_t cols, int64_t ld, hipStream_t st, i
 {
     DirectSht& D = P->dir;
     const int32_t J = P->niter;
-    const int32_t ct = direct_alias_ct(D, J, cols, P->lds_max);
+    const int32_t ct = direct_alias_ct(D, J, P->lds_max);
     const size_t shm = alias_lds(D.S, J, ct, D.nterm);
     HIP_TRY(hipFuncSetAttribute((const void*)k_alias_solve, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
     hipLaunchKernelGGL(k_alias_solve, dim3(nblk(cols, ct), split < 0 ? 2u : 1u), dim3(1024), shm, st, D.S, J,

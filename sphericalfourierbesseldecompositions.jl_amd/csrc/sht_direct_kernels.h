@@ -105,7 +105,7 @@ struct AliasTerm {
 // stay in LDS over the J steps, with the states and couplings beside them, so that after one round
 // of loads only the Q rows come from L2.  What bounds it is the chain of 2 J dependent phases
 // over a few hundred states, not bytes (states, couplings and h read phase by phase: 115 us for
-// 5028 columns and 441 states, 28 us for 320 columns; now 78 and 20 us).
+// 5028 columns and 441 states, 28 us for 320 columns; now 77 and 20 us).
 __host__ __device__ inline size_t alias_lds(int32_t S, int32_t J, int32_t CT, int32_t nterm)
 {
     return sizeof(double) * (size_t)(J + 1) * (size_t)S * (size_t)CT + sizeof(AliasTerm) * (size_t)nterm +

@@ -12,7 +12,7 @@ from test_gpu_shells import block_error
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nside,nl,n", [(2, (20, 8), 3 * 1024 - 1), (2, (20, 8), 3 * 1024), (2, (20, 8), 60001),
+@pytest.mark.parametrize("nside,nl,n", [(2, (20, 8), 3 * 512 - 1), (2, (20, 8), 3 * 512), (2, (20, 8), 60001),
                                         (4, (30, 8), 12 * 1024), (8, (30, 12), 300007), (16, (30, 12), 196608),
                                         (32, (30, 12), 1600001)])
 def test_parts(nside, nl, n):
