@@ -4513,7 +4513,9 @@ static int phi_transform(sfb_plan* P, int32_t nq, hipStream_t st, bool f32, bool
 // ones, once each.  Candidates: maps per FFT block (powers of two whose LDS fits) x 256 / 512
 // threads.  Each runs the whole transform over the first TUNE_MAPS maps of the plan's
 // (zeroed) map buffer (every map alike; 1024 maps give the grid thousands of blocks per
-// ring-pair class), once to warm up and three times timed on the plan's stream; the fastest stays.
+// ring-pair class), or, for FP64 on a plan with radial shells, over as many as its calls transform,
+// in their compact rows and pixel order; once to warm up and three times timed on the plan's
+// stream; the fastest stays.
 // Tile shapes change no arithmetic (each ring sequence is transformed alike), so the search
 // moves only the time.  SFB_TUNE=0 in the environment keeps the fixed defaults.
 static int autotune_phi(sfb_plan* P, bool f32)
@@ -4523,7 +4525,9 @@ static int autotune_phi(sfb_plan* P, bool f32)
     const auto t_start = std::chrono::steady_clock::now();
     hipStream_t st = P->stream;
     constexpr int32_t TUNE_MAPS = 1024;
-    const int32_t nq = (int32_t)std::min<int64_t>(P->nmaps, TUNE_MAPS);
+    const bool shells = !f32 && P->shells.ok;
+    const int32_t nq = shells ? P->shells.nc + 1 : (int32_t)std::min<int64_t>(P->nmaps, TUNE_MAPS);
+    const int64_t ld = shells ? 2 * (int64_t)nq : P->M2;
     const int64_t nd = (int64_t)nq * P->npix;
     hipLaunchKernelGGL(k_fill_f64, dim3(nblk(nd, 256)), dim3(256), 0, st, P->d_delta.as<double>(), nd, 0.0);
     LAUNCH_CHECK();
@@ -4543,7 +4547,7 @@ static int autotune_phi(sfb_plan* P, bool f32)
         }
     } release_perm{d_perm, P, P->prof};
     P->prof = false;
-    if (P->sell_ok && P->npix % 64 == 0) {
+    if (!shells && P->sell_ok && P->npix % 64 == 0) {
         std::vector<uint32_t> perm((size_t)P->npix);
         uint64_t x = 0x9E3779B97F4A7C15ull;
         for (int64_t w0 = 0; w0 < P->npix; w0 += SELL_SIGMA) {
@@ -4569,12 +4573,12 @@ static int autotune_phi(sfb_plan* P, bool f32)
     int rc = SFB_OK;
     auto timed = [&](bool f32, float* best) -> int {  // min over 3 runs, after one warm-up
         int r;
-        if ((r = phi_transform(P, nq, st, f32))) return r;
+        if ((r = phi_transform(P, nq, st, f32, true, nullptr, ld))) return r;
         *best = 1e30f;
         for (int it = 0; it < 3; ++it) {
             float ms = 0.0f;
             if (hipEventRecord(e0, st) != hipSuccess) return fail(SFB_ERR_DEVICE, "hipEventRecord failed");
-            if ((r = phi_transform(P, nq, st, f32))) return r;
+            if ((r = phi_transform(P, nq, st, f32, true, nullptr, ld))) return r;
             if (hipEventRecord(e1, st) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
                 hipEventElapsedTime(&ms, e0, e1) != hipSuccess)
                 return fail(SFB_ERR_DEVICE, "tile search timing failed");
