@@ -87,13 +87,14 @@ static int shells_enqueue(sfb_plan* P, int64_t N, const double* d_rtp, const dou
     {
         PhaseTimer timer(P, SFB_PHASE_SCATTER, st);
         const size_t shm = sh_lds(nc);
-        HIP_TRY(hipFuncSetAttribute((const void*)k_shell_spread, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
         const int32_t parts = shell_parts(N, P->npix);
         const int64_t n = (int64_t)nc * P->npix;
         if (parts > 1 && (rc = S.d_part.ensure(sizeof(double) * (size_t)(parts * n)))) return rc;
         double* D = P->d_delta.as<double>();
         double* to = parts > 1 ? S.d_part.as<double>() : D;
-        hipLaunchKernelGGL(k_shell_spread, dim3(nblk(P->npix, SH_PT), (unsigned)parts), dim3(SH_NT), shm, st, P->npix,
+        const auto spread = parts > 1 ? k_shell_spread<true> : k_shell_spread<false>;
+        HIP_TRY(hipFuncSetAttribute((const void*)spread, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
+        hipLaunchKernelGGL(spread, dim3(nblk(P->npix, SH_PT), (unsigned)parts), dim3(SH_NT), shm, st, P->npix,
                            nc, S.d_knots.as<double>(), P->d_pstart.as<int32_t>(), P->d_rs.as<double>(),
                            P->d_ws.as<double>(), d_mask, to, D + n);
         LAUNCH_CHECK();

@@ -38,8 +38,10 @@ __device__ __forceinline__ double rcp64(double d)
 // small blocks, four to a CU (32 pixels, 256 threads and tabulated reciprocals, two blocks to a
 // CU, ran 121 us at N = 1e6, nside 128, nc 159 and 1025 us at 4e6, nside 256, nc 219; now 109
 // and 515 us, 2.3 and 2.7 TB/s of the maps' write).
-// gridDim.y parts, for grids of few pixels with many galaxies each: part y takes its share of every
-// block's run and writes its own maps (part y at D + y nc npix), which k_shell_sum adds up.
+// PARTS: gridDim.y parts, for grids of few pixels with many galaxies each: part y takes its share of
+// every block's run and writes its own maps (part y at D + y nc npix), which k_shell_sum adds up (a
+// kernel of its own: the shares' divisions cost 4 of 99 us where there is one part).
+template <bool PARTS>
 __global__ __launch_bounds__(SH_NT) void k_shell_spread(int64_t npix, int32_t nc, const double* __restrict__ knots,
                                                         const int32_t* __restrict__ pstart,
                                                         const double* __restrict__ r_s, const double* __restrict__ w_s,
@@ -55,8 +57,12 @@ __global__ __launch_bounds__(SH_NT) void k_shell_spread(int64_t npix, int32_t nc
     const int64_t p0 = (int64_t)blockIdx.x * SH_PT;
     const int np = (int)min((int64_t)SH_PT, npix - p0);
     const int pl = tid % SH_PT, sub = tid / SH_PT;
-    const int64_t b0 = pstart[p0], run = pstart[p0 + np] - b0;
-    const int g0 = (int)(b0 + run * blockIdx.y / gridDim.y), g1 = (int)(b0 + run * (blockIdx.y + 1) / gridDim.y);
+    int g0 = pstart[p0], g1 = pstart[p0 + np];
+    if (PARTS) {
+        const int64_t b0 = g0, run = g1 - g0;
+        g0 = (int)(b0 + run * blockIdx.y / gridDim.y);
+        g1 = (int)(b0 + run * (blockIdx.y + 1) / gridDim.y);
+    }
     const int a0 = pl < np ? pstart[p0 + pl] : 0, a1 = pl < np ? pstart[p0 + pl + 1] : 0;
     for (int e = tid; e < nc * SH_PT; e += SH_NT) tile[e] = 0.0;
     if (g1 > g0)
@@ -106,10 +112,10 @@ __global__ __launch_bounds__(SH_NT) void k_shell_spread(int64_t npix, int32_t nc
         }
     }
     __syncthreads();
-    D += (int64_t)blockIdx.y * nc * npix;
+    if (PARTS) D += (int64_t)blockIdx.y * nc * npix;
     if (pl < np)
         for (int s = sub; s < nc; s += SH_SUB) D[(int64_t)s * npix + p0 + pl] = tile[s * SH_PT + pl];
-    if (blockIdx.y == 0 && tid < np) Dmask[p0 + tid] = mask[p0 + tid];
+    if ((!PARTS || blockIdx.y == 0) && tid < np) Dmask[p0 + tid] = mask[p0 + tid];
 }
 
 // D[e] = sum of the parts' maps in order, e < n = nc npix.  Bound by the parts' bytes.
