@@ -547,13 +547,13 @@ __global__ __launch_bounds__(256) void k_phi_ipolar4_fold(const R* __restrict__ 
 // 1/h, applied once to their sum.  Outside the knots the pseudo-records' slopes are 0.  R = float:
 // FP32 records, delta-bar and products, FP64 sums.
 // Bound: VALU (82% busy in FP32, 19 instructions per galaxy and map), then the random 16-byte
-// record reads from LDS.  1e6 galaxies, 2514 maps, FP32: 1.69 ms; whole tables staged, two
+// record reads from LDS.  1e6 galaxies, 2514 maps, FP32: 1.71 ms; whole tables staged, two
 // at a time by 1024 threads, ran 2.87 ms and moved 5.4 GB past L2.
 constexpr int VF_THR = 512;         // two blocks per CU: one sums while the other stages
 constexpr int VF_MAPS = 16;          // maps per stage at most
 constexpr int VF_LDS = 78 << 10;
-constexpr int VF_BIN = 7 << 10;     // record bytes of one map in a radius bin (1e6 galaxies, 2514 maps, FP32: one
-                                    // bin of 40 KB 3.18 ms, 10: 1.92, 7: 1.80, 5: 1.80; 2e5, 344 maps, FP64:
+constexpr int VF_BIN = 7 << 10;     // record bytes of one map in a radius bin (1e6 galaxies, 2514 maps, FP32, events
+                                    // around the launch: one bin of 40 KB 3.18 ms, 10: 1.92, 7: 1.80, 5: 1.80; 2e5, 344 maps, FP64:
                                     // 153, 127, 125 and 124 us)
 constexpr int VF_BLOCKS = 2048;     // blocks wanted (with the reduction of their sums, the same cases: 1024 1.98 ms
                                     // and 130 us, 2048 1.88 and 141, 4096 1.92 and 142)
