@@ -204,11 +204,13 @@ __global__ __launch_bounds__(1024) void k_shell_mono(int64_t N, int32_t nmx, con
 // coefficients of the shell maps (a layout, row stride ld, shell s at 2 s).  A block takes one
 // l and SC_M values of m: their Z rows stay in LDS, and 32 lanes take the maps of this l (lq,
 // cnt of them from l0) over gamma by shell, gt[l0 nc + s cnt + j].  A few MB and 0.1 GFLOP:
-// latency-bound, 36 to 40 us at nside 128 (159 shells, 116 345 coefficients), 112 us at nside 256.  The monopoles (l = 0: a wave per map) add c00 inv (exact sum - sum_s gamma_s
+// latency-bound, 36 us at nside 128 (159 shells, 116 345 coefficients), 112 us at nside 256.  The monopoles (l = 0: a wave per map) add c00 inv (exact sum - sum_s gamma_s
 // T_s), T_s = sum_p D_s(p) (at tsum[2 s]): the refinements pass an error of the first
 // analysis' monopole to a_00 one to one.
+// Aligned so that its 3.2 KB of code lie in one 4 KB page: where the linker had put the loop across two, the
+// same instructions took 40 us.
 constexpr int SC_M = 8;
-__global__ __launch_bounds__(256) void k_shell_contract(int32_t L, int32_t nc, const double* __restrict__ gt,
+__attribute__((aligned(4096))) __global__ __launch_bounds__(256) void k_shell_contract(int32_t L, int32_t nc, const double* __restrict__ gt,
                                                         const int32_t* __restrict__ lstart,
                                                         const int32_t* __restrict__ lq,
                                                         const MapInfo* __restrict__ maps,
