@@ -6,9 +6,9 @@
 //
 // The rank pass compares a pixel's galaxies pairwise.  A catalogue with many galaxies in every
 // pixel takes stable radix sorts instead (known from its size); a few crowded pixels
-// do not: their rank costs less than the sum over a pixel's galaxies in order that follows it, up
-// to PS_CROWD galaxies.  A pixel beyond raises flag[2] bit 1 and the call is redone with the
-// radix sorts.
+// do not: their rank costs little beside the sum over a pixel's galaxies in order that follows it, up
+// to PS_CROWD galaxies (1.5e5 in one pixel, nside 64: 0.3 of 21.4 ms mixed, 0.65 of 21.3 ms in FP64).  A
+// pixel beyond raises flag[2] bit 1 and the call is redone with the radix sorts.
 #pragma once
 
 // Mean galaxies per pixel above which the radix sorts run.  FP64 (by pixel and r, two sorts): at
@@ -21,6 +21,10 @@ constexpr int PS_MEAN_R = 1024, PS_MEAN = 96, PS_MEAN_ANY = 640;
 constexpr int PS_CROWD = 1 << 20; // galaxies of one pixel that the rank takes
 constexpr int PS_WALK = 64;       // galaxies of a pixel up to which each lane walks them (call at 96 per
                                   // pixel, nside 32 FP64: 478 us; 128: 550, 256: 534)
+constexpr int PS_OWN = 1024;      // galaxies a block ranks together in a giant pixel
+constexpr int PS_GIANT = 4096;    // galaxies of a pixel from which blocks rank it (catalogue stage of 3e5 galaxies with one
+                                  // such pixel, by wavefronts / by blocks: mixed 100 / 110 us at 3000, 124 / 117 at
+                                  // 4000, 205 / 174 at 10000; FP64 135 / 149, 182 / 184 at 7000, 223 / 210)
 constexpr int PS_CHUNK = 2048;    // pixels per scan block
 constexpr int PS_SMALL = 32;      // scan blocks up to which each adds up the counts before it itself (one launch
                                   // less; 4 blocks: 5.0 us against 7.2 in two, 13: 8.2 / 9.1, 49: 17.8 / 9.3)
@@ -203,6 +207,117 @@ __device__ __forceinline__ bool rank_less(const RankKey& x, const RankKey& y)
     return (x.a < y.a) | ((x.a == y.a) & (x.b < y.b));
 }
 
+// The places of a giant pixel's galaxies [e, e + PS_OWN) (the pixel's run ends at s1), by a whole block:
+// its own galaxies, sorted, stay in LDS and every galaxy of the pixel finds its place among them.  The list
+// entries of its own galaxies are written.
+struct RankLds {
+    uint64_t a[PS_OWN];
+    uint32_t b[PS_OWN], hist[PS_OWN];
+    int32_t wsum[4];
+};
+// o before the own galaxy at place i (b decides ties of a: radii bit for bit the same)
+template <int ORDER> __device__ __forceinline__ bool rank_before(const RankKey& o, const RankLds& L, int i)
+{
+    const uint64_t a = L.a[i];
+    bool less = o.a < a;
+    if (ORDER == 2 && o.a == a) less = o.b < L.b[i];
+    return less;
+}
+template <int ORDER>
+__device__ __forceinline__ void rank_block(const CatSlot* __restrict__ slot, int32_t e, int32_t s0, int32_t s1, RankLds& L,
+                                           uint32_t* __restrict__ idx, uint32_t* __restrict__ pix_s,
+                                           double* __restrict__ r_s, double* __restrict__ w_s)
+{
+    constexpr int U = PS_OWN / 256;
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, n = min(PS_OWN, s1 - e);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int j = t + 256 * u;
+        const RankKey k = j < n ? rank_key<ORDER>(slot[e + j]) : RankKey{~0ull, ~0u};
+        L.a[j] = k.a;
+        L.b[j] = k.b;
+        L.hist[j] = 0;
+    }
+    __syncthreads();
+    for (int m = 2; m <= PS_OWN; m <<= 1)  // bitonic sort
+        for (int d = m >> 1; d > 0; d >>= 1) {
+#pragma unroll
+            for (int u = 0; u < U / 2; ++u) {
+                const int q = t + 256 * u, i = ((q & ~(d - 1)) << 1) | (q & (d - 1));
+                const RankKey x{L.a[i], L.b[i]}, y{L.a[i + d], L.b[i + d]};
+                if (rank_less(y, x) == ((i & m) == 0)) {
+                    L.a[i] = y.a;
+                    L.b[i] = y.b;
+                    L.a[i + d] = x.a;
+                    L.b[i + d] = x.b;
+                }
+            }
+            __syncthreads();
+        }
+    constexpr int V = 2;  // searches in flight
+    int32_t none = 0;     // galaxies before every own one
+    RankKey nx[V];
+    auto load = [&](uint32_t c) {
+#pragma unroll
+        for (int u = 0; u < V; ++u) nx[u] = rank_key<ORDER>(slot[min(c + 256 * u, (uint32_t)s1 - 1)]);
+    };
+    load((uint32_t)s0 + t);
+    for (uint32_t c = (uint32_t)s0 + t; c < (uint32_t)s1; c += 256 * V) {
+        RankKey o[V];
+        int at[V];  // own galaxies up to o
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            o[u] = nx[u];
+            at[u] = 0;
+        }
+        load(c + 256 * V);
+#pragma unroll
+        for (int step = PS_OWN / 2; step > 0; step >>= 1)
+#pragma unroll
+            for (int u = 0; u < V; ++u) at[u] += rank_before<ORDER>(o[u], L, at[u] + step - 1) ? 0 : step;
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            at[u] += !rank_before<ORDER>(o[u], L, at[u]);
+            if (c + 256 * u >= (uint32_t)s1) continue;
+            if (at[u] == 0) ++none;
+            else if (at[u] < PS_OWN) atomicAdd(&L.hist[at[u]], 1u);
+        }
+    }
+    for (int o = 32; o > 0; o >>= 1) none += __shfl_xor(none, o, 64);
+    if (lane == 0) atomicAdd(&L.hist[0], (uint32_t)none);
+    __syncthreads();
+    int32_t h[U], sum = 0;
+#pragma unroll
+    for (int u = 0; u < U; ++u) h[u] = sum += (int32_t)L.hist[U * t + u];
+    int32_t inc = sum;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int32_t v = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += v;
+    }
+    if (lane == 63) L.wsum[wv] = inc;
+    __syncthreads();
+    int32_t base = inc - sum;
+    for (int i = 0; i < wv; ++i) base += L.wsum[i];
+#pragma unroll
+    for (int u = 0; u < U; ++u) L.hist[U * t + u] = (uint32_t)(base + h[u]);
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (t + 256 * u >= n) continue;
+        const CatSlot c = slot[e + t + 256 * u];
+        const RankKey k = rank_key<ORDER>(c);
+        int p = 0;  // place among the own galaxies
+#pragma unroll
+        for (int step = PS_OWN / 2; step > 0; step >>= 1) p += rank_less({L.a[p + step - 1], L.b[p + step - 1]}, k) ? step : 0;
+        const int64_t f = (int64_t)s0 + L.hist[p];
+        idx[f] = c.i;
+        pix_s[f] = c.pix;
+        r_s[f] = c.r;
+        w_s[f] = c.w;
+    }
+    __syncthreads();  // the next pixel's galaxies take the LDS
+}
+
 // order inside a pixel: 0 as placed (where any order does), 1 by input index, 2 by (r, input
 // index), the order of the reference's sums; in a folded pixel northern galaxies first, as the
 // radix sorts leave them.  Writes the sorted list of input indices, and
@@ -210,21 +325,38 @@ __device__ __forceinline__ bool rank_less(const RankKey& x, const RankKey& y)
 // Bound: the scattered 32-byte writes while pixels hold a few galaxies: each lane walks its own
 // pixel's.  A wavefront that meets a crowded pixel takes its pixels one after another: its own
 // galaxies of the pixel, sorted, stay in LDS, every other galaxy finds its place among them (seven
-// LDS reads, 64 galaxies at a time), and a galaxy's rank is the sum of the places up to its own.
+// LDS reads, 64 galaxies at a time), and a galaxy's rank is the sum of the places up to its own.  Pixels
+// beyond PS_GIANT go to whole blocks, PS_OWN own galaxies at a time (1.5e5 in one pixel: 0.33 ms by input
+// index and 0.66 by radius; by wavefronts 1.9 and 1.2), which costs the others one early barrier.
 template <int ORDER>
-__global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restrict__ slot,
+__global__ __launch_bounds__(256, 8) void k_rank(int64_t N, const CatSlot* __restrict__ slot,
                                               const int32_t* __restrict__ pstart, int32_t sh,
                                               uint32_t* __restrict__ idx,
                                               uint32_t* __restrict__ pix_s, double* __restrict__ r_s,
                                               double* __restrict__ w_s)
 {
-    __shared__ uint64_t own_a[4][64];
-    __shared__ uint32_t own_b[4][64], hist[4][64];
+    __shared__ RankLds lds;
+    __shared__ int32_t lead[4][2];  // a wavefront's slots meet two giant pixels at most (-1: none)
+    uint64_t(*own_a)[64] = (uint64_t(*)[64])lds.a;
+    uint32_t(*own_b)[64] = (uint32_t(*)[64])lds.b, (*hist)[64] = (uint32_t(*)[64])lds.hist;
     const int64_t e0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, e = min(e0, N - 1);
     const CatSlot me = slot[e];
     int64_t f = e;
+    bool giant = false, giants = false;  // this galaxy's pixel; a set of own galaxies starts in this block
     if (ORDER) {
         const int32_t s0 = pstart[me.pix >> sh], s1 = pstart[(me.pix >> sh) + 1];
+        giant = s1 - s0 > PS_GIANT && s1 - s0 <= PS_CROWD;
+        {
+            const int wv = threadIdx.x >> 6;
+            const uint64_t at = __ballot(giant && e0 < N && ((int32_t)e - s0) % PS_OWN == 0), next = at & (at - 1);
+            if ((threadIdx.x & 63) == 0) {
+                lead[wv][0] = at ? (int32_t)e + __ffsll((unsigned long long)at) - 1 : -1;
+                lead[wv][1] = next ? (int32_t)e + __ffsll((unsigned long long)next) - 1 : -1;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < 4; ++q) giants |= lead[q][0] >= 0;
+        }
         int32_t before = 0;
         if (__ballot(s1 - s0 > PS_WALK) == 0) {
             const uint64_t k = sortable_bits(me.r);
@@ -245,7 +377,7 @@ __global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restri
                 const int32_t u0 = __builtin_amdgcn_readlane(s0, l), u1 = __builtin_amdgcn_readlane(s1, l);
                 const uint64_t group = __ballot(s0 == u0 && e0 < N);
                 todo &= ~group;
-                if (u1 - u0 > PS_CROWD) continue;
+                if (u1 - u0 > PS_GIANT) continue;
                 int p = 0;  // place among the wavefront's galaxies of this pixel
                 for (uint64_t m = group; m; m &= m - 1) {
                     const int j = __ffsll((unsigned long long)m) - 1;
@@ -263,16 +395,16 @@ __global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restri
                     own_b[wv][p] = k.b;
                 }
                 wave_lds_sync();
-                CatSlot nx = slot[min(u0 + lane, u1 - 1)];
-                for (int32_t c = u0; c < u1; c += 64) {
+                CatSlot nx = slot[min((uint32_t)(u0 + lane), (uint32_t)u1 - 1)];
+                for (uint32_t c = (uint32_t)u0; c < (uint32_t)u1; c += 64) {
                     const RankKey o = rank_key<ORDER>(nx);
-                    nx = slot[min(c + 64 + lane, u1 - 1)];  // the next 64 in flight
+                    nx = slot[min(c + 64u + lane, (uint32_t)u1 - 1)];  // the next 64 in flight
                     int at = 0;  // own galaxies up to o
 #pragma unroll
                     for (int step = 32; step > 0; step >>= 1)
                         at += rank_less(o, {own_a[wv][at + step - 1], own_b[wv][at + step - 1]}) ? 0 : step;
                     at += !rank_less(o, {own_a[wv][at], own_b[wv][at]});
-                    if (c + lane < u1 && at < 64) atomicAdd(&hist[wv][at], 1u);
+                    if (c + lane < (uint32_t)u1 && at < 64) atomicAdd(&hist[wv][at], 1u);
                 }
                 wave_lds_sync();
                 int32_t inc = (int32_t)hist[wv][lane];
@@ -287,11 +419,21 @@ __global__ __launch_bounds__(256) void k_rank(int64_t N, const CatSlot* __restri
         }
         if (s1 - s0 <= PS_CROWD) f = (int64_t)s0 + before;  // (fuller: as placed, the call is redone)
     }
-    if (e0 >= N) return;
-    idx[f] = me.i;
-    pix_s[f] = me.pix;
-    r_s[f] = me.r;
-    w_s[f] = me.w;
+    if (e0 < N && !giant) {
+        idx[f] = me.i;
+        pix_s[f] = me.pix;
+        r_s[f] = me.r;
+        w_s[f] = me.w;
+    }
+    if (ORDER && giants) {
+        __syncthreads();  // the wavefronts' use of the LDS
+        for (int q = 0; q < 8; ++q) {
+            const int32_t e1 = lead[q >> 1][q & 1];
+            if (e1 < 0) continue;
+            const uint32_t p1 = slot[e1].pix >> sh;
+            rank_block<ORDER>(slot, e1, pstart[p1], pstart[p1 + 1], lds, idx, pix_s, r_s, w_s);
+        }
+    }
 }
 
 // Slices of the sliced layout from the counts: one block per window of SELL_SIGMA pixels orders
